@@ -32,10 +32,11 @@ __device__ __forceinline__ void load_cell(const R* __restrict__ base, int64_t pl
 }
 
 // Whole-wave lane shifts by one lane through DPP (wave_shr:1 / wave_shl:1):
-// lane l receives lane l-1 (up) or lane l+1 (down); the end lanes keep their
-// own value.  No LDS round trip, unlike a bpermute shuffle.
-__device__ __forceinline__ int dpp_up(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false); }
-__device__ __forceinline__ int dpp_dn(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false); }
+// lane l receives lane l-1 (up) or lane l+1 (down); the end lane, a halo lane
+// in every sweep, receives zero (to keep its own value would take a move ahead
+// of every shift).  No LDS round trip, unlike a bpermute shuffle.
+__device__ __forceinline__ int dpp_up(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, true); }
+__device__ __forceinline__ int dpp_dn(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x130, 0xf, 0xf, true); }
 __device__ __forceinline__ double shfl_up1(double x)
 {
     const long long b = __double_as_longlong(x);
@@ -183,10 +184,118 @@ __device__ __forceinline__ void load_row(const R* __restrict__ Acol, const R* __
 }
 
 // ---------------------------------------------------------- MUSCL-Hancock --
+// Rows of an item in range (q64 in hf_physics.h), from the first on: returns
+// the number of rows done, it.rows unless a lane left the range.  The caller
+// finishes with the general rows.
+// Per row: the new row's differences to the one before it serve the y slopes
+// of this row and, kept, of the next; the x slopes take theirs from the right
+// neighbour, and the left one's by a lane shift.
+// FP64 VALU issue bounds it, with two waves per SIMD: 8192^2 Van Leer runs at
+// 27.8 Gcell-updates/s, 21.5 with the general rows.
+template <class M, int LIM>
+__device__ __forceinline__ int muscl_rows_q64(const HfStepArgs<double>& a, const HfItem it, const HfBlockDev& bd,
+                                              const int lane, const double dt_step, const double hx, const double hy,
+                                              double& mx, double& my)
+{
+    const double gam = a.gamma, g1 = a.gamma - 1.0;
+    if (!(q64::constants_in_range(gam, g1) && q64::half_step_in_range(hx) && q64::half_step_in_range(hy))) return 0;
+    const double ig1 = 1.0 / g1;
+    const int xraw = it.x0 + lane;
+    const bool valid = xraw < bd.tx;
+    const int xc = valid ? xraw : bd.tx - 1;
+    const bool gcol = xc < 2 || xc >= bd.tx - 2;
+    const double* Acol = a.A + bd.off + xc;
+    const double* Gcol = a.G + bd.off + xc;
+    const int pitch = bd.pitch, ty = bd.ty;
+    const int64_t plane = bd.plane;
+#define ROW(y, u) load_row<double>(Acol, Gcol, gcol, (y), 2, ty, pitch, plane, (u))
+    const bool out = valid && lane >= 2 && lane < 62 && xraw >= 2 && xraw < bd.tx - 2;
+    // lanes that write, whose x faces those use, and that those are reconstructed from
+    const q64::mask m0 = __ballot(out), m1 = m0 | m0 << 1 | m0 >> 1, m2 = m1 | m1 << 1 | m1 >> 1;
+    const double rdx = 1.0 / bd.dx, rdy = 1.0 / bd.dy;
+
+    const int y0 = it.y0;
+    double uc[4], up[4], un[4], dl[4], cl[4], Gs[4], Tc[4];
+    q64::mask bad = 0, bc, bp, bn;   // rows y, y+1, y+2 out of range
+    {
+        double um[4], dr[4], cr[4], lo[4], hi[4];
+        ROW(y0 - 2, um);
+        ROW(y0 - 1, uc);
+        ROW(y0, up);
+        ROW(y0 + 1, un);
+        bad = q64::out_of_range(um) | q64::out_of_range(uc);
+        bc = q64::out_of_range(up);
+        bp = q64::out_of_range(un);
+        q64::differences(um, uc, dl, cl);
+        q64::differences(uc, up, dr, cr);
+        q64::reconstruct<LIM, false>(uc, dl, dr, cl, cr, hy, g1, ig1, lo, hi, bad);     // cell y0-1
+        const q64::State sl = q64::make_state(hi, gam, g1, ig1, bad);
+        q64::differences(up, un, dl, cl);
+        q64::reconstruct<LIM, false>(up, dr, dl, cr, cl, hy, g1, ig1, lo, Tc, bad);     // cell y0
+        const q64::State sr = q64::make_state(lo, gam, g1, ig1, bad);
+        q64::hllc<false>(sl, sr, Gs, bad);
+        if ((bad | bc | bp) & m0) return 0;
+    }
+    for (int k = 0; k < 4; k++) { uc[k] = up[k]; up[k] = un[k]; }
+    ROW(y0 + 2, un);
+
+    double* Ob = a.O + bd.off;
+    for (int r = 0; r < it.rows; r++) {
+        const int y = y0 + r;
+        double nn[4];
+        ROW(y + 3 < ty ? y + 3 : ty - 1, nn);     // next iteration's U(y+2)
+        bn = q64::out_of_range(un);
+
+        // y direction: reconstruct cell y+1, flux through face y+1/2
+        q64::mask by = 0, bx = 0;
+        double dn[4], cn[4], Bn[4], Tn[4], Gn[4];
+        q64::differences(up, un, dn, cn);
+        q64::reconstruct<LIM, false>(up, dl, dn, cl, cn, hy, g1, ig1, Bn, Tn, by);
+        {
+            const q64::State sl = q64::make_state(Tc, gam, g1, ig1, by);
+            const q64::State sr = q64::make_state(Bn, gam, g1, ig1, by);
+            q64::hllc<false>(sl, sr, Gn, by);
+        }
+
+        // x direction: reconstruct cell (x, y) from lane neighbours
+        double ur[4], xl[4], xr[4], kl[4], kr[4], Lf[4], Rf[4], Rl[4], Fw[4], Fe[4];
+        for (int k = 0; k < 4; k++) ur[k] = shfl_dn1(uc[k]);
+        q64::differences(uc, ur, xr, kr);
+        for (int k = 0; k < 4; k++) { xl[k] = shfl_up1(xr[k]); kl[k] = shfl_up1(kr[k]); }
+        q64::reconstruct<LIM, true>(uc, xl, xr, kl, kr, hx, g1, ig1, Lf, Rf, bx);
+        for (int k = 0; k < 4; k++) Rl[k] = shfl_up1(Rf[k]);
+        {
+            const q64::State sl = q64::make_state(Rl, gam, g1, ig1, bx);
+            const q64::State sr = q64::make_state(Lf, gam, g1, ig1, bx);
+            q64::hllc<true>(sl, sr, Fw, bx);          // face x-1/2
+        }
+        for (int k = 0; k < 4; k++) Fe[k] = shfl_dn1(Fw[k]);   // face x+1/2
+
+        double Ln[4], Un[4], dx_, dy_;
+        update_cell<M>(rdx, rdy, dt_step, Fw, Fe, Gs, Gn, uc, Ln, Un);
+        q64::wave_speeds(Un, gam, g1, dx_, dy_, by);
+        if (((by | bp | bn) & m0) | (bx & m1) | (bc & m2)) return r;
+        if (out) {
+            double* o = Ob + (int64_t)y * pitch + xraw;
+            for (int k = 0; k < 4; k++) o[k * plane] = Un[k];
+            mx = dmax_nan(mx, dx_);
+            my = dmax_nan(my, dy_);
+        }
+        bc = bp;
+        bp = bn;
+        for (int k = 0; k < 4; k++) {
+            Gs[k] = Gn[k]; Tc[k] = Tn[k]; uc[k] = up[k]; up[k] = un[k]; un[k] = nn[k];
+            dl[k] = dn[k]; cl[k] = cn[k];
+        }
+    }
+    return it.rows;
+#undef ROW
+}
+
 // MUSCLHancockScheme::operator() (scheme/muscl_hancock/muscl_hancock.cpp:41-55)
 // fused with ForwardEulerODESolver (scheme/ode/forward_euler/forward_euler.cpp:25-30).
 // Output columns per wave: 60 (lanes 2..61); lanes 0,1,62,63 are halo.
-template <class M, int LIM, bool RESID>
+template <class M, int LIM, bool RESID, bool QUICK>
 __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, const HfItem it, const int lane,
                                            const double dt_step, const double dt_pred,
                                            unsigned long long* __restrict__ imax_out)
@@ -212,7 +321,11 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
     const R dtR = R(dt_step);
     const R gam = R(a.gamma), g1 = R(a.gamma - 1.0);
 
-    const int y0 = it.y0;
+    double mx = 0.0, my = 0.0;
+    int done = 0;
+    if constexpr (QUICK && !RESID && !M::fast) done = muscl_rows_q64<M, LIM>(a, it, bd, lane, dt_step, hx, hy, mx, my);
+    if (done < it.rows) {
+    const int y0 = it.y0 + done, rows = it.rows - done;
     R um[4], uc[4], up[4], un[4];
     ROW(y0 - 2, um);
     ROW(y0 - 1, uc);
@@ -236,8 +349,7 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
     ROW(y0 + 2, un);
 
     R* Ob = RESID ? a.O : a.O + bd.off;
-    double mx = 0.0, my = 0.0;
-    for (int r = 0; r < it.rows; r++) {
+    for (int r = 0; r < rows; r++) {
         const int y = y0 + r;
         R nn[4];
         ROW(y + 3 < ty ? y + 3 : ty - 1, nn);     // next iteration's U(y+2)
@@ -278,6 +390,7 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
         }
         for (int k = 0; k < 4; k++) { Gs[k] = Gn[k]; Tc[k] = Tn[k]; uc[k] = up[k]; up[k] = un[k]; un[k] = nn[k]; }
     }
+    }
     if (!RESID) store_maxima(imax_out, it.block, wave_max(mx), wave_max(my), a.probe_max != 0);
 #undef ROW
 }
@@ -293,7 +406,109 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
 // write, up to nrows of them.
 __device__ __forceinline__ bool item_transposed(const HfItem& it) { return it.rows < 0; }
 
-template <class M, int LIM, bool RESID>
+// Columns of a transposed item in range, as muscl_rows_q64.
+template <class M, int LIM>
+__device__ __forceinline__ int muscl_cols_q64(const HfStepArgs<double>& a, const HfItem it, const HfBlockDev& bd,
+                                              const int lane, const double dt_step, const double hx, const double hy,
+                                              double& mx, double& my)
+{
+    const double gam = a.gamma, g1 = a.gamma - 1.0;
+    if (!(q64::constants_in_range(gam, g1) && q64::half_step_in_range(hx) && q64::half_step_in_range(hy))) return 0;
+    const double ig1 = 1.0 / g1;
+    const int code = -it.rows;
+    const int cols = code & 255, nrows = code >> 8;
+    const int yraw = it.y0 + lane;
+    const bool valid = yraw < bd.ty;
+    const int yc = valid ? yraw : bd.ty - 1;
+    const bool grow = yc < 2 || yc >= bd.ty - 2;
+    const int pitch = bd.pitch, tx = bd.tx;
+    const double* Arow = a.A + bd.off + (int64_t)yc * pitch;
+    const double* Grow = a.G + bd.off + (int64_t)yc * pitch;
+    const int64_t plane = bd.plane;
+#define COL(x, u) load_cell<double>(((grow || (x) < 2 || (x) >= tx - 2) ? Grow : Arow) + (x), plane, (u))
+    const bool out = valid && lane >= 2 && lane < 62 && lane < 2 + nrows && yraw >= 2 && yraw < bd.ty - 2;
+    const q64::mask m0 = __ballot(out), m1 = m0 | m0 << 1 | m0 >> 1, m2 = m1 | m1 << 1 | m1 >> 1;
+    const double rdx = 1.0 / bd.dx, rdy = 1.0 / bd.dy;
+
+    const int x0 = it.x0;
+    double uc[4], up[4], un[4], dl[4], cl[4], Fw[4], Rc[4];
+    q64::mask bad = 0, bc, bp, bn;   // columns x, x+1, x+2 out of range
+    {
+        double um[4], dr[4], cr[4], lo[4], hi[4];
+        COL(x0 - 2, um);
+        COL(x0 - 1, uc);
+        COL(x0, up);
+        COL(x0 + 1, un);
+        bad = q64::out_of_range(um) | q64::out_of_range(uc);
+        bc = q64::out_of_range(up);
+        bp = q64::out_of_range(un);
+        q64::differences(um, uc, dl, cl);
+        q64::differences(uc, up, dr, cr);
+        q64::reconstruct<LIM, true>(uc, dl, dr, cl, cr, hx, g1, ig1, lo, hi, bad);      // column x0-1
+        const q64::State sl = q64::make_state(hi, gam, g1, ig1, bad);
+        q64::differences(up, un, dl, cl);
+        q64::reconstruct<LIM, true>(up, dr, dl, cr, cl, hx, g1, ig1, lo, Rc, bad);      // column x0
+        const q64::State sr = q64::make_state(lo, gam, g1, ig1, bad);
+        q64::hllc<true>(sl, sr, Fw, bad);
+        if ((bad | bc | bp) & m0) return 0;
+    }
+    for (int k = 0; k < 4; k++) { uc[k] = up[k]; up[k] = un[k]; }
+    COL(x0 + 2, un);
+
+    double* Ob = a.O + bd.off;
+    for (int c = 0; c < cols; c++) {
+        const int x = x0 + c;
+        double nn[4];
+        COL(x + 3 < tx ? x + 3 : tx - 1, nn);     // next iteration's U(x+2)
+        bn = q64::out_of_range(un);
+
+        // x direction: reconstruct column x+1, flux through face x+1/2
+        q64::mask by = 0, bx = 0;
+        double dn[4], cn[4], Ln[4], Rn[4], Fe[4];
+        q64::differences(up, un, dn, cn);
+        q64::reconstruct<LIM, true>(up, dl, dn, cl, cn, hx, g1, ig1, Ln, Rn, bx);
+        {
+            const q64::State sl = q64::make_state(Rc, gam, g1, ig1, bx);
+            const q64::State sr = q64::make_state(Ln, gam, g1, ig1, bx);
+            q64::hllc<true>(sl, sr, Fe, bx);
+        }
+
+        // y direction: reconstruct cell (x, y) from lane neighbours
+        double ut[4], xl[4], xr[4], kl[4], kr[4], Bf[4], Tf[4], Tl[4], Gs[4], Gn[4];
+        for (int k = 0; k < 4; k++) ut[k] = shfl_dn1(uc[k]);
+        q64::differences(uc, ut, xr, kr);
+        for (int k = 0; k < 4; k++) { xl[k] = shfl_up1(xr[k]); kl[k] = shfl_up1(kr[k]); }
+        q64::reconstruct<LIM, false>(uc, xl, xr, kl, kr, hy, g1, ig1, Bf, Tf, by);
+        for (int k = 0; k < 4; k++) Tl[k] = shfl_up1(Tf[k]);
+        {
+            const q64::State sl = q64::make_state(Tl, gam, g1, ig1, by);
+            const q64::State sr = q64::make_state(Bf, gam, g1, ig1, by);
+            q64::hllc<false>(sl, sr, Gs, by);         // face y-1/2
+        }
+        for (int k = 0; k < 4; k++) Gn[k] = shfl_dn1(Gs[k]);   // face y+1/2
+
+        double Lu[4], Un[4], dx_, dy_;
+        update_cell<M>(rdx, rdy, dt_step, Fw, Fe, Gs, Gn, uc, Lu, Un);
+        q64::wave_speeds(Un, gam, g1, dx_, dy_, bx);
+        if (((bx | bp | bn) & m0) | (by & m1) | (bc & m2)) return c;
+        if (out) {
+            double* o = Ob + (int64_t)yraw * pitch + x;
+            for (int k = 0; k < 4; k++) o[k * plane] = Un[k];
+            mx = dmax_nan(mx, dx_);
+            my = dmax_nan(my, dy_);
+        }
+        bc = bp;
+        bp = bn;
+        for (int k = 0; k < 4; k++) {
+            Fw[k] = Fe[k]; Rc[k] = Rn[k]; uc[k] = up[k]; up[k] = un[k]; un[k] = nn[k];
+            dl[k] = dn[k]; cl[k] = cn[k];
+        }
+    }
+    return cols;
+#undef COL
+}
+
+template <class M, int LIM, bool RESID, bool QUICK>
 __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a, const HfItem it, const int lane,
                                              const double dt_step, const double dt_pred,
                                              unsigned long long* __restrict__ imax_out)
@@ -321,7 +536,12 @@ __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a,
     const R dtR = R(dt_step);
     const R gam = R(a.gamma), g1 = R(a.gamma - 1.0);
 
-    const int x0 = it.x0;
+    double mx = 0.0, my = 0.0;
+    int done = 0;
+    if constexpr (QUICK && !RESID && !M::fast)
+        done = muscl_cols_q64<M, LIM>(a, it, bd, lane, dt_step, hx, hy, mx, my);
+    if (done < cols) {
+    const int x0 = it.x0 + done, left = cols - done;
     R um[4], uc[4], up[4], un[4];
     COL(x0 - 2, um);
     COL(x0 - 1, uc);
@@ -343,8 +563,7 @@ __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a,
     COL(x0 + 2, un);
 
     R* Ob = RESID ? a.O : a.O + bd.off;
-    double mx = 0.0, my = 0.0;
-    for (int c = 0; c < cols; c++) {
+    for (int c = 0; c < left; c++) {
         const int x = x0 + c;
         R nn[4];
         COL(x + 3 < tx ? x + 3 : tx - 1, nn);     // next iteration's U(x+2)
@@ -384,6 +603,7 @@ __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a,
             }
         }
         for (int k = 0; k < 4; k++) { Fw[k] = Fe[k]; Rc[k] = Rn[k]; uc[k] = up[k]; up[k] = un[k]; un[k] = nn[k]; }
+    }
     }
     if (!RESID) store_maxima(imax_out, it.block, wave_max(mx), wave_max(my), a.probe_max != 0);
 #undef COL
@@ -441,14 +661,14 @@ __device__ __forceinline__ int round_of(const HfStepArgs<R>& a, unsigned idx)
     return l;
 }
 
-template <class M, int LIM, bool RESID>
+template <class M, int LIM, bool RESID, bool QUICK = true>
 __device__ __forceinline__ void muscl_go(const HfStepArgs<typename M::R>& a, const HfItem& it, int lane, double dt_step,
                                          double dt_pred, unsigned long long* imax_out)
 {
     if (!RESID && item_transposed(it))
-        muscl_item_t<M, LIM, RESID>(a, it, lane, dt_step, dt_pred, imax_out);
+        muscl_item_t<M, LIM, RESID, QUICK>(a, it, lane, dt_step, dt_pred, imax_out);
     else
-        muscl_item<M, LIM, RESID>(a, it, lane, dt_step, dt_pred, imax_out);
+        muscl_item<M, LIM, RESID, QUICK>(a, it, lane, dt_step, dt_pred, imax_out);
 }
 
 template <class R>
@@ -549,56 +769,59 @@ __device__ __forceinline__ void main_item(const HfStepArgs<typename M::R>& a, un
     typedef typename M::R R;
     const HfItem it = a.items[a.item0 + idx];
     if (a.use_fixed) {
-        muscl_go<M, LIM, RESID>(a, it, lane, a.fixed_step, a.fixed_pred, a.imax_new);
-        return;
+        c_step = a.fixed_step;
+        c_pred = a.fixed_pred;
+    } else {
+        if (a.skip[it.block]) return;   // left to the guess launch
+        const HfBlockDev bd = a.blocks[it.block];
+        if (it.block != cached) {
+            cached = it.block;
+            step_dts<R>(a, bd, true, c_step, c_pred, c_kstep, c_kpred);
+        }
+        record_dts<R>(a, it, bd, true, c_step, c_pred, c_kstep, c_kpred);
     }
-    if (a.skip[it.block]) return;   // left to the guess launch
-    const HfBlockDev bd = a.blocks[it.block];
-    if (it.block != cached) {
-        cached = it.block;
-        step_dts<R>(a, bd, true, c_step, c_pred, c_kstep, c_kpred);
-    }
-    record_dts<R>(a, it, bd, true, c_step, c_pred, c_kstep, c_kpred);
     muscl_go<M, LIM, RESID>(a, it, lane, c_step, c_pred, a.imax_new);
 }
 
 template <class M, int LIM, bool RESID>
-__global__ __launch_bounds__(256) void k_muscl(const HfStepArgs<typename M::R> a)
+__global__ __launch_bounds__(256, 2) void k_muscl(const HfStepArgs<typename M::R> a)
 {
+    typedef typename M::R R;
     const int lane = threadIdx.x & 63;
     int cached = -1;   // the block whose speculative dts this wave has computed
     double c_step = 0.0, c_pred = 0.0;
     long long c_kstep = 0, c_kpred = 0;
-    const unsigned nsk = (a.nskip && !a.use_fixed) ? __builtin_amdgcn_readfirstlane(*a.nskip) : 0u;
-    if (nsk == 0u) {   // every item of the list
-        const unsigned n = (unsigned)a.nmain;
-        for (unsigned idx = ticket_first(n); idx < n; idx = ticket_next(a.sync, lane, n))
-            main_item<M, LIM, RESID>(a, idx, lane, cached, c_step, c_pred, c_kstep, c_kpred);
-        return;
-    }
-    // tickets over the segments of the blocks not skipped
+    // every item of the list, or with skipped blocks tickets over the
+    // segments of the others
+    const bool some = a.nskip && !a.use_fixed && __builtin_amdgcn_readfirstlane(*a.nskip) != 0u;
     const int nseg = 3 * a.nblocks;
-    unsigned n = 0u;
-    for (int c0 = 0; c0 < nseg; c0 += 64) {
-        const int k = c0 + lane;
-        const unsigned cnt = (k < nseg && !a.skip[k % a.nblocks]) ? (unsigned)a.segs[2 * k + 1] : 0u;
-        unsigned tot;
-        lane_prefix(cnt, tot);
-        n += tot;
-    }
+    unsigned n = (unsigned)a.nmain;
     RangeCursor cur;
-    main_chunk<typename M::R>(a, cur, 0);
-    cur.base = 0u;
-    for (unsigned t = ticket_first(n); t < n; t = ticket_next(a.sync, lane, n)) {
-        while (t >= cur.base + cur.total) {
-            const unsigned nb_ = cur.base + cur.total;
-            if (cur.c0 + 64 >= nseg) return;   // not reached: the chunks hold n items
-            main_chunk<typename M::R>(a, cur, cur.c0 + 64);
-            cur.base = nb_;
+    if (some) {
+        n = 0u;
+        for (int c0 = 0; c0 < nseg; c0 += 64) {
+            const int k = c0 + lane;
+            const unsigned cnt = (k < nseg && !a.skip[k % a.nblocks]) ? (unsigned)a.segs[2 * k + 1] : 0u;
+            unsigned tot;
+            lane_prefix(cnt, tot);
+            n += tot;
         }
-        int j;
-        const unsigned idx = cursor_item(cur, t, j);
-        if (idx >= (unsigned)a.nmain) return;
+        main_chunk<R>(a, cur, 0);
+        cur.base = 0u;
+    }
+    for (unsigned t = ticket_first(n); t < n; t = ticket_next(a.sync, lane, n)) {
+        unsigned idx = t;
+        if (some) {
+            while (t >= cur.base + cur.total) {
+                const unsigned nb_ = cur.base + cur.total;
+                if (cur.c0 + 64 >= nseg) return;   // not reached: the chunks hold n items
+                main_chunk<R>(a, cur, cur.c0 + 64);
+                cur.base = nb_;
+            }
+            int j;
+            idx = cursor_item(cur, t, j);
+            if (idx >= (unsigned)a.nmain) return;
+        }
         main_item<M, LIM, RESID>(a, idx, lane, cached, c_step, c_pred, c_kstep, c_kpred);
     }
 }
@@ -652,7 +875,7 @@ __device__ __forceinline__ void guess_enter(const HfStepArgs<R>& a, GuessProblem
 }
 
 template <class M, int LIM>
-__global__ __launch_bounds__(256) void k_muscl_guess(const HfStepArgs<typename M::R> a)
+__global__ __launch_bounds__(256, 2) void k_muscl_guess(const HfStepArgs<typename M::R> a)
 {
     typedef typename M::R R;
     const int lane = threadIdx.x & 63;
@@ -708,7 +931,7 @@ __global__ __launch_bounds__(256) void k_muscl_guess(const HfStepArgs<typename M
 }
 
 template <class M, int LIM>
-__global__ __launch_bounds__(256) void k_muscl_check(const HfStepArgs<typename M::R> a)
+__global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typename M::R> a)
 {
     typedef typename M::R R;
     const int lane = threadIdx.x & 63;
@@ -790,7 +1013,7 @@ __global__ __launch_bounds__(256) void k_muscl_check(const HfStepArgs<typename M
             if (check_verdict<R>(a, bd.problem, pr, a.nblocks, bd.lb, mg, dt_step, dt_pred, kstep, kpred)) {
                 atomicExch(&fixed_chk[it.block], 1u);
                 record_dts<R>(a, it, bd, false, dt_step, dt_pred, kstep, kpred);
-                muscl_go<M, LIM, false>(a, it, lane, dt_step, dt_pred, imax_chk);
+                muscl_go<M, LIM, false, false>(a, it, lane, dt_step, dt_pred, imax_chk);   // rare: the general rows only
                 __builtin_amdgcn_s_waitcnt(0xF70);   // its maxima are performed before the next verdict reads them
             }
         }
@@ -799,6 +1022,74 @@ __global__ __launch_bounds__(256) void k_muscl_check(const HfStepArgs<typename M
 }
 
 // ---------------------------------------------------------------- Godunov --
+// Rows of a Godunov item in range, as muscl_rows_q64.
+template <class M, class DtOf>
+__device__ __forceinline__ int godunov_rows_q64(const HfStepArgs<double>& a, const HfItem it, const HfBlockDev& bd,
+                                                const int lane, DtOf&& dt_of, double& dt, double& mx, double& my)
+{
+    const double gam = a.gamma, g1 = a.gamma - 1.0;
+    const int xraw = it.x0 + lane;
+    const bool valid = xraw < bd.tx;
+    const int xc = valid ? xraw : bd.tx - 1;
+    const bool gcol = xc < 1 || xc >= bd.tx - 1;
+    const double* Acol = a.A + bd.off + xc;
+    const double* Gcol = a.G + bd.off + xc;
+    const int pitch = bd.pitch, ty = bd.ty;
+    const int64_t plane = bd.plane;
+#define ROW(y, u) load_row<double>(Acol, Gcol, gcol, (y), 1, ty, pitch, plane, (u))
+    const bool out = valid && lane >= 1 && lane < 63 && xraw >= 1 && xraw < bd.tx - 1;
+    const q64::mask m0 = __ballot(out), m1 = m0 | m0 << 1 | m0 >> 1;   // lanes that write, and their x neighbours
+    const int y0 = it.y0;
+    double ub[4], uc[4], un[4], Gs[4];
+    ROW(y0 - 1, ub);
+    ROW(y0, uc);
+    ROW(y0 + 1, un);
+    const double ig1 = 1.0 / g1, rdx = 1.0 / bd.dx, rdy = 1.0 / bd.dy;
+    q64::mask bad = q64::out_of_range(ub), bc = q64::out_of_range(uc);
+    q64::State sc = q64::make_state(uc, gam, g1, ig1, bc);
+    {
+        const q64::State sb = q64::make_state(ub, gam, g1, ig1, bad);
+        q64::hllc<false>(sb, sc, Gs, bad);         // face y0-1/2
+    }
+    dt = dt_of();
+    if (!q64::constants_in_range(gam, g1) || (bad & m0)) return 0;
+    double* Ob = a.O + bd.off;
+    for (int r = 0; r < it.rows; r++) {
+        const int y = y0 + r;
+        double nn[4];
+        ROW(y + 2 < ty ? y + 2 : ty - 1, nn);     // next iteration's U(y+1)
+        q64::mask bn = q64::out_of_range(un), bx = 0;
+        const q64::State sn = q64::make_state(un, gam, g1, ig1, bn);
+        double Gn[4], Fw[4], Fe[4];
+        q64::hllc<false>(sc, sn, Gn, bn);          // face y+1/2
+
+        q64::State sw;
+        sw.U0 = shfl_up1(sc.U0); sw.U1 = shfl_up1(sc.U1); sw.U2 = shfl_up1(sc.U2); sw.U3 = shfl_up1(sc.U3);
+        sw.u = shfl_up1(sc.u); sw.v = shfl_up1(sc.v); sw.p = shfl_up1(sc.p); sw.E = shfl_up1(sc.E);
+        sw.a = shfl_up1(sc.a); sw.y = shfl_up1(sc.y);
+        q64::hllc<true>(sw, sc, Fw, bx);           // face x-1/2
+        for (int k = 0; k < 4; k++) Fe[k] = shfl_dn1(Fw[k]);
+
+        const double U[4] = {sc.U0, sc.U1, sc.U2, sc.U3};
+        double Ln[4], Un[4], dx_, dy_;
+        update_cell<M>(rdx, rdy, dt, Fw, Fe, Gs, Gn, U, Ln, Un);
+        q64::mask bw = 0;
+        q64::wave_speeds(Un, gam, g1, dx_, dy_, bw);
+        if (((bn | bw) & m0) | ((bc | bx) & m1)) return r;
+        if (out) {
+            double* o = Ob + (int64_t)y * pitch + xraw;
+            for (int k = 0; k < 4; k++) o[k * plane] = Un[k];
+            mx = dmax_nan(mx, dx_);
+            my = dmax_nan(my, dy_);
+        }
+        for (int k = 0; k < 4; k++) { Gs[k] = Gn[k]; un[k] = nn[k]; }
+        sc = sn;
+        bc = bn;
+    }
+    return it.rows;
+#undef ROW
+}
+
 // GodunovScheme::operator() (scheme/godunov/godunov.cpp:27-118) fused with
 // the forward Euler update.  Each cell's primitives and sound speed are
 // computed once and shared by its four faces.  Output columns per wave: 62.
@@ -827,7 +1118,12 @@ __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a,
     const R rdy = R(1.0 / bd.dy);
     const R gam = R(a.gamma), g1 = R(a.gamma - 1.0);
 
-    const int y0 = it.y0;
+    double mx = 0.0, my = 0.0, dt = 0.0;
+    int done = 0;
+    constexpr bool QUICK = !RESID && !M::fast;
+    if constexpr (QUICK) done = godunov_rows_q64<M>(a, it, bd, lane, dt_of, dt, mx, my);
+    if (done < it.rows) {
+    const int y0 = it.y0 + done, rows = it.rows - done;
     R ub[4], uc[4], un[4];
     ROW(y0 - 1, ub);
     ROW(y0, uc);
@@ -836,10 +1132,9 @@ __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a,
     State<R> sc = make_state<M>(uc, gam, g1);
     R Gs[4];
     hllc<M, false>(sb, sc, Gs);                    // face y0-1/2
-    const R dtR = R(dt_of());
+    const R dtR = QUICK ? R(dt) : R(dt_of());
     R* Ob = RESID ? a.O : a.O + bd.off;
-    double mx = 0.0, my = 0.0;
-    for (int r = 0; r < it.rows; r++) {
+    for (int r = 0; r < rows; r++) {
         const int y = y0 + r;
         R nn[4];
         ROW(y + 2 < ty ? y + 2 : ty - 1, nn);     // next iteration's U(y+1)
@@ -869,6 +1164,7 @@ __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a,
         }
         for (int k = 0; k < 4; k++) { Gs[k] = Gn[k]; un[k] = nn[k]; }
         sc = sn;
+    }
     }
     if (!RESID) store_maxima(imax_out, it.block, wave_max(mx), wave_max(my), false);
 #undef ROW

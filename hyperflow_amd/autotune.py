@@ -15,6 +15,10 @@ problem (1, 2-8, 9 or more) and the median block size (cells, to the nearest
 power of 4).  A workload whose class has no entry gets the plan of the
 nearest tuned class with the same scheme, limiter, precision and dt mode.
 
+The library itself caps tile_rows where a launch would leave resident waves
+without an item (build_plan in csrc/hf_capi.cpp), so the plans below matter to
+launches of more than one round.
+
 Every candidate is timed `repeats` times (each run from the same state, after
 warm-up steps); its time is the median, and the chosen plan records the
 spread (max - min) / median of its runs.
@@ -207,10 +211,10 @@ def _workloads(names):
     for name in names:
         if name == "godunov-quadrants":
             c = C.godunov_quadrants(0)
-            # 160k cells fill a fraction of the resident waves: short items
-            # keep more SIMDs busy (a Godunov item has one halo row per side)
+            # 160k cells are one round of the resident waves at any tile_rows
+            # of 3 or more
             out.append(("godunov-quadrants", [c], [c.initial_fields()[0]], "fp64", "compat", False,
-                        {"rows": (2, 3, 4, 6, 8, 12, 16), "tails": (1, 2, 3, 4, 6, 8)}))
+                        {"rows": (0, 2, 3, 4, 8), "tails": (0,)}))
         elif name == "step-channel":
             c = C.muscl_step_channel(1024)
             # past the first 10 TimeStep calls' reduced CFL, as the benchmark times it

@@ -276,7 +276,6 @@ HfStepArgs<R> step_args(hf_ctx* c, int item0, int nitems, const void* A, const v
     a.fixrange = c->d_rounds + fixrange_offset(*c);
     a.nskip = nullptr;
     a.wait_ticks = c->wait_ticks;
-    a.probe_max = c->probe_max;
     a.nrounds = 0;
     a.pending = c->d_pending;
     a.npending = c->npending;
@@ -286,6 +285,8 @@ HfStepArgs<R> step_args(hf_ctx* c, int item0, int nitems, const void* A, const v
     a.skip_next = c->d_skip_next;
     a.imax_old = c->imax(c->cur);
     a.imax_new = c->imax(c->cur ^ 1);
+    a.ways = c->ways;
+    a.way_stride = c->way_stride;
     a.gmax = c->gmax(c->cur);
     a.calls = c->d_calls;
     a.hist = c->d_hist;
@@ -432,13 +433,14 @@ int full_dt(hf_ctx* c, int p, F src, double* dt)
 int ensure_partials(hf_ctx* c)
 {
     if (c->partials_valid) return HF_OK;
-    HF_HIP(hipMemsetAsync(c->imax(c->cur), 0, sizeof(unsigned long long) * 2 * c->nb, c->stream));
+    HF_HIP(hipMemsetAsync(c->imax(c->cur), 0, sizeof(unsigned long long) * c->max_words(), c->stream));
     HF_HIP(hipMemsetAsync(c->gmax(c->cur), 0, sizeof(unsigned long long) * 2 * c->nb, c->stream));
-    HF_HIP(hipMemsetAsync(c->d_imax_fix, 0, sizeof(unsigned long long) * 4 * c->nb, c->stream));
+    HF_HIP(hipMemsetAsync(c->d_imax_fix, 0, sizeof(unsigned long long) * 2 * c->max_words(), c->stream));
     HF_HIP(hipMemsetAsync(c->d_fixed, 0, sizeof(uint32_t) * 2 * c->nb, c->stream));
     HF_HIP(hipMemsetAsync(c->d_skip_next, 0, sizeof(uint32_t) * c->nb, c->stream));
     for (int b = 0; b < c->nb; b++) {
-        int rc = launch_scan(c, b, c->buf[c->cur], c->buf[c->cur], 1, c->imax(c->cur) + 2 * b);
+        int rc = launch_scan(c, b, c->buf[c->cur], c->buf[c->cur], 1,
+                             c->imax(c->cur) + HF_MAX_SLOT(b, 0, c->ways, c->way_stride));
         if (rc) return rc;
     }
     c->partials_valid = true;
@@ -464,7 +466,9 @@ int enqueue_steps(hf_ctx* c, int nsteps, bool timed, bool fixed = false, double 
         bk.bump = fixed ? 0 : 1;
         bk.clear0 = c->gmax(k ^ 1);
         bk.clear1 = c->imax(k ^ 1);
-        bk.nclear = 2 * c->nb;
+        bk.nclear0 = 2 * c->nb;
+        bk.nclear1 = (int)c->max_words();
+        bk.block_words = c->nrounds ? c->ways * c->way_stride : 0;
         bk.queue = c->d_sync;
         bk.nqueue = HF_SLOTS * HF_SYNC_WORDS;
         bk.pending = c->d_pending;
@@ -619,6 +623,7 @@ int build_plan(hf_ctx* c, const hf_case_desc* desc, bool dense)
     c->calls.assign(c->np, 0);
 
     // resident waves of a persistent update launch (the work items are sized for them)
+    int64_t simds = 0;
     {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -627,6 +632,7 @@ int build_plan(hf_ctx* c, const hf_case_desc* desc, bool dense)
         const int per_cu = c->prec == HF_FP64 ? hf::update_wgs_per_cu<double>(c->scheme, c->limiter, false)
                                               : hf::update_wgs_per_cu<float>(c->scheme, c->limiter, false);
         c->wg_cap = std::max(1, cus * per_cu);
+        simds = 4LL * cus;
         // in-launch waits give up after 10 ms of the counter kernels read
         // with s_memrealtime (its rate in kHz)
         int khz = 0;
@@ -640,37 +646,96 @@ int build_plan(hf_ctx* c, const hf_case_desc* desc, bool dense)
     // for compat MUSCL problems of several blocks, the lb-th blocks of all
     // problems for each fix-up launch lb = 1, 2, ..
     const int W = c->g == 2 ? 60 : 62;
-    const int rows = desc->tile_rows > 0 ? desc->tile_rows : (c->scheme == HF_MUSCL_HANCOCK ? 48 : 32);
+    const int most_rows = desc->tile_rows > 0 ? desc->tile_rows : (c->scheme == HF_MUSCL_HANCOCK ? 48 : 32);
     for (auto& P : c->probs) c->maxnb = std::max(c->maxnb, P.nb);
     c->item_begin.assign(c->nb, 0);
     c->item_count.assign(c->nb, 0);
-    // Items are taken from a queue in list order, so the list ends with small
-    // items: the last round of a launch then finishes together instead of
-    // waiting on a few long items (a timeline of the 8-block channel's main
+    // A launch that fits the resident waves at no more than tile_rows rows an
+    // item is one round of equal items (round_rows below).  A larger one takes
+    // its items from a queue in list order, so the list ends with small items:
+    // the last round then finishes together instead of waiting on a few long
+    // items (a timeline of the 8-block channel's main
     // launch showed half of the SIMDs idle over its last fifth with a 3/4
     // split into `rows`- and 32-row items).  Main launch: `rows`-row items,
     // then rows/2, then 8-row items (on the channel 11/16, 1/4 and 1/16 of the
     // rows, measured fastest among eight such plans; launches of many rounds
     // keep the small phases to about one round's worth of work).  A
-    // fix-up launch computes a single block on the whole GPU: uniform items
-    // sized so that one round of the resident waves takes them all.
+    // fix-up launch computes a single block on the whole GPU: one round.
+    // One round instead of tile_rows-row items, us per step: FP64 300^2 (96
+    // rows before, 2 now) 303 -> 20, 2048^2 (35) 311 -> 176, 8 x 97^2 channel
+    // (42 -> 2) 170 -> 47, Godunov 400^2 (8 -> 3) 25.3 -> 16.3, 1600^2 (21)
+    // 288 -> 55, FP32 1024^2 (6) 42 -> 29.
     // A MUSCL block whose last column strip would carry at most TR_COLS of its
     // 60 output columns (1024 = 17 x 60 + 4) gets that band as transposed
     // items instead: lanes along rows, the wave walking the band's columns,
     // 60 rows per item (k_muscl's muscl_item_t; rows = -(cols + 256 * nrows)).
     constexpr int TR_COLS = 30;
+    auto banded = [&](int b) {
+        const int nx = c->blocks[b].nx, strips = (nx + W - 1) / W;
+        return c->scheme == HF_MUSCL_HANCOCK && strips > 1 && nx - (strips - 1) * W <= TR_COLS;
+    };
+    auto band_items = [&](int b, int ny, int cols) {
+        const int nx = c->blocks[b].nx, rem = nx - ((nx + W - 1) / W - 1) * W;
+        return (ny + 59) / 60 * ((rem + cols - 1) / cols);
+    };
     auto add_rows = [&](int b, int y0, int y1, int r, bool tr) {
         const HfBlockDev& B = c->blocks[b];
         int strips = (B.nx + W - 1) / W;
         const int rem = B.nx - (strips - 1) * W;
-        const bool band = tr && c->scheme == HF_MUSCL_HANCOCK && strips > 1 && rem <= TR_COLS;
+        // A transposed item walks `cols` columns where the others walk r rows:
+        // with short items the band is cut into several.
+        const int cols = std::min(rem, std::max(r, 1));
+        const bool band = tr && banded(b) && band_items(b, y1 - y0, cols) <= (y1 - y0 + r - 1) / r;
         if (band) strips--;
         for (int y = y0; y < y1; y += r)
             for (int s = 0; s < strips; s++) c->items.push_back(HfItem{b, s * W, c->g + y, std::min(r, y1 - y)});
         if (band)
             for (int y = y0; y < y1; y += 60)
-                c->items.push_back(HfItem{b, c->g + strips * W, c->g + y - 2, -(rem + 256 * std::min(60, y1 - y))});
+                for (int x = 0; x < rem; x += cols)
+                    c->items.push_back(HfItem{b, c->g + strips * W + x, c->g + y - 2,
+                                              -(std::min(cols, rem - x) + 256 * std::min(60, y1 - y))});
     };
+    // items of a block in r-row pieces, as add_rows lists them
+    auto count_rows = [&](int b, int r) {
+        const HfBlockDev& B = c->blocks[b];
+        const int strips = (B.nx + W - 1) / W, rem = B.nx - (strips - 1) * W;
+        const int pieces = (B.ny + r - 1) / r, t = band_items(b, B.ny, std::min(rem, r));
+        return (int64_t)(strips - 1) * pieces + ((banded(b) && t <= pieces) ? t : pieces);
+    };
+    auto count_items = [&](const std::vector<int>& list, int r) {
+        int64_t n = 0;
+        for (int b : list) n += count_rows(b, r);
+        return n;
+    };
+    // The fewest rows an item may have so that one round of `waves` takes the
+    // items of the blocks, but at most `most`.
+    auto fit_rows = [&](const std::vector<int>& list, int64_t waves, int most) {
+        int lo = 1, hi = most;   // count_items() falls with r
+        while (lo < hi) {
+            const int mid = (lo + hi) / 2;
+            if (count_items(list, mid) <= waves) hi = mid;
+            else lo = mid + 1;
+        }
+        return lo;
+    };
+    // Items sized for one round of the resident waves, so that every wave takes
+    // one item and none draws a ticket: tickets and the maxima of short items
+    // are what a small launch would otherwise wait for.  With fewer than
+    // SHORT rows an item spends too much on its first rows (the reconstruction
+    // of two cells and a face before the first one it writes): then one wave
+    // per SIMD with items of twice the rows.  Per step, items for all resident
+    // waves / for one per SIMD: FP64 Godunov 400^2 (2 / 3 rows) 17.9 / 16.2 us,
+    // 8 x 256^2 channel (5 / 9) 79 / 76, 700^2 Van Leer (5 / 9) 39.6 / 40.2,
+    // 1024^2 (9 / 18) 57 / 63, FP32 1024^2 (6 / 18) 31.5 / 35.5.
+    constexpr int SHORT = 6;
+    auto round_rows = [&](const std::vector<int>& list, int most) {
+        const int r = fit_rows(list, wave_slots, most);
+        return r < SHORT ? std::min(most, fit_rows(list, simds, 2 * SHORT)) : r;
+    };
+    std::vector<int> all_blocks(c->nb);
+    for (int b = 0; b < c->nb; b++) all_blocks[b] = b;
+    const int rows = round_rows(all_blocks, most_rows);
+    const bool one_round = count_items(all_blocks, rows) <= wave_slots;
     // column strips of a block without its transposed band (the band is cheap)
     auto full_strips = [&](int b) {
         const HfBlockDev& B = c->blocks[b];
@@ -697,8 +762,8 @@ int build_plan(hf_ctx* c, const hf_case_desc* desc, bool dense)
         std::vector<int> y1(c->nb), y2(c->nb);
         for (int b = 0; b < c->nb; b++) {
             const int ny = c->blocks[b].ny;
-            y1[b] = std::min(ny, (int)(ny * (1.0 - f2 - f3)) / rows * rows);
-            y2[b] = std::min(ny, y1[b] + std::max(0, (int)(ny * (1.0 - f3)) - y1[b]) / r2 * r2);
+            y1[b] = one_round ? ny : std::min(ny, (int)(ny * (1.0 - f2 - f3)) / rows * rows);
+            y2[b] = one_round ? ny : std::min(ny, y1[b] + std::max(0, (int)(ny * (1.0 - f3)) - y1[b]) / r2 * r2);
         }
         c->segs.assign(6 * (size_t)c->nb, 0);
         for (int ph = 0; ph < 3; ph++)
@@ -713,26 +778,31 @@ int build_plan(hf_ctx* c, const hf_case_desc* desc, bool dense)
     }
     c->main_begin = perblock_end;
     c->main_items = (int)c->items.size() - perblock_end;
-    // Wave maxima read their slot before raising it where hundreds of a
-    // block's items end together (raise_max in hf_kernels.h); not for
-    // Godunov, whose items are short, nor for blocks of few items.
-    int most = 0;
-    for (int b = 0; b < c->nb; b++) most = std::max(most, c->item_count[b]);
-    c->probe_max = (c->scheme == HF_MUSCL_HANCOCK && most >= 256) ? 1 : 0;
+    // Maxima slots: about 16 items of a block to a slot, fewer slots where
+    // blocks are many (the ghost fill's last workgroup clears them all) or
+    // where every wave of the fix-up launches reads every block's.  One slot
+    // against these, us per step: 1024^2 FP32 49 / 31, 8 x 97^2 channel 60 /
+    // 49, Godunov 400^2 45 / 18, 900^2 64 / 27.
+    {
+        int per = 0;   // items of the block with most in the main list
+        for (int b = 0; b < c->nb; b++) {
+            int n = 0;
+            for (int ph = 0; ph < 3; ph++) n += c->segs[2 * (ph * c->nb + b) + 1];
+            per = std::max(per, n);
+        }
+        const int cap = c->maxnb == 1 ? 64 : 8;
+        c->ways = 1;
+        while (c->ways < cap && c->ways * 16 < per && c->ways * 2 * c->nb <= 256) c->ways *= 2;
+        c->way_stride = c->ways > 1 ? 16 : 2;
+    }
     c->fixrange.assign(2 * (size_t)c->nb, 0);
     if (c->scheme == HF_MUSCL_HANCOCK && c->dt_mode == HF_DT_COMPAT)
         for (int lb = 1; lb < c->maxnb; lb++) {
-            // rows per item so that the launch's wave-rows fill about 95 % of
-            // one round of the resident waves, within 4..16 rows
-            int64_t work = 0;
+            // items for one round of the resident waves, of at most 16 rows
+            std::vector<int> list;
             for (const auto& P : c->probs)
-                if (P.nb > lb) {
-                    work += (int64_t)full_strips(P.first + lb) * c->blocks[P.first + lb].ny;
-                }
-            const int64_t target = std::max<int64_t>(1, wave_slots * 95 / 100);
-            const int fr = desc->fix_rows > 0
-                               ? desc->fix_rows
-                               : (int)std::max<int64_t>(4, std::min<int64_t>(16, (work + target - 1) / target));
+                if (P.nb > lb) list.push_back(P.first + lb);
+            const int fr = desc->fix_rows > 0 ? desc->fix_rows : round_rows(list, 16);
             const int first = (int)c->items.size();
             for (const auto& P : c->probs)
                 if (P.nb > lb) {
@@ -818,13 +888,13 @@ int hf_create(const hf_case_desc* desc, hf_ctx** out)
             HF_HIPC(hipMemcpy(C->d_consts, cf.data(), cf.size() * 4, hipMemcpyHostToDevice));
         }
     }
-    HF_HIPC(hipMalloc(&C->d_imax, sizeof(unsigned long long) * 4 * C->nb));
+    HF_HIPC(hipMalloc(&C->d_imax, sizeof(unsigned long long) * 2 * C->max_words()));
     HF_HIPC(hipMalloc(&C->d_gmax, sizeof(unsigned long long) * 4 * C->nb));
     HF_HIPC(hipMalloc(&C->d_scan, sizeof(unsigned long long) * 4 * C->nb));
-    HF_HIPC(hipMemset(C->d_imax, 0, sizeof(unsigned long long) * 4 * C->nb));
+    HF_HIPC(hipMemset(C->d_imax, 0, sizeof(unsigned long long) * 2 * C->max_words()));
     HF_HIPC(hipMemset(C->d_gmax, 0, sizeof(unsigned long long) * 4 * C->nb));
-    HF_HIPC(hipMalloc(&C->d_imax_fix, sizeof(unsigned long long) * 4 * C->nb));
-    HF_HIPC(hipMemset(C->d_imax_fix, 0, sizeof(unsigned long long) * 4 * C->nb));
+    HF_HIPC(hipMalloc(&C->d_imax_fix, sizeof(unsigned long long) * 2 * C->max_words()));
+    HF_HIPC(hipMemset(C->d_imax_fix, 0, sizeof(unsigned long long) * 2 * C->max_words()));
     HF_HIPC(hipMalloc(&C->d_fixed, sizeof(uint32_t) * 2 * C->nb));
     HF_HIPC(hipMalloc(&C->d_fixstats, sizeof(unsigned long long) * 4));
     HF_HIPC(hipMemset(C->d_fixstats, 0, sizeof(unsigned long long) * 4));
@@ -1178,9 +1248,9 @@ int hf_step_noalloc(const hf_case_desc* desc, const void* d_in, void* d_out, int
     const size_t nb = (size_t)c.nb, np = (size_t)c.np;
     const size_t o_blocks = take(sizeof(HfBlockDev) * nb), o_probs = take(sizeof(HfProbDev) * np),
                  o_items = take(sizeof(HfItem) * c.items.size()), o_fill = take(sizeof(HfGhost) * fill.size()),
-                 o_consts = take(c.esize * 16 * nb), o_imax = take(sizeof(unsigned long long) * 4 * nb),
+                 o_consts = take(c.esize * 16 * nb), o_imax = take(sizeof(unsigned long long) * 2 * c.max_words()),
                  o_gmax = take(sizeof(unsigned long long) * 4 * nb),
-                 o_fix = take(sizeof(unsigned long long) * 4 * nb), o_fixed = take(sizeof(uint32_t) * 2 * nb),
+                 o_fix = take(sizeof(unsigned long long) * 2 * c.max_words()), o_fixed = take(sizeof(uint32_t) * 2 * nb),
                  o_skip = take(sizeof(uint32_t) * nb), o_skipn = take(sizeof(uint32_t) * nb),
                  o_sync = take(sizeof(uint32_t) * HF_SLOTS * HF_SYNC_WORDS),
                  o_rounds = take(sizeof(int32_t) * plan_table(c).size()), o_pend = take(sizeof(uint32_t) * c.npending),
@@ -1248,7 +1318,7 @@ int hf_step_noalloc(const hf_case_desc* desc, const void* d_in, void* d_out, int
     // wave-speed maxima of the input's interior (a device-resident loop gets
     // them from the previous step's update epilogue)
     for (int b = 0; b < c.nb; b++) {
-        rc = launch_scan(&c, b, d_in, d_in, 1, c.imax(0) + 2 * b);
+        rc = launch_scan(&c, b, d_in, d_in, 1, c.imax(0) + HF_MAX_SLOT(b, 0, c.ways, c.way_stride));
         if (rc) return rc;
     }
     rc = enqueue_steps(&c, 1, false);

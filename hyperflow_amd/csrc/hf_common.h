@@ -51,8 +51,11 @@ struct HfStepArgs {
     const R* A;   // interior source (U^n)
     const R* G;   // ghost source (filled ghosts)
     R* O;         // destination: U^{n+1} interior, or the residual L
-    const unsigned long long* imax_old;  // [nblocks][2] max wave speed of the U^n interior
-    unsigned long long* imax_new;        // [nblocks][2] max wave speed of the new interior
+    // Max wave speeds (x, y) of the U^n interior and of the new one: block b's
+    // are the maxima over its `ways` slots, slot w at HF_MAX_SLOT words.
+    const unsigned long long* imax_old;
+    unsigned long long* imax_new;
+    int32_t ways, way_stride;            // slots per block (a power of two), words per slot
     const unsigned long long* gmax;      // [nblocks][2] max wave speed of the ghosts
     const uint32_t* calls;               // TimeStep calls per problem (already bumped for this step)
     double* hist;                        // TimeStep results of problem 0: call k goes to hist[k - 1 - hist_base]
@@ -73,17 +76,20 @@ struct HfStepArgs {
     const int32_t* fixrange;
     const uint32_t* nskip;
     unsigned long long wait_ticks;       // bound of an in-launch wait in s_memrealtime ticks (10 ms)
-    int32_t probe_max;                   // 1: a wave reads a maxima slot before raising it (raise_max)
     uint32_t* pending;                   // [npending] bitmap over the fix-up items left to the check launch's last wave
     // Fix-up state of the step.  Slot 0 belongs to the guess launch, slot 1 to
-    // the check launch: imax_fix[s * 2 * nblocks + 2 * b + axis] holds the
-    // maxima of block b recomputed by launch s, fixed[s * nblocks + b] says
-    // that it was.
+    // the check launch: imax_fix + s * nblocks * ways * way_stride holds the
+    // maxima of the blocks recomputed by launch s (laid out as imax_new; the
+    // check launch uses slot 0 of a block only), fixed[s * nblocks + b] says
+    // that block b was.
     unsigned long long* imax_fix;
     uint32_t* fixed;
     uint32_t* skip;                      // [nblocks] the main list leaves the block to the guess launch
     uint32_t* skip_next;                 // [nblocks] the exact verdict for the next step
 };
+
+// First word (x; y follows) of slot w of block b in a maxima array.
+#define HF_MAX_SLOT(b, w, ways, stride) (((int64_t)(b) * (ways) + (w)) * (stride))
 
 // Counters of one update launch: the work-queue ticket counter, the number of
 // completed items (bit 31: the abort flag of the bounded waits) and the
@@ -104,7 +110,8 @@ struct GhostBook {
     int32_t bump;                 // add cps to every problem's counter
     unsigned long long* clear0;   // arrays to zero (next step's partials)
     unsigned long long* clear1;
-    int32_t nclear;               // elements in each
+    int32_t nclear0, nclear1;     // words in each
+    int32_t block_words;          // words per block in a maxima array (ways * way_stride)
     uint32_t* queue;              // sync counters of this step's update launches (HF_SLOTS x HF_SYNC_WORDS)
     int32_t nqueue;
     uint32_t* pending;            // pending bitmap of this step's check launch

@@ -44,7 +44,6 @@ struct hf_ctx {
     int maxnb = 1;
     int wg_cap = 1024;                            // resident workgroups of an update launch
     unsigned long long wait_ticks = 1000000;      // bound of an in-launch wait (s_memrealtime ticks)
-    int probe_max = 0;                            // HfStepArgs::probe_max of the context's launches
     int64_t total = 0;                            // elements per state buffer
     void* buf[2] = {nullptr, nullptr};
     int cur = 0;
@@ -58,10 +57,11 @@ struct hf_ctx {
     HfGhost* d_copy = nullptr;     // ghost identity table (copy ghosts between buffers)
     int nfill = 0, ncopy = 0;
     void* d_consts = nullptr;
-    unsigned long long* d_imax = nullptr;   // [2][nb][2]
+    unsigned long long* d_imax = nullptr;   // [2][nb][ways][way_stride]
+    int ways = 1, way_stride = 2;           // maxima slots per block, words per slot (HfStepArgs)
     unsigned long long* d_gmax = nullptr;   // [2][nb][2]
     unsigned long long* d_scan = nullptr;   // [nb][2] scan results + [nb][2] scratch maxima
-    unsigned long long* d_imax_fix = nullptr;   // [2][nb][2] maxima of blocks recomputed by the guess / check launch
+    unsigned long long* d_imax_fix = nullptr;   // [2][nb][ways][way_stride] maxima of blocks recomputed by the guess / check launch
     uint32_t* d_fixed = nullptr;                // [2][nb] block recomputed by the guess / check launch
     uint32_t* d_sync = nullptr;                 // [HF_SLOTS][HF_SYNC_WORDS] launch counters (HF_SLOT_MAIN, ..)
     int32_t* d_rounds = nullptr;                // plan_table(): round starts, main-list segments, fix-up ranges
@@ -91,6 +91,7 @@ struct hf_ctx {
     int64_t prof_launches = 0;
     double prof_ms = 0.0;
 
-    unsigned long long* imax(int parity) { return d_imax + (size_t)parity * nb * 2; }
+    size_t max_words() const { return (size_t)nb * ways * way_stride; }   // a maxima array
+    unsigned long long* imax(int parity) { return d_imax + parity * max_words(); }
     unsigned long long* gmax(int parity) { return d_gmax + (size_t)parity * nb * 2; }
 };

@@ -8,8 +8,7 @@
 // from HBM (plus the 2-lane halo at each strip edge and 2 halo rows per
 // strip) and every output written once; nothing intermediate goes to memory.
 // The new state's max wave speeds (for the next dt) are reduced in the same
-// pass: wave shuffles, then a 64-bit atomic max per wave (store_maxima; where
-// the host enables the probe, only from waves whose value raises the slot).
+// pass: wave shuffles, then a 64-bit atomic max per wave (store_maxima).
 //
 // The interior is read from A and the filled ghosts from G (the ghost fill
 // writes them into the destination buffer), so no launch ever reads a cell
@@ -89,8 +88,7 @@ __device__ __forceinline__ unsigned ticket_next(uint32_t* sync, int lane, unsign
 
 // What waves of one launch tell each other travels only through device-scope
 // atomics (wave-speed maxima, fixed flags, the pending bitmap, the counters):
-// writers update with atomic read-modify-writes (with the maxima probe, a
-// writer skips one that a coherent load shows cannot raise the slot), and
+// writers update with atomic read-modify-writes, and
 // readers of values that decide results read with coherent_read
 // (hf_physics.h), an atomic read-modify-write that changes nothing.  The new
 // states themselves are not read inside the launch.
@@ -140,37 +138,31 @@ __device__ __forceinline__ unsigned long long uniform_bits(double x)
     return ((unsigned long long)hi << 32) | lo;
 }
 
-// Raises the slot at p to the wave-uniform bits b.  A slot is cleared before
-// the launch that fills it and only grows during it, so a wave whose value
-// does not exceed the slot's current one (a coherent load) leaves it alone:
-// the same final maximum, and the device-scope atomics on one address, which
-// serialise, come only from the waves that raise it.  The load puts a memory
-// round trip at the end of the item: it pays where hundreds of items of one
-// block end together (the 8-block channel: 4 % per step) and costs where few
-// do (a 400^2 Godunov block: 15 %; 512 small blocks: 1.5 %), so the host
-// enables it per context (HfStepArgs::probe_max).
-__device__ __forceinline__ void raise_max(unsigned long long* p, unsigned long long b)
+// Where a wave's maxima go: an array of slots and the wave's own slot of a
+// block.  Device-scope atomics on one address take about 10 ns each, one
+// after the other, so the waves of a launch are spread over a.ways slots on
+// lines of their own (build_plan chooses how many).
+struct MaxOut {
+    unsigned long long* base;
+    int way;
+};
+template <class R>
+__device__ __forceinline__ MaxOut max_out(const HfStepArgs<R>& a, unsigned long long* base)
 {
-    const unsigned long long c = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)c);
-    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(c >> 32));
-    if ((((unsigned long long)hi << 32) | lo) < b) atomicMax(p, b);
+    return MaxOut{base, (int)(wave_id() & (unsigned)(a.ways - 1))};
 }
 
 // Per-wave maxima into the block's slots; every lane holds the reduced value.
 // The value is passed as a scalar: the compiler then issues one atomic from
 // one lane, instead of first reducing 64 lane values it cannot tell are equal
 // (a 64-iteration scalar loop per atomic).
-__device__ __forceinline__ void store_maxima(unsigned long long* out, int block, double mx, double my, bool probe)
+template <class R>
+__device__ __forceinline__ void store_maxima(const HfStepArgs<R>& a, const MaxOut& out, int block, double mx, double my)
 {
     const unsigned long long bx = uniform_bits(mx), by = uniform_bits(my);
-    if (probe) {
-        raise_max(&out[2 * block], bx);
-        raise_max(&out[2 * block + 1], by);
-    } else {
-        atomicMax(&out[2 * block], bx);
-        atomicMax(&out[2 * block + 1], by);
-    }
+    unsigned long long* p = out.base + HF_MAX_SLOT(block, out.way, a.ways, a.way_stride);
+    atomicMax(p, bx);
+    atomicMax(p + 1, by);
 }
 
 // Load row y of this lane's column: ghost rows/columns come from the ghost
@@ -298,7 +290,7 @@ __device__ __forceinline__ int muscl_rows_q64(const HfStepArgs<double>& a, const
 template <class M, int LIM, bool RESID, bool QUICK>
 __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, const HfItem it, const int lane,
                                            const double dt_step, const double dt_pred,
-                                           unsigned long long* __restrict__ imax_out)
+                                           const MaxOut& imax_out)
 {
     typedef typename M::R R;
 
@@ -391,7 +383,7 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
         for (int k = 0; k < 4; k++) { Gs[k] = Gn[k]; Tc[k] = Tn[k]; uc[k] = up[k]; up[k] = un[k]; un[k] = nn[k]; }
     }
     }
-    if (!RESID) store_maxima(imax_out, it.block, wave_max(mx), wave_max(my), a.probe_max != 0);
+    if (!RESID) store_maxima(a, imax_out, it.block, wave_max(mx), wave_max(my));
 #undef ROW
 }
 
@@ -511,7 +503,7 @@ __device__ __forceinline__ int muscl_cols_q64(const HfStepArgs<double>& a, const
 template <class M, int LIM, bool RESID, bool QUICK>
 __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a, const HfItem it, const int lane,
                                              const double dt_step, const double dt_pred,
-                                             unsigned long long* __restrict__ imax_out)
+                                             const MaxOut& imax_out)
 {
     typedef typename M::R R;
 
@@ -605,7 +597,7 @@ __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a,
         for (int k = 0; k < 4; k++) { Fw[k] = Fe[k]; Rc[k] = Rn[k]; uc[k] = up[k]; up[k] = un[k]; un[k] = nn[k]; }
     }
     }
-    if (!RESID) store_maxima(imax_out, it.block, wave_max(mx), wave_max(my), a.probe_max != 0);
+    if (!RESID) store_maxima(a, imax_out, it.block, wave_max(mx), wave_max(my));
 #undef COL
 }
 
@@ -663,7 +655,7 @@ __device__ __forceinline__ int round_of(const HfStepArgs<R>& a, unsigned idx)
 
 template <class M, int LIM, bool RESID, bool QUICK = true>
 __device__ __forceinline__ void muscl_go(const HfStepArgs<typename M::R>& a, const HfItem& it, int lane, double dt_step,
-                                         double dt_pred, unsigned long long* imax_out)
+                                         double dt_pred, const MaxOut& imax_out)
 {
     if (!RESID && item_transposed(it))
         muscl_item_t<M, LIM, RESID, QUICK>(a, it, lane, dt_step, dt_pred, imax_out);
@@ -780,7 +772,7 @@ __device__ __forceinline__ void main_item(const HfStepArgs<typename M::R>& a, un
         }
         record_dts<R>(a, it, bd, true, c_step, c_pred, c_kstep, c_kpred);
     }
-    muscl_go<M, LIM, RESID>(a, it, lane, c_step, c_pred, a.imax_new);
+    muscl_go<M, LIM, RESID>(a, it, lane, c_step, c_pred, max_out(a, a.imax_new));
 }
 
 template <class M, int LIM, bool RESID>
@@ -926,7 +918,7 @@ __global__ __launch_bounds__(256, 2) void k_muscl_guess(const HfStepArgs<typenam
             a.fixed[cb] = 1u;   // the same value from every wave
         }
         record_dts<R>(a, it, bd, false, dt_step, dt_pred, g.kstep, kpred);
-        muscl_go<M, LIM, false>(a, it, lane, dt_step, dt_pred, a.imax_fix);
+        muscl_go<M, LIM, false>(a, it, lane, dt_step, dt_pred, max_out(a, a.imax_fix));
     }
 }
 
@@ -949,7 +941,7 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
     }
     if (first > a.nrounds) return;   // every block has its exact dt
 
-    unsigned long long* imax_chk = a.imax_fix + 2 * a.nblocks;
+    const MaxOut imax_chk = {a.imax_fix + HF_MAX_SLOT(a.nblocks, 0, a.ways, a.way_stride), 0};
     uint32_t* fixed_chk = a.fixed + a.nblocks;
     const unsigned base = (unsigned)a.rounds[first];   // item of queue counter value 0
     int cached = -1, cp = -1;   // the block whose verdict this wave holds, the problem of its guess minimum
@@ -1098,7 +1090,7 @@ __device__ __forceinline__ int godunov_rows_q64(const HfStepArgs<double>& a, con
 // so the dt's chain of dependent loads overlaps their memory latency.
 template <class M, bool RESID, class DtOf>
 __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a, const HfItem it, const int lane,
-                                             DtOf&& dt_of, unsigned long long* __restrict__ imax_out)
+                                             DtOf&& dt_of, const MaxOut& imax_out)
 {
     typedef typename M::R R;
 
@@ -1166,7 +1158,7 @@ __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a,
         sc = sn;
     }
     }
-    if (!RESID) store_maxima(imax_out, it.block, wave_max(mx), wave_max(my), false);
+    if (!RESID) store_maxima(a, imax_out, it.block, wave_max(mx), wave_max(my));
 #undef ROW
 }
 
@@ -1190,7 +1182,7 @@ __global__ __launch_bounds__(256) void k_godunov(const HfStepArgs<typename M::R>
                 a.hist[hs - 1] = dt_step;
             return dt_step;
         };
-        godunov_item<M, RESID>(a, it, lane, dt_of, a.imax_new);
+        godunov_item<M, RESID>(a, it, lane, dt_of, max_out(a, a.imax_new));
     }
 }
 
@@ -1218,14 +1210,20 @@ __global__ __launch_bounds__(256) void k_ghost(const HfGhost* __restrict__ tab, 
     if (blockIdx.x == gridDim.x - 1) {
         for (int p = threadIdx.x; p < book.nprob && book.bump; p += blockDim.x)
             book.calls[p] += (uint32_t)book.probs[p].cps;
-        for (int i = threadIdx.x; i < book.nclear; i += blockDim.x) {
-            if (book.clear0) book.clear0[i] = 0ull;
-            if (book.clear1) book.clear1[i] = 0ull;
-        }
+        for (int i = threadIdx.x; i < book.nclear0; i += blockDim.x) book.clear0[i] = 0ull;
+        for (int i = threadIdx.x; i < book.nclear1; i += blockDim.x) book.clear1[i] = 0ull;
         for (int i = threadIdx.x; i < book.nqueue; i += blockDim.x) book.queue[i] = 0u;
         for (int i = threadIdx.x; i < book.npending; i += blockDim.x) book.pending[i] = 0u;
-        __syncthreads();   // the skip count below starts from zero
-        const int nb = book.nblocks;
+        const int nb = book.nblocks, bw = book.block_words;
+        // the check launch's recomputation over the guess launch's
+        for (int i = threadIdx.x; i < nb * bw && book.fixed; i += blockDim.x) {
+            const int b = i / bw;
+            const int s = book.fixed[nb + b] ? 1 : book.fixed[b] ? 0 : -1;
+            if (s >= 0) book.imax_prev[i] = book.imax_fix[s * nb * bw + i];
+            book.imax_fix[i] = 0ull;
+            book.imax_fix[nb * bw + i] = 0ull;
+        }
+        __syncthreads();   // the fixed flags are read; the skip count below starts from zero
         if (book.fixstats && book.fixed && threadIdx.x == 0) atomicAdd(&book.fixstats[0], 1ull);
         for (int b = threadIdx.x; b < nb && book.fixed; b += blockDim.x) {
             if (book.fixstats) {
@@ -1233,19 +1231,9 @@ __global__ __launch_bounds__(256) void k_ghost(const HfGhost* __restrict__ tab, 
                 if (book.fixed[b]) atomicAdd(&book.fixstats[2], 1ull);
                 if (book.fixed[nb + b]) atomicAdd(&book.fixstats[3], 1ull);
             }
-            // the check launch's recomputation over the guess launch's
-            const int s = book.fixed[nb + b] ? 1 : book.fixed[b] ? 0 : -1;
-            if (s >= 0) {
-                book.imax_prev[2 * b] = book.imax_fix[2 * (s * nb + b)];
-                book.imax_prev[2 * b + 1] = book.imax_fix[2 * (s * nb + b) + 1];
-            }
             book.skip[b] = book.skip_next[b];
             if (book.skip_next[b]) atomicAdd(&book.queue[HF_SLOT_MAIN * HF_SYNC_WORDS + HF_SYNC_NSKIP], 1u);
-            for (int t = 0; t < 2; t++) {
-                book.fixed[t * nb + b] = 0u;
-                book.imax_fix[2 * (t * nb + b)] = 0ull;
-                book.imax_fix[2 * (t * nb + b) + 1] = 0ull;
-            }
+            for (int t = 0; t < 2; t++) book.fixed[t * nb + b] = 0u;
         }
         return;
     }

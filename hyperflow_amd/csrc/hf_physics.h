@@ -759,12 +759,16 @@ __device__ __forceinline__ void step_dts(const HfStepArgs<R>& a, const HfBlockDe
     const HfProbDev pr = a.probs[bd.problem];
     kstep = (long long)a.calls[bd.problem] - pr.cps + 1;
     kpred = kstep + 1 + bd.lb;
+    // A lane takes one slot of a block: the quotient by the largest of a
+    // block's maxima is the least of the quotients by each.
     double dtx = 1e16, dty = 1e16;
-    const int end = pr.first + pr.nb;
-    for (int c = pr.first + (int)(threadIdx.x & 63); c < end; c += 64) {
+    const int n = pr.nb * a.ways;
+    for (int e = (int)(threadIdx.x & 63); e < n; e += 64) {
+        const int c = pr.first + e / a.ways;
+        const int64_t s = HF_MAX_SLOT(pr.first, e, a.ways, a.way_stride);
         const double cdx = a.blocks[c].dx, cdy = a.blocks[c].dy;
         const double gx = bitsd(a.gmax[2 * c]), gy = bitsd(a.gmax[2 * c + 1]);
-        const double ox = smax(bitsd(a.imax_old[2 * c]), gx), oy = smax(bitsd(a.imax_old[2 * c + 1]), gy);
+        const double ox = smax(bitsd(a.imax_old[s]), gx), oy = smax(bitsd(a.imax_old[s + 1]), gy);
         dtx = smin(dtx, cdx / ox);
         dty = smin(dty, cdy / oy);
     }
@@ -785,21 +789,34 @@ __device__ __forceinline__ void step_dts(const HfStepArgs<R>& a, const HfBlockDe
 // cfl_eff(k_l) * min(1e16, min over all c of old_c); the step dt is
 // cfl_eff(k_step) times the same minimum.
 
-template <class R>
-__device__ __forceinline__ double term_old(const HfStepArgs<R>& a, int c)
-{
-    const double cdx = a.blocks[c].dx, cdy = a.blocks[c].dy;
-    const double gx = bitsd(a.gmax[2 * c]), gy = bitsd(a.gmax[2 * c + 1]);
-    return smin(cdx / smax(bitsd(a.imax_old[2 * c]), gx), cdy / smax(bitsd(a.imax_old[2 * c + 1]), gy));
-}
-
-// pre_c from the given new maxima bit patterns
+// min(dx_c / mx, dy_c / my) for the given maxima bit patterns of block c's
+// interior and its ghosts'
 template <class R>
 __device__ __forceinline__ double term_new(const HfStepArgs<R>& a, int c, unsigned long long mx, unsigned long long my)
 {
     const double cdx = a.blocks[c].dx, cdy = a.blocks[c].dy;
     const double gx = bitsd(a.gmax[2 * c]), gy = bitsd(a.gmax[2 * c + 1]);
     return smin(cdx / smax(bitsd(mx), gx), cdy / smax(bitsd(my), gy));
+}
+
+// The same from the block's slots in a maxima array
+template <class R>
+__device__ __forceinline__ double term_slots(const HfStepArgs<R>& a, int c, const unsigned long long* m)
+{
+    const unsigned long long* p = m + HF_MAX_SLOT(c, 0, a.ways, a.way_stride);
+    unsigned long long mx = p[0], my = p[1];
+    for (int w = 1; w < a.ways; w++) {
+        const unsigned long long x = p[(int64_t)w * a.way_stride], y = p[(int64_t)w * a.way_stride + 1];
+        mx = x > mx ? x : mx;
+        my = y > my ? y : my;
+    }
+    return term_new(a, c, mx, my);
+}
+
+template <class R>
+__device__ __forceinline__ double term_old(const HfStepArgs<R>& a, int c)
+{
+    return term_slots(a, c, a.imax_old);
 }
 
 // Which maxima are final for pre_c:
@@ -829,15 +846,14 @@ __device__ __forceinline__ unsigned long long coherent_read(unsigned long long* 
 template <class R, int SRC>
 __device__ __forceinline__ double term_pre(const HfStepArgs<R>& a, int nb_all, int c)
 {
-    unsigned long long* fix1 = a.imax_fix + 2 * nb_all;
+    unsigned long long* fix1 = a.imax_fix + HF_MAX_SLOT(nb_all + c, 0, a.ways, a.way_stride);
     if (SRC == PRE_CHECK) {
         const bool f2 = coherent_read(&a.fixed[nb_all + c]) != 0u;
-        const unsigned long long x2 = coherent_read(&fix1[2 * c]);
-        const unsigned long long y2 = coherent_read(&fix1[2 * c + 1]);
+        const unsigned long long x2 = coherent_read(&fix1[0]);
+        const unsigned long long y2 = coherent_read(&fix1[1]);
         if (f2) return term_new(a, c, x2, y2);
     }
-    if (SRC != PRE_MAIN && a.fixed[c]) return term_new(a, c, a.imax_fix[2 * c], a.imax_fix[2 * c + 1]);
-    return term_new(a, c, a.imax_new[2 * c], a.imax_new[2 * c + 1]);
+    return term_slots(a, c, (SRC != PRE_MAIN && a.fixed[c]) ? a.imax_fix : a.imax_new);
 }
 
 // Inclusive minimum over lanes 0..lane (scan_lo) or lane..63 (scan_hi).

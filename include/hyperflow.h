@@ -77,7 +77,8 @@ typedef struct {
     double cfl;              /* TimeStep(model, cfl), timestep.cpp:14-21 */
     int32_t nblocks;
     /* Work plan of the update launches (results do not depend on it; 0 = the
-     * library default): rows a wave sweeps per item of the main list, rows per
+     * library default): rows a wave sweeps per item of the main list (at most:
+     * fewer where one round of the resident waves takes smaller items), rows per
      * item of the main list's closing phase, rows per item of the fix-up
      * rounds of the compat predictor dt. */
     int32_t tile_rows;

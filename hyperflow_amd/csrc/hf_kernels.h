@@ -976,7 +976,11 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
                 c_need = check_verdict<R>(a, bd.problem, pr, a.nblocks, bd.lb, cm, c_step, c_pred, c_kstep, c_kpred);
             }
             if (c_need) {
-                atomicExch(&fixed_chk[it.block], 1u);
+                // Or, not an exchange: the compiler leaves one lane's of an or
+                // with one value for the wave, and 64 of an exchange, which
+                // took 1.3 ms of the 1.5 ms a recomputed 1024^2 block cost
+                // (the channel's first 200 steps: 2.9 -> 0.83 ms per step).
+                atomicOr(&fixed_chk[it.block], 1u);
                 record_dts<R>(a, it, bd, false, c_step, c_pred, c_kstep, c_kpred);
                 muscl_go<M, LIM, false>(a, it, lane, c_step, c_pred, imax_chk);
             }
@@ -1003,7 +1007,7 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
             long long kstep, kpred;
             guess_plan<R>(a, bd.problem, pr, O, mg, kstep);
             if (check_verdict<R>(a, bd.problem, pr, a.nblocks, bd.lb, mg, dt_step, dt_pred, kstep, kpred)) {
-                atomicExch(&fixed_chk[it.block], 1u);
+                atomicOr(&fixed_chk[it.block], 1u);
                 record_dts<R>(a, it, bd, false, dt_step, dt_pred, kstep, kpred);
                 muscl_go<M, LIM, false, false>(a, it, lane, dt_step, dt_pred, imax_chk);   // rare: the general rows only
                 __builtin_amdgcn_s_waitcnt(0xF70);   // its maxima are performed before the next verdict reads them

@@ -376,14 +376,19 @@ int launch_ghost(hf_ctx* c, const HfGhost* tab, int n, const void* S, void* D, u
     return HF_OK;
 }
 
-int launch_scan(hf_ctx* c, int b, const void* I, const void* Gh, int interior_only, unsigned long long* out)
+// Wave-speed maxima of blocks [b0, b1): the interior into imax-style slots, or
+// (slots = false) every padded cell into [nb][2].
+int launch_scan(hf_ctx* c, int b0, int b1, const void* S, bool slots, unsigned long long* out)
 {
+    const HfItem* items = c->d_scan_items + c->scan_begin[b0];
+    const int n = c->scan_begin[b1] - c->scan_begin[b0];
+    const int ways = slots ? c->ways : 1, stride = slots ? c->way_stride : 2;
     if (c->prec == HF_FP64)
-        HF_HIP(hf::launch_scan<double>(c->blocks[b], (const double*)I, (const double*)Gh, interior_only, c->gamma, out,
-                                       c->stream));
+        HF_HIP(hf::launch_scan<double>(items, n, c->d_blocks, (const double*)S, (const double*)S, slots, c->gamma, out,
+                                       ways, stride, c->stream));
     else
-        HF_HIP(hf::launch_scan<float>(c->blocks[b], (const float*)I, (const float*)Gh, interior_only, c->gamma, out,
-                                      c->stream));
+        HF_HIP(hf::launch_scan<float>(items, n, c->d_blocks, (const float*)S, (const float*)S, slots, c->gamma, out,
+                                      ways, stride, c->stream));
     return HF_OK;
 }
 
@@ -407,9 +412,9 @@ int full_dt(hf_ctx* c, int p, F src, double* dt)
 {
     const HfProbDev& P = c->probs[p];
     HF_HIP(hipMemsetAsync(c->d_scan, 0, sizeof(unsigned long long) * 2 * c->nb, c->stream));
-    for (int q = P.first; q < P.first + P.nb; q++) {
-        const void* s = src(q);
-        int rc = launch_scan(c, q, s, s, 0, c->d_scan + 2 * q);
+    for (int q = P.first, r; q < P.first + P.nb; q = r) {   // runs of blocks from one buffer
+        for (r = q + 1; r < P.first + P.nb && src(r) == src(q); r++) {}
+        int rc = launch_scan(c, q, r, src(q), false, c->d_scan);
         if (rc) return rc;
     }
     std::vector<unsigned long long> mx(2 * c->nb);
@@ -433,16 +438,17 @@ int full_dt(hf_ctx* c, int p, F src, double* dt)
 int ensure_partials(hf_ctx* c)
 {
     if (c->partials_valid) return HF_OK;
-    HF_HIP(hipMemsetAsync(c->imax(c->cur), 0, sizeof(unsigned long long) * c->max_words(), c->stream));
-    HF_HIP(hipMemsetAsync(c->gmax(c->cur), 0, sizeof(unsigned long long) * 2 * c->nb, c->stream));
-    HF_HIP(hipMemsetAsync(c->d_imax_fix, 0, sizeof(unsigned long long) * 2 * c->max_words(), c->stream));
-    HF_HIP(hipMemsetAsync(c->d_fixed, 0, sizeof(uint32_t) * 2 * c->nb, c->stream));
-    HF_HIP(hipMemsetAsync(c->d_skip_next, 0, sizeof(uint32_t) * c->nb, c->stream));
-    for (int b = 0; b < c->nb; b++) {
-        int rc = launch_scan(c, b, c->buf[c->cur], c->buf[c->cur], 1,
-                             c->imax(c->cur) + HF_MAX_SLOT(b, 0, c->ways, c->way_stride));
-        if (rc) return rc;
-    }
+    hf::ClearArgs z;
+    std::memset(&z, 0, sizeof z);
+    auto clear = [&, k = 0](void* p, size_t words) mutable { z.p[k] = (uint32_t*)p; z.n[k++] = (int)words; };
+    clear(c->imax(c->cur), 2 * c->max_words());
+    clear(c->gmax(c->cur), 4 * (size_t)c->nb);
+    clear(c->d_imax_fix, 4 * c->max_words());
+    clear(c->d_fixed, 2 * (size_t)c->nb);
+    clear(c->d_skip_next, (size_t)c->nb);
+    HF_HIP(hf::launch_clear(z, c->stream));
+    int rc = launch_scan(c, 0, c->nb, c->buf[c->cur], true, c->imax(c->cur));
+    if (rc) return rc;
     c->partials_valid = true;
     return HF_OK;
 }
@@ -613,6 +619,14 @@ int build_plan(hf_ctx* c, const hf_case_desc* desc, bool dense)
         c->resid_elems = std::max<int64_t>(c->resid_elems, 4 * B.plane);
     }
     c->total = off;
+    // scan items: about 4 k cells each, at least a row per wave
+    for (int b = 0; b < c->nb; b++) {
+        const HfBlockDev& B = c->blocks[b];
+        c->scan_begin.push_back((int)c->scan_items.size());
+        const int rows = std::max(4, 4096 / B.tx);
+        for (int y = 0; y < B.ty; y += rows) c->scan_items.push_back(HfItem{b, 0, y, std::min(rows, B.ty - y)});
+    }
+    c->scan_begin.push_back((int)c->scan_items.size());
     // problems
     for (int b = 0; b < c->nb; b++) {
         const int p = c->blocks[b].problem;
@@ -870,6 +884,8 @@ int hf_create(const hf_case_desc* desc, hf_ctx** out)
     HF_HIPC(hipMemcpy(C->d_probs, C->probs.data(), sizeof(HfProbDev) * C->np, hipMemcpyHostToDevice));
     HF_HIPC(hipMalloc(&C->d_items, sizeof(HfItem) * C->items.size()));
     HF_HIPC(hipMemcpy(C->d_items, C->items.data(), sizeof(HfItem) * C->items.size(), hipMemcpyHostToDevice));
+    HF_HIPC(hipMalloc(&C->d_scan_items, sizeof(HfItem) * C->scan_items.size()));
+    HF_HIPC(hipMemcpy(C->d_scan_items, C->scan_items.data(), sizeof(HfItem) * C->scan_items.size(), hipMemcpyHostToDevice));
     HF_HIPC(hipMalloc(&C->d_fill, sizeof(HfGhost) * fill.size()));
     HF_HIPC(hipMemcpy(C->d_fill, fill.data(), sizeof(HfGhost) * fill.size(), hipMemcpyHostToDevice));
     HF_HIPC(hipMalloc(&C->d_copy, sizeof(HfGhost) * copy.size()));
@@ -938,7 +954,7 @@ void hf_destroy(hf_ctx* c)
     destroy_graphs(c);
     for (auto& e : c->ev_pending) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
     for (auto& e : c->ev_free) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
-    for (void* p : {c->buf[0], c->buf[1], (void*)c->d_blocks, (void*)c->d_probs, (void*)c->d_items, (void*)c->d_fill,
+    for (void* p : {c->buf[0], c->buf[1], (void*)c->d_blocks, (void*)c->d_probs, (void*)c->d_items, (void*)c->d_scan_items, (void*)c->d_fill,
                     (void*)c->d_copy, c->d_consts, (void*)c->d_imax, (void*)c->d_gmax, (void*)c->d_scan,
                     (void*)c->d_calls, (void*)c->d_hist, (void*)c->d_part, c->d_resid, (void*)c->d_imax_fix,
                     (void*)c->d_fixed, (void*)c->d_fixstats, (void*)c->d_sync, (void*)c->d_rounds, (void*)c->d_pending, (void*)c->d_skip,
@@ -1247,7 +1263,7 @@ int hf_step_noalloc(const hf_case_desc* desc, const void* d_in, void* d_out, int
     };
     const size_t nb = (size_t)c.nb, np = (size_t)c.np;
     const size_t o_blocks = take(sizeof(HfBlockDev) * nb), o_probs = take(sizeof(HfProbDev) * np),
-                 o_items = take(sizeof(HfItem) * c.items.size()), o_fill = take(sizeof(HfGhost) * fill.size()),
+                 o_items = take(sizeof(HfItem) * c.items.size()), o_scan = take(sizeof(HfItem) * c.scan_items.size()), o_fill = take(sizeof(HfGhost) * fill.size()),
                  o_consts = take(c.esize * 16 * nb), o_imax = take(sizeof(unsigned long long) * 2 * c.max_words()),
                  o_gmax = take(sizeof(unsigned long long) * 4 * nb),
                  o_fix = take(sizeof(unsigned long long) * 2 * c.max_words()), o_fixed = take(sizeof(uint32_t) * 2 * nb),
@@ -1267,6 +1283,7 @@ int hf_step_noalloc(const hf_case_desc* desc, const void* d_in, void* d_out, int
     std::memcpy(img.data() + o_blocks, c.blocks.data(), sizeof(HfBlockDev) * nb);
     std::memcpy(img.data() + o_probs, c.probs.data(), sizeof(HfProbDev) * np);
     std::memcpy(img.data() + o_items, c.items.data(), sizeof(HfItem) * c.items.size());
+    std::memcpy(img.data() + o_scan, c.scan_items.data(), sizeof(HfItem) * c.scan_items.size());
     std::memcpy(img.data() + o_fill, fill.data(), sizeof(HfGhost) * fill.size());
     for (size_t b = 0; b < nb; b++)
         for (int sd = 0; sd < 4; sd++)
@@ -1297,6 +1314,7 @@ int hf_step_noalloc(const hf_case_desc* desc, const void* d_in, void* d_out, int
     c.d_blocks = (HfBlockDev*)(S + o_blocks);
     c.d_probs = (HfProbDev*)(S + o_probs);
     c.d_items = (HfItem*)(S + o_items);
+    c.d_scan_items = (HfItem*)(S + o_scan);
     c.d_fill = (HfGhost*)(S + o_fill);
     c.nfill = (int)fill.size();
     c.d_consts = S + o_consts;
@@ -1317,10 +1335,8 @@ int hf_step_noalloc(const hf_case_desc* desc, const void* d_in, void* d_out, int
     HF_HIP(hipMemcpyAsync(base, img.data(), used, hipMemcpyHostToDevice, c.stream));
     // wave-speed maxima of the input's interior (a device-resident loop gets
     // them from the previous step's update epilogue)
-    for (int b = 0; b < c.nb; b++) {
-        rc = launch_scan(&c, b, d_in, d_in, 1, c.imax(0) + HF_MAX_SLOT(b, 0, c.ways, c.way_stride));
-        if (rc) return rc;
-    }
+    rc = launch_scan(&c, 0, c.nb, d_in, true, c.imax(0));
+    if (rc) return rc;
     rc = enqueue_steps(&c, 1, false);
     if (rc) return rc;
     // the host image must outlive its copy, and the caller gets a finished step

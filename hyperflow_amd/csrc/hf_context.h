@@ -40,6 +40,9 @@ struct hf_ctx {
     std::vector<std::pair<int, int>> fix_rounds;  // item ranges of the fix-up launches (lb = 1, 2, ..)
     std::vector<int32_t> segs;       // [3][nb][2] (first, count) of each block in the main list's phases
     std::vector<int32_t> fixrange;   // [nb][2] (first, count) of each block in the fix-up rounds
+    std::vector<HfItem> scan_items;  // rows of every block for the wave-speed scan, block by block
+    std::vector<int> scan_begin;     // [nb + 1] first scan item of each block
+    HfItem* d_scan_items = nullptr;
     int main_begin = 0, main_items = 0;           // item range of a step's main launch
     int maxnb = 1;
     int wg_cap = 1024;                            // resident workgroups of an update launch

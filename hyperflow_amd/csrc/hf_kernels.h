@@ -1322,33 +1322,53 @@ __global__ __launch_bounds__(256) void k_ghost(const HfGhost* __restrict__ tab, 
 }
 
 // -------------------------------------------------------------- wave scan --
-// Max of |u|+c and |v|+c over cells of one block (TimeStep::operator(),
-// timestep.cpp:37-55).  Interior cells are read from I, ghost cells from Gh;
-// with interior_only the ghosts are skipped.
+// Max of |u|+c and |v|+c over cells of blocks (TimeStep::operator(),
+// timestep.cpp:37-55), one workgroup per item (rows [y0, y0 + rows) of a
+// block, lanes along x, a wave per row): interior cells are read from I, ghost
+// cells from Gh; with interior_only the ghosts are skipped.  Reads each value
+// once; HBM bounds it.  One atomic pair per workgroup, on the block's slots:
+// with one per wave on one word the scan of 1024^2 FP64 cells took 375 us, of
+// 8192^2 FP32 506, of 512 blocks (a launch each) 17 ms; now 20, 331 and 166 us.
 template <class M>
-__global__ __launch_bounds__(256) void k_scan(HfBlockDev bd, const typename M::R* __restrict__ I,
-                                              const typename M::R* __restrict__ Gh, int interior_only,
-                                              double gamma, unsigned long long* outmax)
+__global__ __launch_bounds__(256) void k_scan(const HfItem* __restrict__ items, const HfBlockDev* __restrict__ blocks,
+                                              const typename M::R* __restrict__ I,
+                                              const typename M::R* __restrict__ Gh, int interior_only, double gamma,
+                                              unsigned long long* outmax, int ways, int stride)
 {
     typedef typename M::R R;
-    const int64_t n = (int64_t)bd.tx * bd.ty;
+    const HfItem it = items[blockIdx.x];
+    const HfBlockDev bd = blocks[it.block];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     double mx = 0.0, my = 0.0;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int y = (int)(i / bd.tx), x = (int)(i % bd.tx);
-        const bool gh = x < bd.g || x >= bd.tx - bd.g || y < bd.g || y >= bd.ty - bd.g;
-        if (gh && interior_only) continue;
-        R u[4];
-        load_cell<R>((gh ? Gh : I) + bd.off + (int64_t)y * bd.pitch + x, bd.plane, u);
-        double dx_, dy_;
-        wave_speeds<M>(u[0], u[1], u[2], u[3], R(gamma), R(gamma - 1.0), dx_, dy_);
-        mx = dmax_nan(mx, dx_);
-        my = dmax_nan(my, dy_);
+    for (int y = it.y0 + w; y < it.y0 + it.rows; y += 4) {
+        const bool gy = y < bd.g || y >= bd.ty - bd.g;
+        if (gy && interior_only) continue;
+        const int64_t row = bd.off + (int64_t)y * bd.pitch;
+#pragma unroll 4
+        for (int x = lane; x < bd.tx; x += 64) {
+            const bool gh = gy || x < bd.g || x >= bd.tx - bd.g;
+            if (gh && interior_only) continue;
+            R u[4];
+            load_cell<R>((gh ? Gh : I) + row + x, bd.plane, u);
+            double dx_, dy_;
+            wave_speeds<M>(u[0], u[1], u[2], u[3], R(gamma), R(gamma - 1.0), dx_, dy_);
+            mx = dmax_nan(mx, dx_);
+            my = dmax_nan(my, dy_);
+        }
     }
+    __shared__ double sx[4], sy[4];
     mx = wave_max(mx);
     my = wave_max(my);
-    if ((threadIdx.x & 63) == 0) {
-        atomicMax(&outmax[0], dbits(mx));
-        atomicMax(&outmax[1], dbits(my));
+    if (lane == 0) {
+        sx[w] = mx;
+        sy[w] = my;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {   // thread 0: x, thread 1: y
+        const double* s = threadIdx.x == 0 ? sx : sy;
+        double m = s[0];
+        for (int k = 1; k < 4; k++) m = s[k] > m ? s[k] : m;
+        atomicMax(outmax + HF_MAX_SLOT(it.block, blockIdx.x & (ways - 1), ways, stride) + threadIdx.x, dbits(m));
     }
 }
 

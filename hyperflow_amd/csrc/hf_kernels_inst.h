@@ -73,13 +73,13 @@ hipError_t launch_ghost<Real>(const HfGhost* tab, int n, const HfBlockDev* block
 }
 
 template <>
-hipError_t launch_scan<Real>(const HfBlockDev& bd, const Real* I, const Real* Gh, int interior_only, double gamma,
-                             unsigned long long* out, hipStream_t s)
+hipError_t launch_scan<Real>(const HfItem* items, int n, const HfBlockDev* blocks, const Real* I, const Real* Gh,
+                             int interior_only, double gamma, unsigned long long* out, int ways, int stride,
+                             hipStream_t s)
 {
-    const long long cells = (long long)bd.tx * bd.ty;
-    long long nb = (cells + 255) / 256;
-    if (nb > 4096) nb = 4096;
-    hipLaunchKernelGGL((k_scan<Math>), dim3((unsigned)nb), dim3(256), 0, s, bd, I, Gh, interior_only, gamma, out);
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL((k_scan<Math>), dim3((unsigned)n), dim3(256), 0, s, items, blocks, I, Gh, interior_only, gamma,
+                       out, ways, stride);
     return hipGetLastError();
 }
 

@@ -24,9 +24,18 @@ int update_wgs_per_cu(int scheme, int limiter, bool resid);
 template <class R>
 hipError_t launch_ghost(const HfGhost* tab, int n, const HfBlockDev* blocks, const R* S, R* D, const R* consts,
                         unsigned long long* gmax, double gamma, const GhostBook& book, hipStream_t s);
+// Wave-speed maxima of the items (rows of blocks) [0, n) raised into out, laid
+// out with `ways` slots of `stride` words per block.
 template <class R>
-hipError_t launch_scan(const HfBlockDev& bd, const R* I, const R* Gh, int interior_only, double gamma,
-                       unsigned long long* out, hipStream_t s);
+hipError_t launch_scan(const HfItem* items, int n, const HfBlockDev* blocks, const R* I, const R* Gh,
+                       int interior_only, double gamma, unsigned long long* out, int ways, int stride, hipStream_t s);
+// Zeroes up to HF_CLEARS arrays of 32-bit words in one launch.
+constexpr int HF_CLEARS = 6;
+struct ClearArgs {
+    uint32_t* p[HF_CLEARS];
+    int n[HF_CLEARS];
+};
+hipError_t launch_clear(const ClearArgs& a, hipStream_t s);
 template <class R>
 hipError_t launch_conserve(const HfBlockDev& bd, const R* A, double* part, int nwg, hipStream_t s);
 

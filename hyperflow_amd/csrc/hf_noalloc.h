@@ -4,7 +4,7 @@
 
 // Size of the per-GPU scratch array: enough for the tables and working arrays
 // of, e.g., one 8192^2 block or 512 blocks of up to 512^2 cells.
-#define HF_NOALLOC_SCRATCH_BYTES (32u << 20)
+#define HF_NOALLOC_SCRATCH_BYTES (40u << 20)
 #define HF_NOALLOC_MAX_DEVICES 64
 
 // Device address of the current device's scratch array (looked up with

@@ -170,7 +170,7 @@ HF_API int hf_conservation(hf_ctx* ctx, int problem, double sums[4]);
  *    this step in call order (1 for Godunov, 1 + blocks for MUSCL-Hancock).
  *  - stream: a hipStream_t, or NULL for the null stream.  Returns when the
  *    step is complete.
- * Tables and working arrays live in one static device array per GPU (32 MiB);
+ * Tables and working arrays live in one static device array per GPU (40 MiB);
  * a case that needs more is rejected with HF_EINVAL.  Every call on a GPU
  * shares that array: calls that overlap on one GPU (other threads or
  * streams) race and must be serialised by the caller. */

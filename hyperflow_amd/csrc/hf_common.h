@@ -11,6 +11,8 @@ struct HfBlockDev {
     int32_t problem;  // owning problem (dt group)
     int32_t lb;       // block index inside its problem
     int32_t g;        // ghost layers
+    int32_t reflect;  // bit s: side s (HF_BOTTOM..HF_LEFT) is reflective
+    int32_t pad;
     double dx, dy;
 };
 
@@ -63,6 +65,17 @@ struct HfStepArgs {
     int32_t hist_cap;
     int32_t dt_mode;                     // 0 compat, 1 uniform
     double gamma, cfl;
+    // Mirrored launches (a context whose problems are single blocks with
+    // transmissive and reflective sides only): ghost cells are read where they
+    // mirror to, G is not read, and the launch's last workgroup keeps the
+    // step's books -- calls holds the counts before this step and calls_next
+    // receives them after it, clear (the maxima of the step after next) and
+    // clear_sync (the next launch's counters) are zeroed, fixstats[0] counts.
+    int32_t mirrored, nclear;
+    unsigned long long* clear;
+    uint32_t* calls_next;
+    uint32_t* clear_sync;
+    unsigned long long* fixstats;
     int32_t use_fixed;                   // 1: dt_step/dt_pred below instead of the device partials
     int32_t nmain;                       // items [0, nmain) form the main list, the rest the fix-up rounds
     double fixed_step, fixed_pred;

@@ -60,7 +60,7 @@ struct hf_ctx {
     HfGhost* d_copy = nullptr;     // ghost identity table (copy ghosts between buffers)
     int nfill = 0, ncopy = 0;
     void* d_consts = nullptr;
-    unsigned long long* d_imax = nullptr;   // [2][nb][ways][way_stride]
+    unsigned long long* d_imax = nullptr;   // [3][nb][ways][way_stride], two used unless mirrored
     int ways = 1, way_stride = 2;           // maxima slots per block, words per slot (HfStepArgs)
     unsigned long long* d_gmax = nullptr;   // [2][nb][2]
     unsigned long long* d_scan = nullptr;   // [nb][2] scan results + [nb][2] scratch maxima
@@ -85,8 +85,8 @@ struct hf_ctx {
     int64_t resid_elems = 0;
     std::vector<int64_t> calls;     // host mirror of the TimeStep call counters
     hipStream_t stream = nullptr;
-    // captured step loops by (steps, start parity, fixed-dt bits or 0 for the CFL dt)
-    std::map<std::tuple<int, int, uint64_t>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
+    // captured step loops by (steps, start parity, fixed-dt bits or 0 for the CFL dt, turn)
+    std::map<std::tuple<int, int, uint64_t, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
 
     int profile = 0;                 // 0 off, else time the launches of every profile-th step
     int64_t prof_step = 0;
@@ -95,6 +95,12 @@ struct hf_ctx {
     double prof_ms = 0.0;
 
     size_t max_words() const { return (size_t)nb * ways * way_stride; }   // a maxima array
+    // Mirrored steps (HfStepArgs::mirrored): three maxima buffers take turns as
+    // the read, the written and the cleared one, the maxima of buf[cur] in
+    // imax(turn); ghost layers are filled once, after the last step of a run.
+    bool mirrored = false;
+    int turn = 0;
+    int now() const { return mirrored ? turn : cur; }   // which imax describes buf[cur]
     unsigned long long* imax(int parity) { return d_imax + parity * max_words(); }
     unsigned long long* gmax(int parity) { return d_gmax + (size_t)parity * nb * 2; }
 };

@@ -11,8 +11,9 @@
 // pass: wave shuffles, then a 64-bit atomic max per wave (store_maxima).
 //
 // The interior is read from A and the filled ghosts from G (the ghost fill
-// writes them into the destination buffer), so no launch ever reads a cell
-// that another wave of the same step writes.
+// writes them into the destination buffer), or ghosts are read from A where
+// they mirror to (Lines), so no launch ever reads a cell that another wave of
+// the same step writes.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -58,7 +59,8 @@ __device__ __forceinline__ float shfl_dn1(float x) { return __int_as_float(dpp_d
 // region surrounds the loop's exit test; lane 0's old value is the wave's
 // ticket.  A lane-0-only branch here let the compiler's control-flow
 // structurizer keep lanes 1..63 in the loop after lane 0 left it.
-__device__ __forceinline__ unsigned total_waves() { return gridDim.x * (blockDim.x >> 6); }
+// (the last workgroup of a mirrored launch, `extra`, takes none)
+__device__ __forceinline__ unsigned total_waves(unsigned extra = 0) { return (gridDim.x - extra) * (blockDim.x >> 6); }
 __device__ __forceinline__ unsigned wave_id()
 {
     // wave-uniform, but derived from threadIdx: say so, or the whole item loop
@@ -75,14 +77,14 @@ __device__ __forceinline__ unsigned next_ticket(uint32_t* sync, int lane, unsign
 // most its own item and no wave touches the counter: a wave would only learn
 // there that the list is done, and those atomics all arrive together when the
 // waves finish together and serialise at the counter.
-__device__ __forceinline__ unsigned ticket_first(unsigned n)
+__device__ __forceinline__ unsigned ticket_first(unsigned n, unsigned extra = 0)
 {
     const unsigned w = wave_id();
-    return (n <= total_waves() && w >= n) ? n : w;   // otherwise w < waves < n
+    return (n <= total_waves(extra) && w >= n) ? n : w;   // otherwise w < waves < n
 }
-__device__ __forceinline__ unsigned ticket_next(uint32_t* sync, int lane, unsigned n)
+__device__ __forceinline__ unsigned ticket_next(uint32_t* sync, int lane, unsigned n, unsigned extra = 0)
 {
-    const unsigned nw = total_waves();
+    const unsigned nw = total_waves(extra);
     return n <= nw ? n : next_ticket(sync, lane, nw);
 }
 
@@ -165,17 +167,85 @@ __device__ __forceinline__ void store_maxima(const HfStepArgs<R>& a, const MaxOu
     atomicMax(p + 1, by);
 }
 
-// Load row y of this lane's column: ghost rows/columns come from the ghost
-// source, interior cells from the interior source.
-template <class R>
-__device__ __forceinline__ void load_row(const R* __restrict__ Acol, const R* __restrict__ Gcol, bool gcol, int y,
-                                         int g, int ty, int pitch, int64_t plane, R u[4])
+// x with its sign flipped where m (0 or the sign bit of a 32-bit word) says so.
+__device__ __forceinline__ double flip_sign(double x, unsigned m)
 {
-    const bool gh = gcol || y < g || y >= ty - g;
-    load_cell<R>((gh ? Gcol : Acol) + (int64_t)y * pitch, plane, u);
+    return __longlong_as_double(__double_as_longlong(x) ^ ((long long)((unsigned long long)m << 32)));
 }
+__device__ __forceinline__ float flip_sign(float x, unsigned m) { return __uint_as_float(__float_as_uint(x) ^ m); }
+
+// A sweep's source of rows (T = false: lane l owns column x0 + l, lines are
+// rows) or columns (T = true: lane l owns row y0 + l).  Ghost cells come from
+// the filled ghost buffer; in a mirrored launch from the interior cell they
+// mirror to, with the momentum normal to a reflective side negated (the fill
+// of such a block puts the same values there: transmissive_boundary.cpp:25-104,
+// reflective_boundary.cpp:25-120).  Corner ghosts, which no sweep uses, read
+// cells inside the buffer.
+template <class R, bool T>
+struct Lines {
+    const R* A;      // this lane's cell of line 0 (interior lines)
+    const R* G;      // the same for ghost lines
+    int64_t step, plane;
+    int n, g;        // lines, ghost layers
+    unsigned flip;   // this lane is mirrored at a reflective side
+    unsigned lo, hi; // ghost lines below / above are mirrored at a reflective side
+    bool mirrored;
+
+    __device__ __forceinline__ Lines(const HfStepArgs<R>& a, const HfBlockDev& bd, int c)
+    {
+        mirrored = a.mirrored != 0;
+        plane = bd.plane;
+        g = bd.g;
+        n = T ? bd.tx : bd.ty;
+        step = T ? 1 : bd.pitch;
+        const int m = T ? bd.ty : bd.tx;                    // lanes' extent
+        const int64_t cs = T ? bd.pitch : 1;
+        const bool below = c < g, ghost = below || c >= m - g;
+        const int low = T ? 0 : 3, high = T ? 2 : 1;        // HF_BOTTOM/HF_TOP, HF_LEFT/HF_RIGHT
+        const int llow = T ? 3 : 0, lhigh = T ? 1 : 2;
+        flip = 0u;
+        lo = hi = 0u;
+        if (mirrored) {
+            const int cm = !ghost ? c : below ? 2 * g - 1 - c : 2 * (m - g) - 1 - c;
+            flip = (ghost && ((bd.reflect >> (below ? low : high)) & 1)) ? 0x80000000u : 0u;
+            lo = ((bd.reflect >> llow) & 1) ? 0x80000000u : 0u;
+            hi = ((bd.reflect >> lhigh) & 1) ? 0x80000000u : 0u;
+            A = a.A + bd.off + cm * cs;
+            G = A;
+        } else {
+            G = a.G + bd.off + c * cs;
+            A = ghost ? G : a.A + bd.off + c * cs;
+        }
+    }
+    // Requests line y into u: signs are applied by signed_line() with the
+    // returned mask, apart, so that nothing waits for the load here.
+    __device__ __forceinline__ unsigned operator()(int y, R u[4]) const
+    {
+        const bool below = y < g, ghost = below || y >= n - g;   // wave-uniform
+        const int ym = !(ghost && mirrored) ? y : below ? 2 * g - 1 - y : 2 * (n - g) - 1 - y;
+        load_cell<R>((ghost ? G : A) + ym * step, plane, u);
+        return below ? lo : ghost ? hi : 0u;
+    }
+    __device__ __forceinline__ void signed_line(R u[4], unsigned f) const
+    {
+        constexpr int L = T ? 2 : 1, N = T ? 1 : 2;   // momenta normal to the lanes' and the lines' sides
+        u[L] = flip_sign(u[L], flip);
+        u[N] = flip_sign(u[N], f);
+    }
+};
 
 // ---------------------------------------------------------- MUSCL-Hancock --
+// The step dt and the half steps dt_pred / (2 dx), dt_pred / (2 dy) (half_dt_dx,
+// muscl_hancock.cpp:248) of an item of block bd.
+template <class Dts>
+__device__ __forceinline__ void half_steps(const HfBlockDev& bd, Dts&& dts, double& dt_step, double& hx, double& hy)
+{
+    double dt_pred;
+    dts(dt_step, dt_pred);
+    hx = (0.5 * dt_pred) / bd.dx;
+    hy = (0.5 * dt_pred) / bd.dy;
+}
+
 // Rows of an item in range (q64 in hf_physics.h), from the first on: returns
 // the number of rows done, it.rows unless a lane left the range.  The caller
 // finishes with the general rows.
@@ -184,23 +254,20 @@ __device__ __forceinline__ void load_row(const R* __restrict__ Acol, const R* __
 // neighbour, and the left one's by a lane shift.
 // FP64 VALU issue bounds it, with two waves per SIMD: 8192^2 Van Leer runs at
 // 27.8 Gcell-updates/s, 21.5 with the general rows.
-template <class M, int LIM>
+template <class M, int LIM, class Dts>
 __device__ __forceinline__ int muscl_rows_q64(const HfStepArgs<double>& a, const HfItem it, const HfBlockDev& bd,
-                                              const int lane, const double dt_step, const double hx, const double hy,
+                                              const int lane, Dts&& dts, double& dt_step, double& hx, double& hy,
                                               double& mx, double& my)
 {
     const double gam = a.gamma, g1 = a.gamma - 1.0;
-    if (!(q64::constants_in_range(gam, g1) && q64::half_step_in_range(hx) && q64::half_step_in_range(hy))) return 0;
     const double ig1 = 1.0 / g1;
+    const q64::Limits lim;
     const int xraw = it.x0 + lane;
     const bool valid = xraw < bd.tx;
     const int xc = valid ? xraw : bd.tx - 1;
-    const bool gcol = xc < 2 || xc >= bd.tx - 2;
-    const double* Acol = a.A + bd.off + xc;
-    const double* Gcol = a.G + bd.off + xc;
+    const Lines<double, false> ROW(a, bd, xc);
     const int pitch = bd.pitch, ty = bd.ty;
     const int64_t plane = bd.plane;
-#define ROW(y, u) load_row<double>(Acol, Gcol, gcol, (y), 2, ty, pitch, plane, (u))
     const bool out = valid && lane >= 2 && lane < 62 && xraw >= 2 && xraw < bd.tx - 2;
     // lanes that write, whose x faces those use, and that those are reconstructed from
     const q64::mask m0 = __ballot(out), m1 = m0 | m0 << 1 | m0 >> 1, m2 = m1 | m1 << 1 | m1 >> 1;
@@ -211,61 +278,65 @@ __device__ __forceinline__ int muscl_rows_q64(const HfStepArgs<double>& a, const
     q64::mask bad = 0, bc, bp, bn;   // rows y, y+1, y+2 out of range
     {
         double um[4], dr[4], cr[4], lo[4], hi[4];
-        ROW(y0 - 2, um);
-        ROW(y0 - 1, uc);
-        ROW(y0, up);
-        ROW(y0 + 1, un);
-        bad = q64::out_of_range(um) | q64::out_of_range(uc);
-        bc = q64::out_of_range(up);
-        bp = q64::out_of_range(un);
-        q64::differences(um, uc, dl, cl);
-        q64::differences(uc, up, dr, cr);
-        q64::reconstruct<LIM, false>(uc, dl, dr, cl, cr, hy, g1, ig1, lo, hi, bad);     // cell y0-1
-        const q64::State sl = q64::make_state(hi, gam, g1, ig1, bad);
-        q64::differences(up, un, dl, cl);
-        q64::reconstruct<LIM, false>(up, dr, dl, cr, cl, hy, g1, ig1, lo, Tc, bad);     // cell y0
-        const q64::State sr = q64::make_state(lo, gam, g1, ig1, bad);
-        q64::hllc<false>(sl, sr, Gs, bad);
+        const unsigned fm = ROW(y0 - 2, um), fc = ROW(y0 - 1, uc), fp = ROW(y0, up), fn = ROW(y0 + 1, un);
+        half_steps(bd, dts, dt_step, hx, hy);   // behind the loads: its own chain of loads overlaps theirs
+        if (!(q64::constants_in_range(gam, g1) && q64::half_step_in_range(hx) && q64::half_step_in_range(hy))) return 0;
+        ROW.signed_line(um, fm);
+        ROW.signed_line(uc, fc);
+        ROW.signed_line(up, fp);
+        ROW.signed_line(un, fn);
+        bad = q64::out_of_range(um, lim) | q64::out_of_range(uc, lim);
+        bc = q64::out_of_range(up, lim);
+        bp = q64::out_of_range(un, lim);
+        q64::differences(um, uc, dl, cl, lim);
+        q64::differences(uc, up, dr, cr, lim);
+        q64::reconstruct<LIM, false>(uc, dl, dr, cl, cr, hy, g1, ig1, lo, hi, bad, lim);     // cell y0-1
+        const q64::State sl = q64::make_state(hi, gam, g1, ig1, bad, lim);
+        q64::differences(up, un, dl, cl, lim);
+        q64::reconstruct<LIM, false>(up, dr, dl, cr, cl, hy, g1, ig1, lo, Tc, bad, lim);     // cell y0
+        const q64::State sr = q64::make_state(lo, gam, g1, ig1, bad, lim);
+        q64::hllc<false>(sl, sr, Gs, bad, lim);
         if ((bad | bc | bp) & m0) return 0;
     }
     for (int k = 0; k < 4; k++) { uc[k] = up[k]; up[k] = un[k]; }
-    ROW(y0 + 2, un);
+    unsigned fn = ROW(y0 + 2, un);
 
     double* Ob = a.O + bd.off;
     for (int r = 0; r < it.rows; r++) {
         const int y = y0 + r;
         double nn[4];
-        ROW(y + 3 < ty ? y + 3 : ty - 1, nn);     // next iteration's U(y+2)
-        bn = q64::out_of_range(un);
+        ROW.signed_line(un, fn);
+        fn = ROW(y + 3 < ty ? y + 3 : ty - 1, nn);     // next iteration's U(y+2)
+        bn = q64::out_of_range(un, lim);
 
         // y direction: reconstruct cell y+1, flux through face y+1/2
         q64::mask by = 0, bx = 0;
         double dn[4], cn[4], Bn[4], Tn[4], Gn[4];
-        q64::differences(up, un, dn, cn);
-        q64::reconstruct<LIM, false>(up, dl, dn, cl, cn, hy, g1, ig1, Bn, Tn, by);
+        q64::differences(up, un, dn, cn, lim);
+        q64::reconstruct<LIM, false>(up, dl, dn, cl, cn, hy, g1, ig1, Bn, Tn, by, lim);
         {
-            const q64::State sl = q64::make_state(Tc, gam, g1, ig1, by);
-            const q64::State sr = q64::make_state(Bn, gam, g1, ig1, by);
-            q64::hllc<false>(sl, sr, Gn, by);
+            const q64::State sl = q64::make_state(Tc, gam, g1, ig1, by, lim);
+            const q64::State sr = q64::make_state(Bn, gam, g1, ig1, by, lim);
+            q64::hllc<false>(sl, sr, Gn, by, lim);
         }
 
         // x direction: reconstruct cell (x, y) from lane neighbours
         double ur[4], xl[4], xr[4], kl[4], kr[4], Lf[4], Rf[4], Rl[4], Fw[4], Fe[4];
         for (int k = 0; k < 4; k++) ur[k] = shfl_dn1(uc[k]);
-        q64::differences(uc, ur, xr, kr);
+        q64::differences(uc, ur, xr, kr, lim);
         for (int k = 0; k < 4; k++) { xl[k] = shfl_up1(xr[k]); kl[k] = shfl_up1(kr[k]); }
-        q64::reconstruct<LIM, true>(uc, xl, xr, kl, kr, hx, g1, ig1, Lf, Rf, bx);
+        q64::reconstruct<LIM, true>(uc, xl, xr, kl, kr, hx, g1, ig1, Lf, Rf, bx, lim);
         for (int k = 0; k < 4; k++) Rl[k] = shfl_up1(Rf[k]);
         {
-            const q64::State sl = q64::make_state(Rl, gam, g1, ig1, bx);
-            const q64::State sr = q64::make_state(Lf, gam, g1, ig1, bx);
-            q64::hllc<true>(sl, sr, Fw, bx);          // face x-1/2
+            const q64::State sl = q64::make_state(Rl, gam, g1, ig1, bx, lim);
+            const q64::State sr = q64::make_state(Lf, gam, g1, ig1, bx, lim);
+            q64::hllc<true>(sl, sr, Fw, bx, lim);          // face x-1/2
         }
         for (int k = 0; k < 4; k++) Fe[k] = shfl_dn1(Fw[k]);   // face x+1/2
 
         double Ln[4], Un[4], dx_, dy_;
         update_cell<M>(rdx, rdy, dt_step, Fw, Fe, Gs, Gn, uc, Ln, Un);
-        q64::wave_speeds(Un, gam, g1, dx_, dy_, by);
+        q64::wave_speeds(Un, gam, g1, dx_, dy_, by, lim);
         if (((by | bp | bn) & m0) | (bx & m1) | (bc & m2)) return r;
         if (out) {
             double* o = Ob + (int64_t)y * pitch + xraw;
@@ -281,16 +352,14 @@ __device__ __forceinline__ int muscl_rows_q64(const HfStepArgs<double>& a, const
         }
     }
     return it.rows;
-#undef ROW
 }
 
 // MUSCLHancockScheme::operator() (scheme/muscl_hancock/muscl_hancock.cpp:41-55)
 // fused with ForwardEulerODESolver (scheme/ode/forward_euler/forward_euler.cpp:25-30).
 // Output columns per wave: 60 (lanes 2..61); lanes 0,1,62,63 are halo.
-template <class M, int LIM, bool RESID, bool QUICK>
+template <class M, int LIM, bool RESID, bool QUICK, class Dts>
 __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, const HfItem it, const int lane,
-                                           const double dt_step, const double dt_pred,
-                                           const MaxOut& imax_out)
+                                           Dts&& dts, const MaxOut& imax_out)
 {
     typedef typename M::R R;
 
@@ -298,31 +367,31 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
     const int xraw = it.x0 + lane;
     const bool valid = xraw < bd.tx;
     const int xc = valid ? xraw : bd.tx - 1;
-    const bool gcol = xc < 2 || xc >= bd.tx - 2;
-    const R* Acol = a.A + bd.off + xc;
-    const R* Gcol = a.G + bd.off + xc;
+    const Lines<R, false> ROW(a, bd, xc);
     const int pitch = bd.pitch, ty = bd.ty;
     const int64_t plane = bd.plane;
-#define ROW(y, u) load_row<R>(Acol, Gcol, gcol, (y), 2, ty, pitch, plane, (u))
     const bool out = valid && lane >= 2 && lane < 62 && xraw >= 2 && xraw < bd.tx - 2;
 
-    const R hx = R((0.5 * dt_pred) / bd.dx);     // half_dt_dx, muscl_hancock.cpp:248
-    const R hy = R((0.5 * dt_pred) / bd.dy);
     const R rdx = R(1.0 / bd.dx);                  // one_dx, muscl_hancock.cpp:352
     const R rdy = R(1.0 / bd.dy);
-    const R dtR = R(dt_step);
+    double dt_step, hx_, hy_;
     const R gam = R(a.gamma), g1 = R(a.gamma - 1.0);
 
     double mx = 0.0, my = 0.0;
     int done = 0;
-    if constexpr (QUICK && !RESID && !M::fast) done = muscl_rows_q64<M, LIM>(a, it, bd, lane, dt_step, hx, hy, mx, my);
+    constexpr bool IN_RANGE = QUICK && !RESID && !M::fast;
+    if constexpr (IN_RANGE) done = muscl_rows_q64<M, LIM>(a, it, bd, lane, dts, dt_step, hx_, hy_, mx, my);
     if (done < it.rows) {
     const int y0 = it.y0 + done, rows = it.rows - done;
     R um[4], uc[4], up[4], un[4];
-    ROW(y0 - 2, um);
-    ROW(y0 - 1, uc);
-    ROW(y0, up);
-    ROW(y0 + 1, un);
+    const unsigned fm = ROW(y0 - 2, um), fc = ROW(y0 - 1, uc), fp = ROW(y0, up);
+    unsigned fn = ROW(y0 + 1, un);
+    if (!IN_RANGE) half_steps(bd, dts, dt_step, hx_, hy_);
+    ROW.signed_line(um, fm);
+    ROW.signed_line(uc, fc);
+    ROW.signed_line(up, fp);
+    ROW.signed_line(un, fn);
+    const R hx = R(hx_), hy = R(hy_), dtR = R(dt_step);
 
     // warm-up: T' of cell y0-1, (B', T') of cell y0, flux through face y0-1/2
     R Gs[4], Tc[4];
@@ -338,13 +407,14 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
     // window: uc = U(y), up = U(y+1), un = U(y+2) (loaded one iteration ahead
     // so that HBM latency overlaps the row's arithmetic)
     for (int k = 0; k < 4; k++) { uc[k] = up[k]; up[k] = un[k]; }
-    ROW(y0 + 2, un);
+    fn = ROW(y0 + 2, un);
 
     R* Ob = RESID ? a.O : a.O + bd.off;
     for (int r = 0; r < rows; r++) {
         const int y = y0 + r;
         R nn[4];
-        ROW(y + 3 < ty ? y + 3 : ty - 1, nn);     // next iteration's U(y+2)
+        ROW.signed_line(un, fn);
+        fn = ROW(y + 3 < ty ? y + 3 : ty - 1, nn);     // next iteration's U(y+2)
 
         // y direction: reconstruct cell y+1, flux through face y+1/2
         R Bn[4], Tn[4], Gn[4];
@@ -384,7 +454,6 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
     }
     }
     if (!RESID) store_maxima(a, imax_out, it.block, wave_max(mx), wave_max(my));
-#undef ROW
 }
 
 // The same update for a narrow column band at a block's right edge, with the
@@ -399,25 +468,22 @@ __device__ __forceinline__ void muscl_item(const HfStepArgs<typename M::R>& a, c
 __device__ __forceinline__ bool item_transposed(const HfItem& it) { return it.rows < 0; }
 
 // Columns of a transposed item in range, as muscl_rows_q64.
-template <class M, int LIM>
+template <class M, int LIM, class Dts>
 __device__ __forceinline__ int muscl_cols_q64(const HfStepArgs<double>& a, const HfItem it, const HfBlockDev& bd,
-                                              const int lane, const double dt_step, const double hx, const double hy,
+                                              const int lane, Dts&& dts, double& dt_step, double& hx, double& hy,
                                               double& mx, double& my)
 {
     const double gam = a.gamma, g1 = a.gamma - 1.0;
-    if (!(q64::constants_in_range(gam, g1) && q64::half_step_in_range(hx) && q64::half_step_in_range(hy))) return 0;
     const double ig1 = 1.0 / g1;
+    const q64::Limits lim;
     const int code = -it.rows;
     const int cols = code & 255, nrows = code >> 8;
     const int yraw = it.y0 + lane;
     const bool valid = yraw < bd.ty;
     const int yc = valid ? yraw : bd.ty - 1;
-    const bool grow = yc < 2 || yc >= bd.ty - 2;
+    const Lines<double, true> COL(a, bd, yc);
     const int pitch = bd.pitch, tx = bd.tx;
-    const double* Arow = a.A + bd.off + (int64_t)yc * pitch;
-    const double* Grow = a.G + bd.off + (int64_t)yc * pitch;
     const int64_t plane = bd.plane;
-#define COL(x, u) load_cell<double>(((grow || (x) < 2 || (x) >= tx - 2) ? Grow : Arow) + (x), plane, (u))
     const bool out = valid && lane >= 2 && lane < 62 && lane < 2 + nrows && yraw >= 2 && yraw < bd.ty - 2;
     const q64::mask m0 = __ballot(out), m1 = m0 | m0 << 1 | m0 >> 1, m2 = m1 | m1 << 1 | m1 >> 1;
     const double rdx = 1.0 / bd.dx, rdy = 1.0 / bd.dy;
@@ -427,61 +493,65 @@ __device__ __forceinline__ int muscl_cols_q64(const HfStepArgs<double>& a, const
     q64::mask bad = 0, bc, bp, bn;   // columns x, x+1, x+2 out of range
     {
         double um[4], dr[4], cr[4], lo[4], hi[4];
-        COL(x0 - 2, um);
-        COL(x0 - 1, uc);
-        COL(x0, up);
-        COL(x0 + 1, un);
-        bad = q64::out_of_range(um) | q64::out_of_range(uc);
-        bc = q64::out_of_range(up);
-        bp = q64::out_of_range(un);
-        q64::differences(um, uc, dl, cl);
-        q64::differences(uc, up, dr, cr);
-        q64::reconstruct<LIM, true>(uc, dl, dr, cl, cr, hx, g1, ig1, lo, hi, bad);      // column x0-1
-        const q64::State sl = q64::make_state(hi, gam, g1, ig1, bad);
-        q64::differences(up, un, dl, cl);
-        q64::reconstruct<LIM, true>(up, dr, dl, cr, cl, hx, g1, ig1, lo, Rc, bad);      // column x0
-        const q64::State sr = q64::make_state(lo, gam, g1, ig1, bad);
-        q64::hllc<true>(sl, sr, Fw, bad);
+        const unsigned fm = COL(x0 - 2, um), fc = COL(x0 - 1, uc), fp = COL(x0, up), fn = COL(x0 + 1, un);
+        half_steps(bd, dts, dt_step, hx, hy);   // behind the loads: its own chain of loads overlaps theirs
+        if (!(q64::constants_in_range(gam, g1) && q64::half_step_in_range(hx) && q64::half_step_in_range(hy))) return 0;
+        COL.signed_line(um, fm);
+        COL.signed_line(uc, fc);
+        COL.signed_line(up, fp);
+        COL.signed_line(un, fn);
+        bad = q64::out_of_range(um, lim) | q64::out_of_range(uc, lim);
+        bc = q64::out_of_range(up, lim);
+        bp = q64::out_of_range(un, lim);
+        q64::differences(um, uc, dl, cl, lim);
+        q64::differences(uc, up, dr, cr, lim);
+        q64::reconstruct<LIM, true>(uc, dl, dr, cl, cr, hx, g1, ig1, lo, hi, bad, lim);      // column x0-1
+        const q64::State sl = q64::make_state(hi, gam, g1, ig1, bad, lim);
+        q64::differences(up, un, dl, cl, lim);
+        q64::reconstruct<LIM, true>(up, dr, dl, cr, cl, hx, g1, ig1, lo, Rc, bad, lim);      // column x0
+        const q64::State sr = q64::make_state(lo, gam, g1, ig1, bad, lim);
+        q64::hllc<true>(sl, sr, Fw, bad, lim);
         if ((bad | bc | bp) & m0) return 0;
     }
     for (int k = 0; k < 4; k++) { uc[k] = up[k]; up[k] = un[k]; }
-    COL(x0 + 2, un);
+    unsigned fn = COL(x0 + 2, un);
 
     double* Ob = a.O + bd.off;
     for (int c = 0; c < cols; c++) {
         const int x = x0 + c;
         double nn[4];
-        COL(x + 3 < tx ? x + 3 : tx - 1, nn);     // next iteration's U(x+2)
-        bn = q64::out_of_range(un);
+        COL.signed_line(un, fn);
+        fn = COL(x + 3 < tx ? x + 3 : tx - 1, nn);     // next iteration's U(x+2)
+        bn = q64::out_of_range(un, lim);
 
         // x direction: reconstruct column x+1, flux through face x+1/2
         q64::mask by = 0, bx = 0;
         double dn[4], cn[4], Ln[4], Rn[4], Fe[4];
-        q64::differences(up, un, dn, cn);
-        q64::reconstruct<LIM, true>(up, dl, dn, cl, cn, hx, g1, ig1, Ln, Rn, bx);
+        q64::differences(up, un, dn, cn, lim);
+        q64::reconstruct<LIM, true>(up, dl, dn, cl, cn, hx, g1, ig1, Ln, Rn, bx, lim);
         {
-            const q64::State sl = q64::make_state(Rc, gam, g1, ig1, bx);
-            const q64::State sr = q64::make_state(Ln, gam, g1, ig1, bx);
-            q64::hllc<true>(sl, sr, Fe, bx);
+            const q64::State sl = q64::make_state(Rc, gam, g1, ig1, bx, lim);
+            const q64::State sr = q64::make_state(Ln, gam, g1, ig1, bx, lim);
+            q64::hllc<true>(sl, sr, Fe, bx, lim);
         }
 
         // y direction: reconstruct cell (x, y) from lane neighbours
         double ut[4], xl[4], xr[4], kl[4], kr[4], Bf[4], Tf[4], Tl[4], Gs[4], Gn[4];
         for (int k = 0; k < 4; k++) ut[k] = shfl_dn1(uc[k]);
-        q64::differences(uc, ut, xr, kr);
+        q64::differences(uc, ut, xr, kr, lim);
         for (int k = 0; k < 4; k++) { xl[k] = shfl_up1(xr[k]); kl[k] = shfl_up1(kr[k]); }
-        q64::reconstruct<LIM, false>(uc, xl, xr, kl, kr, hy, g1, ig1, Bf, Tf, by);
+        q64::reconstruct<LIM, false>(uc, xl, xr, kl, kr, hy, g1, ig1, Bf, Tf, by, lim);
         for (int k = 0; k < 4; k++) Tl[k] = shfl_up1(Tf[k]);
         {
-            const q64::State sl = q64::make_state(Tl, gam, g1, ig1, by);
-            const q64::State sr = q64::make_state(Bf, gam, g1, ig1, by);
-            q64::hllc<false>(sl, sr, Gs, by);         // face y-1/2
+            const q64::State sl = q64::make_state(Tl, gam, g1, ig1, by, lim);
+            const q64::State sr = q64::make_state(Bf, gam, g1, ig1, by, lim);
+            q64::hllc<false>(sl, sr, Gs, by, lim);         // face y-1/2
         }
         for (int k = 0; k < 4; k++) Gn[k] = shfl_dn1(Gs[k]);   // face y+1/2
 
         double Lu[4], Un[4], dx_, dy_;
         update_cell<M>(rdx, rdy, dt_step, Fw, Fe, Gs, Gn, uc, Lu, Un);
-        q64::wave_speeds(Un, gam, g1, dx_, dy_, bx);
+        q64::wave_speeds(Un, gam, g1, dx_, dy_, bx, lim);
         if (((bx | bp | bn) & m0) | (by & m1) | (bc & m2)) return c;
         if (out) {
             double* o = Ob + (int64_t)yraw * pitch + x;
@@ -497,13 +567,11 @@ __device__ __forceinline__ int muscl_cols_q64(const HfStepArgs<double>& a, const
         }
     }
     return cols;
-#undef COL
 }
 
-template <class M, int LIM, bool RESID, bool QUICK>
+template <class M, int LIM, bool RESID, bool QUICK, class Dts>
 __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a, const HfItem it, const int lane,
-                                             const double dt_step, const double dt_pred,
-                                             const MaxOut& imax_out)
+                                             Dts&& dts, const MaxOut& imax_out)
 {
     typedef typename M::R R;
 
@@ -513,32 +581,32 @@ __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a,
     const int yraw = it.y0 + lane;
     const bool valid = yraw < bd.ty;
     const int yc = valid ? yraw : bd.ty - 1;
-    const bool grow = yc < 2 || yc >= bd.ty - 2;
+    const Lines<R, true> COL(a, bd, yc);
     const int pitch = bd.pitch, tx = bd.tx;
-    const R* Arow = a.A + bd.off + (int64_t)yc * pitch;
-    const R* Grow = a.G + bd.off + (int64_t)yc * pitch;
     const int64_t plane = bd.plane;
-#define COL(x, u) load_cell<R>(((grow || (x) < 2 || (x) >= tx - 2) ? Grow : Arow) + (x), plane, (u))
     const bool out = valid && lane >= 2 && lane < 62 && lane < 2 + nrows && yraw >= 2 && yraw < bd.ty - 2;
 
-    const R hx = R((0.5 * dt_pred) / bd.dx);     // half_dt_dx, muscl_hancock.cpp:248
-    const R hy = R((0.5 * dt_pred) / bd.dy);
     const R rdx = R(1.0 / bd.dx);                  // one_dx, muscl_hancock.cpp:352
     const R rdy = R(1.0 / bd.dy);
-    const R dtR = R(dt_step);
+    double dt_step, hx_, hy_;
     const R gam = R(a.gamma), g1 = R(a.gamma - 1.0);
 
     double mx = 0.0, my = 0.0;
     int done = 0;
-    if constexpr (QUICK && !RESID && !M::fast)
-        done = muscl_cols_q64<M, LIM>(a, it, bd, lane, dt_step, hx, hy, mx, my);
+    constexpr bool IN_RANGE = QUICK && !RESID && !M::fast;
+    if constexpr (IN_RANGE)
+        done = muscl_cols_q64<M, LIM>(a, it, bd, lane, dts, dt_step, hx_, hy_, mx, my);
     if (done < cols) {
     const int x0 = it.x0 + done, left = cols - done;
     R um[4], uc[4], up[4], un[4];
-    COL(x0 - 2, um);
-    COL(x0 - 1, uc);
-    COL(x0, up);
-    COL(x0 + 1, un);
+    const unsigned fm = COL(x0 - 2, um), fc = COL(x0 - 1, uc), fp = COL(x0, up);
+    unsigned fn = COL(x0 + 1, un);
+    if (!IN_RANGE) half_steps(bd, dts, dt_step, hx_, hy_);
+    COL.signed_line(um, fm);
+    COL.signed_line(uc, fc);
+    COL.signed_line(up, fp);
+    COL.signed_line(un, fn);
+    const R hx = R(hx_), hy = R(hy_), dtR = R(dt_step);
 
     // warm-up: R' of column x0-1, (L', R') of column x0, flux through face x0-1/2
     R Fw[4], Rc[4];
@@ -552,13 +620,14 @@ __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a,
         hllc<M, true>(sl, sr, Fw);
     }
     for (int k = 0; k < 4; k++) { uc[k] = up[k]; up[k] = un[k]; }
-    COL(x0 + 2, un);
+    fn = COL(x0 + 2, un);
 
     R* Ob = RESID ? a.O : a.O + bd.off;
     for (int c = 0; c < left; c++) {
         const int x = x0 + c;
         R nn[4];
-        COL(x + 3 < tx ? x + 3 : tx - 1, nn);     // next iteration's U(x+2)
+        COL.signed_line(un, fn);
+        fn = COL(x + 3 < tx ? x + 3 : tx - 1, nn);     // next iteration's U(x+2)
 
         // x direction: reconstruct column x+1, flux through face x+1/2
         R Ln[4], Rn[4], Fe[4];
@@ -598,7 +667,6 @@ __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a,
     }
     }
     if (!RESID) store_maxima(a, imax_out, it.block, wave_max(mx), wave_max(my));
-#undef COL
 }
 
 // The guess launch's plan of problem p (plan_scan with the main list's
@@ -653,14 +721,16 @@ __device__ __forceinline__ int round_of(const HfStepArgs<R>& a, unsigned idx)
     return l;
 }
 
-template <class M, int LIM, bool RESID, bool QUICK = true>
-__device__ __forceinline__ void muscl_go(const HfStepArgs<typename M::R>& a, const HfItem& it, int lane, double dt_step,
-                                         double dt_pred, const MaxOut& imax_out)
+// dts(step, pred) gives the item's step and predictor dt; it is called once,
+// after the item's first lines are requested.
+template <class M, int LIM, bool RESID, bool QUICK = true, class Dts>
+__device__ __forceinline__ void muscl_go(const HfStepArgs<typename M::R>& a, const HfItem& it, int lane, Dts&& dts,
+                                         const MaxOut& imax_out)
 {
     if (!RESID && item_transposed(it))
-        muscl_item_t<M, LIM, RESID, QUICK>(a, it, lane, dt_step, dt_pred, imax_out);
+        muscl_item_t<M, LIM, RESID, QUICK>(a, it, lane, dts, imax_out);
     else
-        muscl_item<M, LIM, RESID, QUICK>(a, it, lane, dt_step, dt_pred, imax_out);
+        muscl_item<M, LIM, RESID, QUICK>(a, it, lane, dts, imax_out);
 }
 
 template <class R>
@@ -760,25 +830,45 @@ __device__ __forceinline__ void main_item(const HfStepArgs<typename M::R>& a, un
 {
     typedef typename M::R R;
     const HfItem it = a.items[a.item0 + idx];
-    if (a.use_fixed) {
-        c_step = a.fixed_step;
-        c_pred = a.fixed_pred;
-    } else {
-        if (a.skip[it.block]) return;   // left to the guess launch
+    if (!a.use_fixed && !a.mirrored && a.skip[it.block]) return;   // left to the guess launch
+    auto dts = [&](double& step, double& pred) {
+        if (a.use_fixed) {
+            step = a.fixed_step;
+            pred = a.fixed_pred;
+            return;
+        }
         const HfBlockDev bd = a.blocks[it.block];
         if (it.block != cached) {
             cached = it.block;
             step_dts<R>(a, bd, true, c_step, c_pred, c_kstep, c_kpred);
         }
         record_dts<R>(a, it, bd, true, c_step, c_pred, c_kstep, c_kpred);
-    }
-    muscl_go<M, LIM, RESID>(a, it, lane, c_step, c_pred, max_out(a, a.imax_new));
+        step = c_step;
+        pred = c_pred;
+    };
+    muscl_go<M, LIM, RESID>(a, it, lane, dts, max_out(a, a.imax_new));
+}
+
+// The books of a mirrored launch (HfStepArgs::mirrored), kept by its last
+// workgroup; true for its waves.
+template <class R>
+__device__ __forceinline__ bool keeps_books(const HfStepArgs<R>& a)
+{
+    if (!a.mirrored || blockIdx.x != gridDim.x - 1) return false;
+    for (int p = threadIdx.x; p < a.nprob; p += blockDim.x)
+        a.calls_next[p] = a.calls[p] + (a.use_fixed ? 0u : (uint32_t)a.probs[p].cps);
+    for (int i = threadIdx.x; i < a.nclear; i += blockDim.x) a.clear[i] = 0ull;
+    if (threadIdx.x < HF_SYNC_WORDS) a.clear_sync[threadIdx.x] = 0u;
+    if (threadIdx.x == 0 && a.fixstats) a.fixstats[0] += 1ull;   // launches of a context run one after the other
+    return true;
 }
 
 template <class M, int LIM, bool RESID>
 __global__ __launch_bounds__(256, 2) void k_muscl(const HfStepArgs<typename M::R> a)
 {
     typedef typename M::R R;
+    if (keeps_books(a)) return;
+    const unsigned extra = a.mirrored ? 1u : 0u;
     const int lane = threadIdx.x & 63;
     int cached = -1;   // the block whose speculative dts this wave has computed
     double c_step = 0.0, c_pred = 0.0;
@@ -801,7 +891,7 @@ __global__ __launch_bounds__(256, 2) void k_muscl(const HfStepArgs<typename M::R
         main_chunk<R>(a, cur, 0);
         cur.base = 0u;
     }
-    for (unsigned t = ticket_first(n); t < n; t = ticket_next(a.sync, lane, n)) {
+    for (unsigned t = ticket_first(n, extra); t < n; t = ticket_next(a.sync, lane, n, extra)) {
         unsigned idx = t;
         if (some) {
             while (t >= cur.base + cur.total) {
@@ -918,7 +1008,8 @@ __global__ __launch_bounds__(256, 2) void k_muscl_guess(const HfStepArgs<typenam
             a.fixed[cb] = 1u;   // the same value from every wave
         }
         record_dts<R>(a, it, bd, false, dt_step, dt_pred, g.kstep, kpred);
-        muscl_go<M, LIM, false>(a, it, lane, dt_step, dt_pred, max_out(a, a.imax_fix));
+        auto dts = [&](double& step, double& pred) { step = dt_step; pred = dt_pred; };
+        muscl_go<M, LIM, false>(a, it, lane, dts, max_out(a, a.imax_fix));
     }
 }
 
@@ -982,7 +1073,8 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
                 // (the channel's first 200 steps: 2.9 -> 0.83 ms per step).
                 atomicOr(&fixed_chk[it.block], 1u);
                 record_dts<R>(a, it, bd, false, c_step, c_pred, c_kstep, c_kpred);
-                muscl_go<M, LIM, false>(a, it, lane, c_step, c_pred, imax_chk);
+                auto dts = [&](double& step, double& pred) { step = c_step; pred = c_pred; };
+                muscl_go<M, LIM, false>(a, it, lane, dts, imax_chk);
             }
         }
         item_done(a.sync, lane);
@@ -1009,7 +1101,8 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
             if (check_verdict<R>(a, bd.problem, pr, a.nblocks, bd.lb, mg, dt_step, dt_pred, kstep, kpred)) {
                 atomicOr(&fixed_chk[it.block], 1u);
                 record_dts<R>(a, it, bd, false, dt_step, dt_pred, kstep, kpred);
-                muscl_go<M, LIM, false, false>(a, it, lane, dt_step, dt_pred, imax_chk);   // rare: the general rows only
+                auto dts = [&](double& step, double& pred) { step = dt_step; pred = dt_pred; };
+                muscl_go<M, LIM, false, false>(a, it, lane, dts, imax_chk);   // rare: the general rows only
                 __builtin_amdgcn_s_waitcnt(0xF70);   // its maxima are performed before the next verdict reads them
             }
         }
@@ -1027,25 +1120,24 @@ __device__ __forceinline__ int godunov_rows_q64(const HfStepArgs<double>& a, con
     const int xraw = it.x0 + lane;
     const bool valid = xraw < bd.tx;
     const int xc = valid ? xraw : bd.tx - 1;
-    const bool gcol = xc < 1 || xc >= bd.tx - 1;
-    const double* Acol = a.A + bd.off + xc;
-    const double* Gcol = a.G + bd.off + xc;
+    const Lines<double, false> ROW(a, bd, xc);
     const int pitch = bd.pitch, ty = bd.ty;
     const int64_t plane = bd.plane;
-#define ROW(y, u) load_row<double>(Acol, Gcol, gcol, (y), 1, ty, pitch, plane, (u))
     const bool out = valid && lane >= 1 && lane < 63 && xraw >= 1 && xraw < bd.tx - 1;
     const q64::mask m0 = __ballot(out), m1 = m0 | m0 << 1 | m0 >> 1;   // lanes that write, and their x neighbours
     const int y0 = it.y0;
     double ub[4], uc[4], un[4], Gs[4];
-    ROW(y0 - 1, ub);
-    ROW(y0, uc);
-    ROW(y0 + 1, un);
+    const unsigned fb = ROW(y0 - 1, ub), fc = ROW(y0, uc);
+    unsigned fn = ROW(y0 + 1, un);
+    ROW.signed_line(ub, fb);
+    ROW.signed_line(uc, fc);
     const double ig1 = 1.0 / g1, rdx = 1.0 / bd.dx, rdy = 1.0 / bd.dy;
-    q64::mask bad = q64::out_of_range(ub), bc = q64::out_of_range(uc);
-    q64::State sc = q64::make_state(uc, gam, g1, ig1, bc);
+    const q64::Limits lim;
+    q64::mask bad = q64::out_of_range(ub, lim), bc = q64::out_of_range(uc, lim);
+    q64::State sc = q64::make_state(uc, gam, g1, ig1, bc, lim);
     {
-        const q64::State sb = q64::make_state(ub, gam, g1, ig1, bad);
-        q64::hllc<false>(sb, sc, Gs, bad);         // face y0-1/2
+        const q64::State sb = q64::make_state(ub, gam, g1, ig1, bad, lim);
+        q64::hllc<false>(sb, sc, Gs, bad, lim);         // face y0-1/2
     }
     dt = dt_of();
     if (!q64::constants_in_range(gam, g1) || (bad & m0)) return 0;
@@ -1053,24 +1145,25 @@ __device__ __forceinline__ int godunov_rows_q64(const HfStepArgs<double>& a, con
     for (int r = 0; r < it.rows; r++) {
         const int y = y0 + r;
         double nn[4];
-        ROW(y + 2 < ty ? y + 2 : ty - 1, nn);     // next iteration's U(y+1)
-        q64::mask bn = q64::out_of_range(un), bx = 0;
-        const q64::State sn = q64::make_state(un, gam, g1, ig1, bn);
+        ROW.signed_line(un, fn);
+        fn = ROW(y + 2 < ty ? y + 2 : ty - 1, nn);     // next iteration's U(y+1)
+        q64::mask bn = q64::out_of_range(un, lim), bx = 0;
+        const q64::State sn = q64::make_state(un, gam, g1, ig1, bn, lim);
         double Gn[4], Fw[4], Fe[4];
-        q64::hllc<false>(sc, sn, Gn, bn);          // face y+1/2
+        q64::hllc<false>(sc, sn, Gn, bn, lim);          // face y+1/2
 
         q64::State sw;
         sw.U0 = shfl_up1(sc.U0); sw.U1 = shfl_up1(sc.U1); sw.U2 = shfl_up1(sc.U2); sw.U3 = shfl_up1(sc.U3);
         sw.u = shfl_up1(sc.u); sw.v = shfl_up1(sc.v); sw.p = shfl_up1(sc.p); sw.E = shfl_up1(sc.E);
         sw.a = shfl_up1(sc.a); sw.y = shfl_up1(sc.y);
-        q64::hllc<true>(sw, sc, Fw, bx);           // face x-1/2
+        q64::hllc<true>(sw, sc, Fw, bx, lim);           // face x-1/2
         for (int k = 0; k < 4; k++) Fe[k] = shfl_dn1(Fw[k]);
 
         const double U[4] = {sc.U0, sc.U1, sc.U2, sc.U3};
         double Ln[4], Un[4], dx_, dy_;
         update_cell<M>(rdx, rdy, dt, Fw, Fe, Gs, Gn, U, Ln, Un);
         q64::mask bw = 0;
-        q64::wave_speeds(Un, gam, g1, dx_, dy_, bw);
+        q64::wave_speeds(Un, gam, g1, dx_, dy_, bw, lim);
         if (((bn | bw) & m0) | ((bc | bx) & m1)) return r;
         if (out) {
             double* o = Ob + (int64_t)y * pitch + xraw;
@@ -1083,7 +1176,6 @@ __device__ __forceinline__ int godunov_rows_q64(const HfStepArgs<double>& a, con
         bc = bn;
     }
     return it.rows;
-#undef ROW
 }
 
 // GodunovScheme::operator() (scheme/godunov/godunov.cpp:27-118) fused with
@@ -1102,12 +1194,9 @@ __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a,
     const int xraw = it.x0 + lane;
     const bool valid = xraw < bd.tx;
     const int xc = valid ? xraw : bd.tx - 1;
-    const bool gcol = xc < 1 || xc >= bd.tx - 1;
-    const R* Acol = a.A + bd.off + xc;
-    const R* Gcol = a.G + bd.off + xc;
+    const Lines<R, false> ROW(a, bd, xc);
     const int pitch = bd.pitch, ty = bd.ty;
     const int64_t plane = bd.plane;
-#define ROW(y, u) load_row<R>(Acol, Gcol, gcol, (y), 1, ty, pitch, plane, (u))
     const bool out = valid && lane >= 1 && lane < 63 && xraw >= 1 && xraw < bd.tx - 1;
 
     const R rdx = R(1.0 / bd.dx);                  // godunov.cpp:97-98
@@ -1121,9 +1210,10 @@ __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a,
     if (done < it.rows) {
     const int y0 = it.y0 + done, rows = it.rows - done;
     R ub[4], uc[4], un[4];
-    ROW(y0 - 1, ub);
-    ROW(y0, uc);
-    ROW(y0 + 1, un);                               // loaded one iteration ahead
+    const unsigned fb = ROW(y0 - 1, ub), fc = ROW(y0, uc);
+    unsigned fn = ROW(y0 + 1, un);                 // loaded one iteration ahead
+    ROW.signed_line(ub, fb);
+    ROW.signed_line(uc, fc);
     State<R> sb = make_state<M>(ub, gam, g1);
     State<R> sc = make_state<M>(uc, gam, g1);
     R Gs[4];
@@ -1133,7 +1223,8 @@ __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a,
     for (int r = 0; r < rows; r++) {
         const int y = y0 + r;
         R nn[4];
-        ROW(y + 2 < ty ? y + 2 : ty - 1, nn);     // next iteration's U(y+1)
+        ROW.signed_line(un, fn);
+        fn = ROW(y + 2 < ty ? y + 2 : ty - 1, nn);     // next iteration's U(y+1)
         const State<R> sn = make_state<M>(un, gam, g1);
         R Gn[4], Fw[4], Fe[4];
         hllc<M, false>(sc, sn, Gn);                // face y+1/2
@@ -1163,7 +1254,6 @@ __device__ __forceinline__ void godunov_item(const HfStepArgs<typename M::R>& a,
     }
     }
     if (!RESID) store_maxima(a, imax_out, it.block, wave_max(mx), wave_max(my));
-#undef ROW
 }
 
 // Persistent Godunov launch (no predictor, so never a fix-up).
@@ -1171,9 +1261,11 @@ template <class M, bool RESID>
 __global__ __launch_bounds__(256) void k_godunov(const HfStepArgs<typename M::R> a)
 {
     typedef typename M::R R;
+    if (keeps_books(a)) return;
+    const unsigned extra = a.mirrored ? 1u : 0u;
     const int lane = threadIdx.x & 63;
     const unsigned n = (unsigned)a.nitems;
-    for (unsigned idx = ticket_first(n); idx < n; idx = ticket_next(a.sync, lane, n)) {
+    for (unsigned idx = ticket_first(n, extra); idx < n; idx = ticket_next(a.sync, lane, n, extra)) {
         const HfItem it = a.items[a.item0 + idx];
         auto dt_of = [&]() -> double {
             if (a.use_fixed) return a.fixed_step;

@@ -446,10 +446,10 @@ __device__ __forceinline__ void reconstruct(const typename M::R um[4], const typ
 // star state's E/rho).  The square root drops its scaling the same way.
 //
 // What can differ is caught by masks that every function adds lanes to:
-//  * rows of conserved values enter through in_range(): density and energy
-//    within [2^-60, 2^40] and [2^-100, 2^40], momenta zero or at least 2^-800;
-//  * face densities (>= 2^-60), pressures (>= 2^-200) and the numerator of S*
-//    are checked where they arise; a transverse momentum that is zero on one
+//  * rows of conserved values are checked by out_of_range(): density and
+//    energy within [2^-60, 2^40], momenta zero or at least 2^-800;
+//  * face densities and pressures (>= 2^-60) and the numerator of S* (zero or
+//    at least 2^-800) are checked where they arise; a transverse momentum that is zero on one
 //    side of a cell only could become a product of two tiny values, and
 //    counts as out of range;
 //  * a quotient by zero, an overflow or a NaN makes the new state's wave
@@ -470,8 +470,16 @@ namespace q64 {
 
 __device__ __forceinline__ double fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
-constexpr double RHO_MIN = 0x1p-60, RHO_MAX = 0x1p40, E_MIN = 0x1p-100, E_MAX = 0x1p40;
-constexpr double MOM_MIN = 0x1p-800, P_MIN = 0x1p-200, NUM_MIN = 0x1p-960;
+// The bounds and the limiter's constants, in vector registers: as literals
+// they would sit in scalar ones, and a row loop short of those moves others to
+// and from vector lanes (up to 65 instructions a row).
+struct Limits {
+    double low = 0x1p-60, high = 0x1p40, tiny = 0x1p-800, tol = 1e-6, quarter = 0.25;
+    __device__ __forceinline__ Limits()
+    {
+        asm volatile("" : "+v"(low), "+v"(high), "+v"(tiny), "+v"(tol), "+v"(quarter));
+    }
+};
 
 typedef unsigned long long mask;   // lanes, as __ballot gives them
 
@@ -507,11 +515,11 @@ __device__ __forceinline__ double sqrt(double x)
 }
 
 // Lanes whose conserved state is out of range.
-__device__ __forceinline__ mask out_of_range(const double U[4])
+__device__ __forceinline__ mask out_of_range(const double U[4], const Limits& c)
 {
-    return __ballot(!(U[0] >= RHO_MIN)) | __ballot(!(U[0] <= RHO_MAX)) | __ballot(!(U[3] >= E_MIN)) |
-           __ballot(!(U[3] <= E_MAX)) | (__ballot(U[1] != 0.0) & __ballot(__builtin_fabs(U[1]) < MOM_MIN)) |
-           (__ballot(U[2] != 0.0) & __ballot(__builtin_fabs(U[2]) < MOM_MIN));
+    return __ballot(!(U[0] >= c.low)) | __ballot(!(U[0] <= c.high)) | __ballot(!(U[3] >= c.low)) |
+           __ballot(!(U[3] <= c.high)) | (__ballot(U[1] != 0.0) & __ballot(__builtin_fabs(U[1]) < c.tiny)) |
+           (__ballot(U[2] != 0.0) & __ballot(__builtin_fabs(U[2]) < c.tiny));
 }
 // Constants of a launch and the half steps of an item.
 __device__ __forceinline__ bool constants_in_range(double gamma, double g1)
@@ -529,7 +537,7 @@ struct State {
 // Primitives and total energy; ig1 = 1/(gamma - 1) starts the reciprocal of
 // rho (gamma - 1) from that of rho, one Newton step short of it.
 __device__ __forceinline__ void prims(double U0, double U1, double U2, double U3, double g1, double ig1, double& y,
-                                      double& u, double& v, double& p, double& E, mask& bad)
+                                      double& u, double& v, double& p, double& E, mask& bad, const Limits& lim)
 {
     y = rcp(U0);
     u = div_pos(U1, U0, y);
@@ -540,14 +548,15 @@ __device__ __forceinline__ void prims(double U0, double U1, double U2, double U3
     const double y0 = y * ig1;
     const double yc = fma(y0, fma(-c, y0, 1.0), y0);
     E = U0 * fma(0.5, q2, div_pos(p, c, yc));
-    bad |= __ballot(!(U0 >= RHO_MIN)) | __ballot(!(p >= P_MIN));
+    bad |= __ballot(!(U0 >= lim.low)) | __ballot(!(p >= lim.low));
 }
 
-__device__ __forceinline__ State make_state(const double U[4], double gamma, double g1, double ig1, mask& bad)
+__device__ __forceinline__ State make_state(const double U[4], double gamma, double g1, double ig1, mask& bad,
+                                            const Limits& lim)
 {
     State s;
     s.U0 = U[0]; s.U1 = U[1]; s.U2 = U[2]; s.U3 = U[3];
-    prims(U[0], U[1], U[2], U[3], g1, ig1, s.y, s.u, s.v, s.p, s.E, bad);
+    prims(U[0], U[1], U[2], U[3], g1, ig1, s.y, s.u, s.v, s.p, s.E, bad, lim);
     s.a = sqrt(div_pos(gamma * s.p, s.U0, s.y));
     return s;
 }
@@ -555,19 +564,20 @@ __device__ __forceinline__ State make_state(const double U[4], double gamma, dou
 // The limiter's clamped difference: |d| raised to 1e-6 under the sign of d,
 // +1e-6 for either zero.  Only momenta (ZERO) can differ by -0.
 template <bool ZERO>
-__device__ __forceinline__ double clamp_delta(double d)
+__device__ __forceinline__ double clamp_delta(double d, const Limits& lim)
 {
-    return __builtin_copysign(__builtin_fmax(__builtin_fabs(d), 1e-6), ZERO ? d + 0.0 : d);
+    return __builtin_copysign(__builtin_fmax(__builtin_fabs(d), lim.tol), ZERO ? d + 0.0 : d);
 }
 
 // Differences b - a of two neighbouring cells, raw and clamped.
-__device__ __forceinline__ void differences(const double a[4], const double b[4], double d[4], double c[4])
+__device__ __forceinline__ void differences(const double a[4], const double b[4], double d[4], double c[4],
+                                            const Limits& lim)
 {
     for (int k = 0; k < 4; k++) d[k] = b[k] - a[k];
-    c[0] = clamp_delta<false>(d[0]);
-    c[1] = clamp_delta<true>(d[1]);
-    c[2] = clamp_delta<true>(d[2]);
-    c[3] = clamp_delta<false>(d[3]);
+    c[0] = clamp_delta<false>(d[0], lim);
+    c[1] = clamp_delta<true>(d[1], lim);
+    c[2] = clamp_delta<true>(d[2], lim);
+    c[3] = clamp_delta<false>(d[3], lim);
 }
 
 // Twice the limited slope's numerator: xi(r) (dl + dr), from the raw and the
@@ -589,18 +599,18 @@ __device__ __forceinline__ double limited_sum(double dl, double dr, double cl, d
 template <int LIM, bool X>
 __device__ __forceinline__ void reconstruct(const double uc[4], const double dl[4], const double dr[4],
                                             const double cl[4], const double cr[4], double h, double g1, double ig1,
-                                            double lo[4], double hi[4], mask& bad)
+                                            double lo[4], double hi[4], mask& bad, const Limits& lim)
 {
     for (int k = 0; k < 4; k++) {
         const double w = limited_sum<LIM>(dl[k], dr[k], cl[k], cr[k]);
-        lo[k] = fma(-0.25, w, uc[k]);
-        hi[k] = fma(0.25, w, uc[k]);
+        lo[k] = fma(-lim.quarter, w, uc[k]);
+        hi[k] = fma(lim.quarter, w, uc[k]);
     }
     constexpr int T = X ? 2 : 1;   // the transverse momentum
     bad |= __ballot(lo[T] == 0.0) ^ __ballot(hi[T] == 0.0);
     double y, ul, vl, pl, El, ur, vr, pr, Er;
-    prims(lo[0], lo[1], lo[2], lo[3], g1, ig1, y, ul, vl, pl, El, bad);
-    prims(hi[0], hi[1], hi[2], hi[3], g1, ig1, y, ur, vr, pr, Er, bad);
+    prims(lo[0], lo[1], lo[2], lo[3], g1, ig1, y, ul, vl, pl, El, bad, lim);
+    prims(hi[0], hi[1], hi[2], hi[3], g1, ig1, y, ur, vr, pr, Er, bad, lim);
     double Fl[4], Fr[4];
     flux<double, X>(lo[0], ul, vl, pl, El, Fl);
     flux<double, X>(hi[0], ur, vr, pr, Er, Fr);
@@ -615,14 +625,14 @@ __device__ __forceinline__ void reconstruct(const double uc[4], const double dl[
 // exactly when S_L < 0 and S* < 0, and only its flux and star state are
 // evaluated; the star flux holds unless the whole fan lies on K's far side.
 template <bool X>
-__device__ __forceinline__ void hllc(const State& L, const State& Rs, double F[4], mask& bad)
+__device__ __forceinline__ void hllc(const State& L, const State& Rs, double F[4], mask& bad, const Limits& lim)
 {
     const double qL = X ? L.u : L.v, qR = X ? Rs.u : Rs.v;
     const double S_L = __builtin_fmin(qL - L.a, qR - Rs.a);
     const double S_R = __builtin_fmax(qL + L.a, qR + Rs.a);
     const double num = Rs.p - L.p + L.U0 * qL * (S_L - qL) - Rs.U0 * qR * (S_R - qR);
     const double den = L.U0 * (S_L - qL) - Rs.U0 * (S_R - qR);
-    bad |= __ballot(num != 0.0) & __ballot(__builtin_fabs(num) < NUM_MIN);
+    bad |= __ballot(num != 0.0) & __ballot(__builtin_fabs(num) < lim.tiny);
     const double Ss = div_neg(num, den, rcp(den));
 
     const bool useR = (S_L < 0.0) & (Ss < 0.0);
@@ -651,7 +661,7 @@ __device__ __forceinline__ void hllc(const State& L, const State& Rs, double F[4
 // wave_speeds() of a new state; its own range is checked here (a pressure of
 // zero or below makes the speed NaN, which the caller tests).
 __device__ __forceinline__ void wave_speeds(const double U[4], double gamma, double g1, double& Dx, double& Dy,
-                                            mask& bad)
+                                            mask& bad, const Limits& lim)
 {
     const double y = rcp(U[0]);
     const double u = div_pos(U[1], U[0], y), v = div_pos(U[2], U[0], y);
@@ -659,7 +669,7 @@ __device__ __forceinline__ void wave_speeds(const double U[4], double gamma, dou
     const double c = sqrt(div_pos(gamma * p, U[0], y));
     Dx = __builtin_fabs(u) + c;
     Dy = __builtin_fabs(v) + c;
-    bad |= __ballot(!(U[0] >= RHO_MIN)) | __ballot(!(U[3] >= E_MIN)) | __ballot(!(Dx == Dx));
+    bad |= __ballot(!(U[0] >= lim.low)) | __ballot(!(U[3] >= lim.low)) | __ballot(!(Dx == Dx));
 }
 
 }  // namespace q64
@@ -711,24 +721,43 @@ __device__ __forceinline__ void wave_speeds(typename M::R U0, typename M::R U1, 
 
 __device__ __forceinline__ double dmax_nan(double acc, double x) { return (x > acc) ? x : acc; }
 
-// Reduce a per-lane maximum over the wave (NaN-free inputs).
-__device__ __forceinline__ double wave_max(double x)
+// Reduction of a per-lane value over the wave by DPP: within rows of 16 lanes
+// by shifts, then row ends broadcast into the next rows; lane 63 ends with the
+// whole wave's, which every lane gets (a scalar).  About 30 instructions
+// without an LDS round trip, where six bpermute shuffles of a double wait for
+// twelve.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double x)   // the partner's x, or x where there is none
 {
-    for (int off = 32; off > 0; off >>= 1) {
-        const double o = __shfl_xor(x, off, 64);
-        x = (o > x) ? o : x;
-    }
-    return x;
+    const long long b = __double_as_longlong(x);
+    const int lo = (int)(b & 0xffffffffll), hi = (int)(b >> 32);
+    const int l2 = __builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false);
+    const int h2 = __builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false);
+    return __longlong_as_double(((long long)h2 << 32) | (unsigned int)l2);
+}
+template <class F>
+__device__ __forceinline__ double wave_reduce(double x, F pick)
+{
+    x = pick(x, dpp_f64<0x111, 0xf>(x));   // row_shr:1, 2, 4, 8
+    x = pick(x, dpp_f64<0x112, 0xf>(x));
+    x = pick(x, dpp_f64<0x114, 0xf>(x));
+    x = pick(x, dpp_f64<0x118, 0xf>(x));
+    x = pick(x, dpp_f64<0x142, 0xa>(x));   // row_bcast:15 into rows 1 and 3
+    x = pick(x, dpp_f64<0x143, 0xc>(x));   // row_bcast:31 into rows 2 and 3
+    const long long b = __double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), 63);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-// Reduce a per-lane minimum over the wave (NaN-free inputs).
+// Maximum / minimum over the wave (NaN-free inputs; every lane calls).
+__device__ __forceinline__ double wave_max(double x)
+{
+    return wave_reduce(x, [](double a, double b) { return (b > a) ? b : a; });
+}
 __device__ __forceinline__ double wave_min(double x)
 {
-    for (int off = 32; off > 0; off >>= 1) {
-        const double o = __shfl_xor(x, off, 64);
-        x = (o < x) ? o : x;
-    }
-    return x;
+    return wave_reduce(x, [](double a, double b) { return (b < a) ? b : a; });
 }
 
 // The step and predictor dt of a block from the device partial maxima
@@ -757,7 +786,7 @@ __device__ __forceinline__ void step_dts(const HfStepArgs<R>& a, const HfBlockDe
     // depend on the order, so the results equal the sequential loop's.  Every
     // lane of the wave calls this (wave-uniform arguments).
     const HfProbDev pr = a.probs[bd.problem];
-    kstep = (long long)a.calls[bd.problem] - pr.cps + 1;
+    kstep = (long long)a.calls[bd.problem] - (a.mirrored ? 0 : pr.cps) + 1;
     kpred = kstep + 1 + bd.lb;
     // A lane takes one slot of a block: the quotient by the largest of a
     // block's maxima is the least of the quotients by each.

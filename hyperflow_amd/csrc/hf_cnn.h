@@ -48,6 +48,18 @@ struct WgradArgs {
     int32_t nx, ny, rows;
 };
 
+// One layer's weight-gradient partials and where their sum goes.
+struct ReduceLayer {
+    const float* part;
+    float* grads;
+    int32_t nparts, ci, co, ci_r, co_r, first;   // first: set by launch_reduce_grad
+};
+constexpr int MAX_LAYERS = 5;
+struct ReduceArgs {
+    ReduceLayer layer[MAX_LAYERS];
+    int32_t nlayers;
+};
+
 // Input normalisation + optional shock sensor.  U: planes of the conserved
 // variables with the interior origin at U, element (v, y, x) at
 // U[v*plane + y*pitch + x].
@@ -75,13 +87,11 @@ struct LossArgs {
 // Launchers (hf_cnn.hip).  cin/cout are storage channel counts (8 or 32).
 hipError_t launch_conv(int cin, int cout, int mode, const ConvArgs& a, hipStream_t s);
 hipError_t launch_wgrad(int ci, int co, const WgradArgs& a, int* nwg, hipStream_t s);
-int wgrad_workgroups(int nx, int ny, int rows);
+int wgrad_rows(int nx, int ny);   // rows per workgroup, WgradArgs::rows
+int wgrad_workgroups(int nx, int ny);
 hipError_t launch_pack(const PackArgs& a, hipStream_t s);
 hipError_t launch_loss(const LossArgs& a, int* nblocks, hipStream_t s);
-// tmp: REDUCE_SPLIT * (9*ci*co + co) floats of scratch.
-constexpr int REDUCE_SPLIT = 16;
-hipError_t launch_reduce_grad(const float* part, int nparts, int ci, int co, int ci_r, int co_r, float* g,
-                              float* tmp, hipStream_t s);
+hipError_t launch_reduce_grad(ReduceArgs a, hipStream_t s);
 hipError_t launch_reduce_sum(const float* part, int n, float scale, float* out, hipStream_t s);
 hipError_t launch_adam(float* w, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
                        float c1, float c2, hipStream_t s);

@@ -205,8 +205,14 @@ __global__ __launch_bounds__(256, 3) void k_conv(const ConvArgs a)
 // of three slots, so each input row is staged once.  Each lane's 8
 // consecutive pixels of one channel are then one aligned 16-byte LDS read.
 // The pixels are the MFMA reduction dimension: A = gz^T (rows = co), B =
-// shifted input (columns = ci).  Each wave owns a fixed set of (tap, co
-// tile, ci tile) products; partial sums go to part[workgroup].
+// shifted input (columns = ci).  A row's A operands are read once per wave; a
+// wave owns a fixed set of (tap, ci tile) pairs, reads each pair's B operand
+// once for all co tiles, and wave 3 also multiplies A by ones, which gives db;
+// partial sums go to part[workgroup].
+// Bound by the LDS round of a row (staging, barrier, operand reads), so a
+// small image is cut into as few rows per workgroup as fill the chip
+// (wgrad_rows).  256^2, 32 -> 32: 16 rows, a B and an A read per product and
+// db summed by 32 threads took 44.6 us, now 13.3.
 constexpr int LPX = 72;   // LDS row pitch in elements (64 pixels + 8 padding)
 
 template <int CI, int CO>
@@ -215,8 +221,8 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradArgs a)
     constexpr int CIL = CI < 16 ? 16 : CI;
     constexpr int COL = CO < 16 ? 16 : CO;
     constexpr int MT = COL / 16, NT = CIL / 16;
-    constexpr int ITEMS = 9 * MT * NT;
-    constexpr int NPW = (ITEMS + 3) / 4;
+    constexpr int PAIRS = 9 * NT;
+    constexpr int NPW = (PAIRS + 3) / 4;
     __shared__ __attribute__((aligned(16))) uint16_t aT[3][3][CIL][LPX];
     __shared__ __attribute__((aligned(16))) uint16_t gT[COL][LPX];
 
@@ -257,10 +263,15 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradArgs a)
         }
     };
 
-    f32x4 acc[NPW];
+    f32x4 acc[NPW][MT], db[MT];
 #pragma unroll
-    for (int u = 0; u < NPW; u++) acc[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    float db = 0.0f;
+    for (int mt = 0; mt < MT; mt++) {
+        db[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int u = 0; u < NPW; u++) acc[u][mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    const uint4 one4 = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, one4);
 
     stage_row(y0 - 1);
     stage_row(y0);
@@ -276,38 +287,52 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradArgs a)
         stage_row(y + 1);
         __syncthreads();
 #pragma unroll
-        for (int u = 0; u < NPW; u++) {
-            const int q = wave + 4 * u;
-            if (q < ITEMS) {
-                const int tap = q % 9, mt = (q / 9) % MT, nt = (q / 9) / MT;
-                const int slot = (y + tap / 3 + 2) % 3;   // input row y + dy, dy = tap/3 - 1
+        for (int ks = 0; ks < 2; ks++) {
+            bf16x8 A[MT];
 #pragma unroll
-                for (int ks = 0; ks < 2; ks++) {
-                    const bf16x8 A = load8(&gT[16 * mt + j][32 * ks + 8 * g]);
+            for (int mt = 0; mt < MT; mt++) A[mt] = load8(&gT[16 * mt + j][32 * ks + 8 * g]);
+#pragma unroll
+            for (int u = 0; u < NPW; u++) {
+                const int q = wave + 4 * u;
+                if (q < PAIRS) {
+                    const int tap = q % 9, nt = q / 9;
+                    const int slot = (y + tap / 3 + 2) % 3;   // input row y + dy, dy = tap/3 - 1
                     const bf16x8 B = load8(&aT[slot][tap % 3][16 * nt + j][32 * ks + 8 * g]);
-                    acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, acc[u], 0, 0, 0);
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++)
+                        acc[u][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt], B, acc[u][mt], 0, 0, 0);
                 }
             }
+            if (wave == 3)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+                    db[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt], ones, db[mt], 0, 0, 0);
         }
-        if (tid < CO)
-            for (int px = 0; px < 64; px++) db += bf2f(gT[tid][px]);
     }
 
     float* P = a.part + (size_t)blockIdx.x * (9 * CI * CO + CO);
 #pragma unroll
     for (int u = 0; u < NPW; u++) {
         const int q = wave + 4 * u;
-        if (q < ITEMS) {
-            const int tap = q % 9, mt = (q / 9) % MT, nt = (q / 9) / MT;
-            const int ci = 16 * nt + j;
+        if (q < PAIRS) {
+            const int tap = q % 9, ci = 16 * (q / 9) + j;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int co = 16 * mt + 4 * g + r;
+                    if (co < CO && ci < CI) P[((size_t)tap * CI + ci) * CO + co] = acc[u][mt][r];
+                }
+        }
+    }
+    if (wave == 3 && j == 0)   // every column holds the sum
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int co = 16 * mt + 4 * g + r;
-                if (co < CO && ci < CI) P[((size_t)tap * CI + ci) * CO + co] = acc[u][r];
+                if (co < CO) P[9 * CI * CO + co] = db[mt][r];
             }
-        }
-    }
-    if (tid < CO) P[9 * CI * CO + tid] = db;
 }
 
 // ------------------------------------------------------------------ helpers --
@@ -377,45 +402,39 @@ __global__ __launch_bounds__(256) void k_loss(const LossArgs a)
     if (threadIdx.x == 0) a.part[blockIdx.x] = red[0];
 }
 
-// Sum of the workgroup partials in two deterministic stages.  Stage 1: block
-// (bx, by) adds partials [by*chunk, (by+1)*chunk) of 64 consecutive entries,
-// four interleaved subsets per entry combined in a fixed order, into
-// tmp[by].  Stage 2 adds the stage-1 rows in order and writes the layer's
-// real layout W[9][ci_r][co_r] followed by b[co_r] (padding channels
-// dropped).
-__global__ __launch_bounds__(256) void k_reduce_stage1(const float* __restrict__ part, int nparts, int stride,
-                                                       int chunk, float* __restrict__ tmp)
+// Sums of the weight gradients' workgroup partials, every layer in one launch:
+// a workgroup adds 64 consecutive entries of one layer, its 16 waves interleaved
+// subsets of the partials, combined in a fixed order, and writes the layer's
+// real layout W[9][ci_r][co_r] followed by b[co_r] (padding channels dropped).
+// Ten launches (two per layer) took 50 us of a 256^2 gradient, this one 13.
+__global__ __launch_bounds__(1024) void k_reduce_grad(const ReduceArgs a)
 {
-    __shared__ float red[4][64];
+    __shared__ float red[16][64];
+    int l = 0;
+    while (l + 1 < a.nlayers && (int)blockIdx.x >= a.layer[l + 1].first) l++;
+    const ReduceLayer L = a.layer[l];
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int s = blockIdx.x * 64 + tx;
-    const int w0 = blockIdx.y * chunk, w1 = min(nparts, w0 + chunk);
+    const int stride = 9 * L.ci * L.co + L.co;
+    const int s = ((int)blockIdx.x - L.first) * 64 + tx;
     float acc = 0.0f;
     if (s < stride)
-        for (int w = w0 + ty; w < w1; w += 4) acc += part[(size_t)w * stride + s];
+        for (int w = ty; w < L.nparts; w += 16) acc += L.part[(size_t)w * stride + s];
     red[ty][tx] = acc;
     __syncthreads();
-    if (ty == 0 && s < stride) tmp[(size_t)blockIdx.y * stride + s] = (red[0][tx] + red[1][tx]) + (red[2][tx] + red[3][tx]);
-}
-
-__global__ __launch_bounds__(256) void k_reduce_grad(const float* __restrict__ part, int nparts, int CI, int CO,
-                                                     int ci_r, int co_r, float* __restrict__ gout)
-{
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    const int stride = 9 * CI * CO + CO;
-    if (s >= stride) return;
+    if (ty != 0 || s >= stride) return;
     float v = 0.0f;
-    for (int w = 0; w < nparts; w++) v += part[(size_t)w * stride + s];
+#pragma unroll
+    for (int k = 0; k < 16; k++) v += red[k][tx];
     int dst = -1;
-    if (s < 9 * CI * CO) {
-        const int tap = s / (CI * CO), rem = s % (CI * CO);
-        const int ci = rem / CO, co = rem % CO;
-        if (ci < ci_r && co < co_r) dst = (tap * ci_r + ci) * co_r + co;
+    if (s < 9 * L.ci * L.co) {
+        const int tap = s / (L.ci * L.co), rem = s % (L.ci * L.co);
+        const int ci = rem / L.co, co = rem % L.co;
+        if (ci < L.ci_r && co < L.co_r) dst = (tap * L.ci_r + ci) * L.co_r + co;
     } else {
-        const int co = s - 9 * CI * CO;
-        if (co < co_r) dst = 9 * ci_r * co_r + co;
+        const int co = s - 9 * L.ci * L.co;
+        if (co < L.co_r) dst = 9 * L.ci_r * L.co_r + co;
     }
-    if (dst >= 0) gout[dst] = v;
+    if (dst >= 0) L.grads[dst] = v;
 }
 
 __global__ __launch_bounds__(256) void k_reduce_sum(const float* __restrict__ part, int n, float scale,
@@ -523,11 +542,23 @@ hipError_t launch_conv(int cin, int cout, int mode, const ConvArgs& a, hipStream
     return hipErrorInvalidValue;
 }
 
-int wgrad_workgroups(int nx, int ny, int rows) { return (nx / 64) * ((ny + rows - 1) / rows); }
+// Rows per workgroup: the most, up to 16, that still make two workgroups for
+// each of the 256 CUs (at least 2 rows: every workgroup stages two more).
+int wgrad_rows(int nx, int ny)
+{
+    int rows = 16;
+    while (rows > 2 && (nx / 64) * ((ny + rows - 1) / rows) < 512) rows /= 2;
+    return rows;
+}
+int wgrad_workgroups(int nx, int ny)
+{
+    const int rows = wgrad_rows(nx, ny);
+    return (nx / 64) * ((ny + rows - 1) / rows);
+}
 
 hipError_t launch_wgrad(int ci, int co, const WgradArgs& a, int* nwg, hipStream_t s)
 {
-    const int n = wgrad_workgroups(a.nx, a.ny, a.rows);
+    const int n = wgrad_workgroups(a.nx, a.ny);
     *nwg = n;
     if (ci == 8 && co == 32) hipLaunchKernelGGL((k_wgrad<8, 32>), dim3(n), dim3(256), 0, s, a);
     else if (ci == 32 && co == 32) hipLaunchKernelGGL((k_wgrad<32, 32>), dim3(n), dim3(256), 0, s, a);
@@ -551,15 +582,14 @@ hipError_t launch_loss(const LossArgs& a, int* nblocks, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_reduce_grad(const float* part, int nparts, int ci, int co, int ci_r, int co_r, float* g,
-                              float* tmp, hipStream_t s)
+hipError_t launch_reduce_grad(ReduceArgs a, hipStream_t s)
 {
-    const int stride = 9 * ci * co + co;
-    const int chunk = (nparts + REDUCE_SPLIT - 1) / REDUCE_SPLIT;
-    hipLaunchKernelGGL(k_reduce_stage1, dim3((stride + 63) / 64, REDUCE_SPLIT), dim3(256), 0, s, part, nparts, stride,
-                       chunk, tmp);
-    hipLaunchKernelGGL(k_reduce_grad, dim3((stride + 255) / 256), dim3(256), 0, s, tmp, REDUCE_SPLIT, ci, co, ci_r,
-                       co_r, g);
+    int blocks = 0;
+    for (int l = 0; l < a.nlayers; l++) {
+        a.layer[l].first = blocks;
+        blocks += (9 * a.layer[l].ci * a.layer[l].co + a.layer[l].co + 63) / 64;
+    }
+    hipLaunchKernelGGL(k_reduce_grad, dim3(blocks), dim3(1024), 0, s, a);
     return hipGetLastError();
 }
 

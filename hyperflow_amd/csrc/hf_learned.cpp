@@ -38,8 +38,14 @@ const Layer LAYERS[NL] = {
     {32, 4, 32, 8, P1 + 3 * PH},
 };
 constexpr int64_t NPARAM = P1 + 3 * PH + P5;
-constexpr int CONV_ROWS = 8;    // rows per wave of the convolutions
-constexpr int WGRAD_ROWS = 16;  // rows per workgroup of the weight gradient
+// Rows per wave of the convolutions: 8, fewer where that leaves SIMDs without
+// a wave (256^2, 32 -> 32 data gradient: 8 rows 10.4 us, 2 rows 7.4).
+int conv_rows(int nx, int ny)
+{
+    int rows = 8;
+    while (rows > 2 && (int64_t)(nx / 16) * ((ny + rows - 1) / rows) < 2048) rows /= 2;
+    return rows;
+}
 
 int fail(int code, const std::string& msg) { return hf_fail(code, msg); }
 
@@ -63,8 +69,7 @@ struct hf_net {
     uint16_t* gz[2] = {};
     float* y = nullptr;
     uint8_t* shock = nullptr;
-    float* part = nullptr;
-    float* part2 = nullptr;   // second stage of the gradient reduction
+    float* part[NL] = {};     // weight-gradient partials of each layer
     float* lossp = nullptr;
     float* loss = nullptr;
     uint32_t* fallback = nullptr;
@@ -83,11 +88,10 @@ void free_images(hf_net* n)
     for (auto& p : n->gz) (void)hipFree(p), p = nullptr;
     (void)hipFree(n->y);
     (void)hipFree(n->shock);
-    (void)hipFree(n->part);
-    (void)hipFree(n->part2);
+    for (auto& p : n->part) (void)hipFree(p), p = nullptr;
     (void)hipFree(n->lossp);
     n->x = n->g8 = nullptr;
-    n->y = n->part = n->part2 = n->lossp = nullptr;
+    n->y = n->lossp = nullptr;
     n->shock = nullptr;
     n->nx = n->ny = 0;
 }
@@ -114,9 +118,9 @@ int ensure_images(hf_net* n, int nx, int ny)
     }
     HF_HIP(hipMalloc(&n->y, (size_t)nx * ny * 4 * sizeof(float)));
     HF_HIP(hipMalloc(&n->shock, (size_t)nx * ny));
-    const int nwg = hfn::wgrad_workgroups(nx, ny, WGRAD_ROWS);
-    HF_HIP(hipMalloc(&n->part, (size_t)nwg * (9 * 32 * 32 + 32) * sizeof(float)));
-    HF_HIP(hipMalloc(&n->part2, (size_t)hfn::REDUCE_SPLIT * (9 * 32 * 32 + 32) * sizeof(float)));
+    const int nwg = hfn::wgrad_workgroups(nx, ny);
+    for (int l = 0; l < NL; l++)
+        HF_HIP(hipMalloc(&n->part[l], (size_t)nwg * (9 * LAYERS[l].cis + 1) * LAYERS[l].cos * sizeof(float)));
     const int nloss = (int)(((int64_t)nx * ny + 255) / 256);
     HF_HIP(hipMalloc(&n->lossp, (size_t)nloss * sizeof(float)));
     n->nx = nx;
@@ -157,7 +161,7 @@ hfn::ConvArgs conv_args(const hf_net* n, int l, const uint16_t* in, int nx, int 
     a.co_real = LAYERS[l].co;
     a.nx = nx;
     a.ny = ny;
-    a.rows = CONV_ROWS;
+    a.rows = conv_rows(nx, ny);
     return a;
 }
 
@@ -190,19 +194,20 @@ int forward_hidden(hf_net* n, const float* U, int64_t plane, int pitch, int nx, 
     return HF_OK;
 }
 
-int wgrad(hf_net* n, int l, const uint16_t* a_in, const uint16_t* gz, int nx, int ny, hipStream_t s)
+int wgrad(hf_net* n, int l, const uint16_t* a_in, const uint16_t* gz, int nx, int ny, hfn::ReduceArgs& red,
+          hipStream_t s)
 {
     const Layer& L = LAYERS[l];
     hfn::WgradArgs w;
     w.a = a_in;
     w.gz = gz;
-    w.part = n->part;
+    w.part = n->part[l];
     w.nx = nx;
     w.ny = ny;
-    w.rows = WGRAD_ROWS;
+    w.rows = hfn::wgrad_rows(nx, ny);
     int nwg = 0;
     HF_HIP(hfn::launch_wgrad(L.cis, L.cos, w, &nwg, s));
-    HF_HIP(hfn::launch_reduce_grad(n->part, nwg, L.cis, L.cos, L.ci, L.co, n->grads + L.off, n->part2, s));
+    red.layer[red.nlayers++] = hfn::ReduceLayer{n->part[l], n->grads + L.off, nwg, L.cis, L.cos, L.ci, L.co, 0};
     return HF_OK;
 }
 
@@ -233,7 +238,9 @@ int gradients(hf_net* n, const float* u, const float* target, int nx, int ny, hi
     HF_HIP(hfn::launch_reduce_sum(n->lossp, nb, inv, n->loss, s));
 
     // layer 5: gradient at its output is g8
-    rc = wgrad(n, 4, n->act[3], n->g8, nx, ny, s);
+    hfn::ReduceArgs red;
+    red.nlayers = 0;
+    rc = wgrad(n, 4, n->act[3], n->g8, nx, ny, red, s);
     if (rc) return rc;
     const uint16_t* gin = n->g8;
     int cin = 8;
@@ -246,16 +253,17 @@ int gradients(hf_net* n, const float* u, const float* target, int nx, int ny, hi
         b.wa = n->wb[l];
         b.nx = nx;
         b.ny = ny;
-        b.rows = CONV_ROWS;
+        b.rows = conv_rows(nx, ny);
         b.out = gout;
         b.mask = n->act[l - 1];
         HF_HIP(hfn::launch_conv(cin, 32, hfn::CONV_BWD, b, s));
         const uint16_t* a_in = (l - 1 == 0) ? n->x : n->act[l - 2];
-        rc = wgrad(n, l - 1, a_in, gout, nx, ny, s);
+        rc = wgrad(n, l - 1, a_in, gout, nx, ny, red, s);
         if (rc) return rc;
         gin = gout;
         cin = 32;
     }
+    HF_HIP(hfn::launch_reduce_grad(red, s));
     return HF_OK;
 }
 

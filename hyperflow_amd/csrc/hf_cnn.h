@@ -20,25 +20,33 @@
 
 namespace hfn {
 
-enum { CONV_HIDDEN = 0, CONV_BWD = 1, CONV_OUT = 2, CONV_APPLY = 3 };
+enum { NET_OUT_PLANES = 0, NET_APPLY = 1 };
 
+// The forward pass.
+struct NetArgs {
+    const uint16_t* x;        // packed input, NHWC BF16, padded, 8 channels
+    const uint16_t* w[5];     // A operands of each layer [MT][S][64 lanes][8]
+    const float* bias[5];
+    int32_t nx, ny, rows;     // interior size; rows per workgroup (set by launch_net)
+    uint16_t* act[4];         // hidden activations, NHWC BF16, padded (null: not stored)
+    float* outf;              // NET_OUT_PLANES: dense planes [4][ny][nx]
+    float* U;                 // NET_APPLY: state planes (interior origin), corrected in place
+    int64_t plane;            // elements per plane of U
+    int32_t pitch;            // row pitch of U
+    float gamma;              // ideal-gas gamma for the pressure check
+    float scale[4];           // correction = scale * network output
+    float max_output;         // fall back where |output| > max_output (<= 0: no bound)
+    const uint8_t* shock;     // per-cell shock flag [ny][nx] (null: none)
+    uint32_t* fallback;       // cells left at the plain state
+};
+
+// The data gradient of one layer.
 struct ConvArgs {
-    const uint16_t* in;     // NHWC BF16, padded, CIN channels
-    const uint16_t* wa;     // A operands [MT][S][64 lanes][8]
-    const float* bias;      // [co_real] (HIDDEN, OUT, APPLY)
-    int32_t co_real;
-    int32_t nx, ny, rows;   // interior size; rows per wave
-    uint16_t* out;          // HIDDEN/BWD: NHWC BF16, padded, COUT channels
-    const uint16_t* mask;   // BWD: activation whose positive entries pass the gradient
-    float* outf;            // OUT: dense planes [4][ny][nx]
-    float* U;               // APPLY: state planes (interior origin), corrected in place
-    int64_t plane;          // APPLY: elements per plane of U
-    int32_t pitch;          // APPLY: row pitch of U
-    float gamma;            // APPLY: ideal-gas gamma for the pressure check
-    float scale[4];         // APPLY: correction = scale * network output
-    float max_output;       // APPLY: fall back where |output| > max_output (<= 0: no bound)
-    const uint8_t* shock;   // APPLY: per-cell shock flag [ny][nx] (null: none)
-    uint32_t* fallback;     // APPLY: cells left at the plain state
+    const uint16_t* in;       // gradient at the layer's output, NHWC BF16, padded, CIN channels
+    const uint16_t* wa;       // A operands [2][S][64 lanes][8]
+    int32_t nx, ny, rows;     // interior size; rows per wave
+    uint16_t* out;            // NHWC BF16, padded, 32 channels
+    const uint16_t* mask;     // activation whose positive entries pass the gradient
 };
 
 struct WgradArgs {
@@ -85,7 +93,8 @@ struct LossArgs {
 };
 
 // Launchers (hf_cnn.hip).  cin/cout are storage channel counts (8 or 32).
-hipError_t launch_conv(int cin, int cout, int mode, const ConvArgs& a, hipStream_t s);
+hipError_t launch_net(NetArgs a, int mode, hipStream_t s);
+hipError_t launch_conv_bwd(int cin, const ConvArgs& a, hipStream_t s);
 hipError_t launch_wgrad(int ci, int co, const WgradArgs& a, int* nwg, hipStream_t s);
 int wgrad_rows(int nx, int ny);   // rows per workgroup, WgradArgs::rows
 int wgrad_workgroups(int nx, int ny);

@@ -34,16 +34,287 @@ __device__ __forceinline__ bf16x8 zero8()
     return __builtin_bit_cast(bf16x8, v);
 }
 
-// ------------------------------------------------------------- convolution --
-// One wave = one 16-pixel segment of a row, walking `rows` rows.  Lane
-// (g = lane/16, j = lane%16) feeds pixel x0+j and K-chunk g of each MFMA and
-// receives output channels 16*mt + 4g + r (r = 0..3) of pixel x0+j.
-// K-chunk c = 4s+g of MFMA step s is 8 input channels of one tap:
-// CIN = 32: tap s, channels 8g..8g+7;  CIN = 8: tap c (c >= 9 is zero).
-template <int CIN, int COUT, int MODE>
-__global__ __launch_bounds__(256, 3) void k_conv(const ConvArgs a)
+// Two FP32 values as packed BF16, round to nearest even (v_cvt_pk_bf16_f32).
+__device__ __forceinline__ uint32_t pk_bf16(float lo, float hi)
 {
-    constexpr int MT = (COUT + 15) / 16;
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    const f32x2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// A workgroup barrier for data in LDS: waits for this wave's LDS operations
+// only.  (__syncthreads also waits for global loads and stores, here those of
+// rows that are not needed before the next step.)
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Output channels 0..3 of pixel (x, y): stored, or applied to the solver state
+// (u, and its shock flag, requested earlier) with the fallbacks.
+template <int MODE>
+__device__ __forceinline__ void output(const NetArgs& a, int x, int y, const f32x4& acc, const float (&bias)[4],
+                                       const float (&u)[4], uint32_t shock, uint32_t& nfb)
+{
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) v[r] = acc[r] + bias[r];
+    if (MODE == NET_OUT_PLANES) {
+        const int64_t np = (int64_t)a.nx * a.ny;
+#pragma unroll
+        for (int r = 0; r < 4; r++) (a.outf + r * np + (int64_t)y * a.nx)[(uint32_t)x] = v[r];
+        return;
+    }
+    float n[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) n[r] = u[r] + a.scale[r] * v[r];
+    const float p = (a.gamma - 1.0f) * (n[3] - 0.5f * (n[1] * n[1] + n[2] * n[2]) / n[0]);
+    bool inrange = true;
+    if (a.max_output > 0.0f)
+#pragma unroll
+        for (int r = 0; r < 4; r++) inrange = inrange && fabsf(v[r]) <= a.max_output;
+    const bool ok = n[0] > 0.0f && p > 0.0f && !shock && inrange && isfinite(p) && isfinite(n[1]) && isfinite(n[2]) &&
+                    isfinite(n[3]);
+    if (ok) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) (a.U + r * a.plane + (int64_t)y * a.pitch)[(uint32_t)x] = n[r];
+    } else {
+        nfb++;
+    }
+}
+
+// ----------------------------------------------------------------- network --
+// The whole forward pass of an 80-column strip in one workgroup of 8 waves,
+// streaming down its rows: at step s, layer k works on row yc - 4 + s -
+// 2 (k - 1), one row of every layer side by side, and a barrier ends the step.
+// A hidden row goes to LDS (two slots per layer; four after layer 4), from
+// where the next layer reads it one step later; nothing but the packed input
+// and the output touches memory (STORE: also each activation's own pixels, for
+// the backward pass).
+//  * Frame: 96 columns from 8 left of the strip, six 16-pixel segments; each
+//    layer's outermost columns are junk that the next one keeps away from (4
+//    columns of halo per side, 8 kept for alignment).
+//  * Waves 0-5: layers 2-4, two waves each, three segments per wave.  Layer k's
+//    18 weight operands stay in registers, and so does the 3-row window of its
+//    input (a ring of rows named at compile time: three LDS reads per segment
+//    and row).  Waves 6-7: layer 1 (input read from memory a row ahead) and
+//    layer 5 (window read from LDS).
+//  * An MFMA is 16x16x32: A = weights (rows = output channels), B = 32 input
+//    values of 16 pixels.  Lane (g = lane/16, j = lane%16) feeds pixel j and K
+//    chunk g and receives channels 16 mt + 4g + r.  For 32 input channels an
+//    MFMA is one tap; for 8, K chunk 4s + g is tap 4s + g.  Pixels outside the
+//    image are stored as zeros ("same" padding of every layer).
+// Bound by the step's chain (LDS reads, 54 MFMAs per wave with two waves per
+// SIMD, the epilogue, the barrier: about 3 900 cycles of which the MFMAs fill
+// 1 728), H + 12 steps.  As five launches, each layer wrote and read 64 bytes a
+// pixel (27 us of memory time per layer, 40 taken): planes at 1024^2 169 us in
+// all, now 120; corrected state 188, now 172; stored activations at 256^2 27,
+// now 26.  A barrier that waits for LDS only lets the loads and stores of a
+// step cross it (planes 128 us with __syncthreads()); a prefetch of the state a
+// step ahead spilled (250 us).
+constexpr int NET_OUT = 80, NET_SEGS = 6, NET_PX = NET_SEGS * 16 + 2;
+
+template <int MODE, bool STORE>
+__global__ __launch_bounds__(512, 2) void k_net(const NetArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t buf[10][NET_PX][32];
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, j = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nstrip = (a.nx + NET_OUT - 1) / NET_OUT;
+    const int X0 = (int)(blockIdx.x % nstrip) * NET_OUT - 8;
+    const int yc = (int)(blockIdx.x / nstrip) * a.rows, ye = min(a.ny, yc + a.rows);
+    const int W2 = a.nx + 2;
+    const int steps = (ye - yc + 12 + 2) / 3 * 3;   // the waves' loops advance by three
+
+    // A 16-pixel segment of a hidden row: bias, ReLU, BF16, zeros outside the
+    // image, into an LDS row and (STORE) the stored activation.
+    auto finish = [&](int k, int row, int f0, const f32x4 (&acc)[2], const float (&bias)[2][4], uint16_t (*dst)[32]) {
+        const int f = f0 + j, x = X0 + f;
+        const bool in = x >= 0 && x < a.nx;
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++) {
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = fmaxf(acc[mt][r] + bias[mt][r], 0.0f);
+            uint2 pk;
+            pk.x = in ? pk_bf16(v[0], v[1]) : 0u;
+            pk.y = in ? pk_bf16(v[2], v[3]) : 0u;
+            *reinterpret_cast<uint2*>(&dst[f + 1][16 * mt + 4 * g]) = pk;
+            if (STORE && in && f >= 8 && f < 8 + NET_OUT && row >= yc && row < ye)
+                *reinterpret_cast<uint2*>(a.act[k - 1] + ((size_t)(row + 1) * W2 + x + 1) * 32 + 16 * mt + 4 * g) = pk;
+        }
+    };
+    auto zero_row = [&](int f0, uint16_t (*dst)[32]) {
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int mt = 0; mt < 2; mt++)
+                *reinterpret_cast<uint2*>(&dst[f0 + 16 * q + j + 1][16 * mt + 4 * g]) = make_uint2(0u, 0u);
+    };
+    auto load_bias = [&](int k, float (&bias)[2][4]) {
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) bias[mt][r] = a.bias[k - 1][16 * mt + 4 * g + r];
+    };
+    uint32_t nfb = 0;
+
+    if (wave < 6) {   // layers 2-4
+        const int k = 2 + (wave >> 1), f0 = (wave & 1) * 48;
+        bf16x8 wA[2][9];
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int t = 0; t < 9; t++) wA[mt][t] = load8(a.w[k - 1] + ((size_t)(mt * 9 + t) * 64 + lane) * 8);
+        float bias[2][4];
+        load_bias(k, bias);
+        bf16x8 ring[3][3][3];   // [row][segment][column shift]
+        for (int s0 = 0; s0 < steps; s0 += 3) {
+#pragma unroll
+            for (int ph = 0; ph < 3; ph++) {
+                const int s = s0 + ph;
+                const uint16_t (*src)[32] = buf[2 * (k - 2) + ((s + 1) & 1)];   // written last step
+#pragma unroll
+                for (int q = 0; q < 3; q++)
+#pragma unroll
+                    for (int d = 0; d < 3; d++) ring[ph][q][d] = load8(&src[f0 + 16 * q + j + d][8 * g]);
+                const int row = yc - 4 + s - 2 * (k - 1);
+                if (row >= yc - (5 - k) && row < ye + (5 - k)) {
+                    uint16_t (*dst)[32] = buf[k < 4 ? 2 * (k - 1) + (s & 1) : 6 + (s & 3)];
+                    if (row >= 0 && row < a.ny) {
+#pragma unroll
+                        for (int q = 0; q < 3; q++) {   // a segment's epilogue runs beside the next one's MFMAs
+                            f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+                            for (int t = 0; t < 9; t++)
+#pragma unroll
+                                for (int mt = 0; mt < 2; mt++)
+                                    acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                        wA[mt][t], ring[(ph + 1 + t / 3) % 3][q][t % 3], acc[mt], 0, 0, 0);
+                            finish(k, row, f0 + 16 * q, acc, bias, dst);
+                        }
+                    } else {
+                        zero_row(f0, dst);
+                    }
+                }
+                lds_barrier();
+            }
+        }
+    } else {          // layers 1 and 5
+        const int h = wave - 6, f0 = h * 48;
+        bf16x8 w1[2][3], w5[9];
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int t = 0; t < 3; t++) w1[mt][t] = load8(a.w[0] + ((size_t)(mt * 3 + t) * 64 + lane) * 8);
+#pragma unroll
+        for (int t = 0; t < 9; t++) w5[t] = load8(a.w[4] + ((size_t)t * 64 + lane) * 8);
+        float bias[2][4], b5[4];
+        load_bias(1, bias);
+#pragma unroll
+        for (int r = 0; r < 4; r++) b5[r] = g == 0 ? a.bias[4][r] : 0.0f;
+        // layer 1's operands of a row; pixels outside the padded image (which
+        // only junk columns and rows reach) read its nearest ones
+        uint32_t xoff[3][3];   // byte offsets in a row; 32 bits reach the largest image
+        int dy[3];
+#pragma unroll
+        for (int t = 0; t < 3; t++) {
+            const int tap = min(4 * t + g, 8);
+            dy[t] = tap / 3;
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                xoff[q][t] = (uint32_t)min(max(X0 + f0 + 16 * q + j + tap % 3, 0), a.nx + 1) * 16u;
+        }
+        auto fetch = [&](int row, bf16x8 (&dst)[3][3]) {
+#pragma unroll
+            for (int t = 0; t < 3; t++) {
+                const uint32_t yoff = (uint32_t)min(max(row + dy[t], 0), a.ny + 1) * (uint32_t)W2 * 16u;
+#pragma unroll
+                for (int q = 0; q < 3; q++)
+                    dst[q][t] = load8(reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(a.x) +
+                                                                        (yoff + xoff[q][t])));
+            }
+        };
+        // the state under layer 5's output pixels (lanes g = 0)
+        auto fetch_state = [&](int row, float (&u)[3][4], uint32_t (&shock)[3]) {
+            if (MODE != NET_APPLY || row < yc || row >= ye) return;
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                const int x = X0 + 8 + 16 * (3 * h + q) + j;
+                if (3 * h + q < NET_OUT / 16 && g == 0 && x < a.nx) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        u[q][r] = (a.U + r * a.plane + (int64_t)row * a.pitch)[(uint32_t)x];
+                    shock[q] = a.shock ? (a.shock + (int64_t)row * a.nx)[(uint32_t)x] : 0u;
+                }
+            }
+        };
+        bf16x8 in1[3][3][3];   // rings of rows, requested a step ahead
+        fetch(yc - 4, in1[0]);
+        for (int s0 = 0; s0 < steps; s0 += 3) {
+#pragma unroll
+            for (int ph = 0; ph < 3; ph++) {
+                const int s = s0 + ph, r1 = yc - 4 + s, r5 = r1 - 8;
+                if (r1 + 1 < ye + 4) fetch(r1 + 1, in1[(ph + 1) % 3]);
+                float us[3][4];
+                uint32_t sh[3];
+                fetch_state(r5, us, sh);   // used at the step's end
+                if (r1 < ye + 4) {
+                    uint16_t (*dst)[32] = buf[s & 1];
+                    if (r1 >= 0 && r1 < a.ny) {
+#pragma unroll
+                        for (int q = 0; q < 3; q++) {
+                            f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+                            for (int t = 0; t < 3; t++) {
+                                const bf16x8 B = (4 * t + g < 9) ? in1[ph][q][t] : zero8();
+#pragma unroll
+                                for (int mt = 0; mt < 2; mt++)
+                                    acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[mt][t], B, acc[mt], 0, 0, 0);
+                            }
+                            finish(1, r1, f0 + 16 * q, acc, bias, dst);
+                        }
+                    } else {
+                        zero_row(f0, dst);
+                    }
+                }
+                if (r5 >= yc && r5 < ye) {
+                    f32x4 acc[3];
+#pragma unroll
+                    for (int q = 0; q < 3; q++) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int t = 0; t < 9; t++)
+#pragma unroll
+                        for (int q = 0; q < 3; q++) {   // five segments: wave 7's last repeats its second
+                            const int f = 8 + 16 * min(3 * h + q, NET_OUT / 16 - 1) + j;
+                            const bf16x8 B = load8(&buf[6 + ((s + 1 + t / 3) & 3)][f + t % 3][8 * g]);
+                            acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w5[t], B, acc[q], 0, 0, 0);
+                        }
+#pragma unroll
+                    for (int q = 0; q < 3; q++) {
+                        const int x = X0 + 8 + 16 * (3 * h + q) + j;
+                        if (3 * h + q < NET_OUT / 16 && g == 0 && x < a.nx)
+                            output<MODE>(a, x, r5, acc[q], b5, us[q], sh[q], nfb);
+                    }
+                }
+                lds_barrier();
+            }
+        }
+    }
+    if (MODE == NET_APPLY) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) nfb += __shfl_xor(nfb, off);
+        if (lane == 0 && nfb) atomicAdd(a.fallback, nfb);
+    }
+}
+
+// --------------------------------------------------------- data gradient --
+// The gradient at a hidden layer's input: the convolution with the taps
+// flipped and the channels swapped (the packed weights), times the ReLU mask of
+// the stored activation.  One wave = one 16-pixel segment of a row, walking
+// `rows` rows; operands and results lie as in k_net.
+template <int CIN>
+__global__ __launch_bounds__(256, 3) void k_conv_bwd(const ConvArgs a)
+{
+    constexpr int COUT = 32, MT = 2;
     constexpr int S = (9 * CIN / 8 + 3) / 4;
     const int lane = threadIdx.x & 63;
     const int g = lane >> 4, j = lane & 15;
@@ -61,74 +332,20 @@ __global__ __launch_bounds__(256, 3) void k_conv(const ConvArgs a)
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int s = 0; s < S; s++) wA[mt][s] = load8(a.wa + ((size_t)(mt * S + s) * 64 + lane) * 8);
-    float bias[MT][4];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int o = 16 * mt + 4 * g + r;
-            bias[mt][r] = (MODE != CONV_BWD && o < a.co_real) ? a.bias[o] : 0.0f;
-        }
 
-    uint32_t nfb = 0;
-    // A row's epilogue: bias, then ReLU (hidden layer), the stored
-    // activation's ReLU mask (data gradient), the FP32 output, or the
-    // correction applied to the solver state with its fallbacks.
     auto finish = [&](const int y, const f32x4 (&acc)[MT]) {
         const size_t pix = (size_t)(y + 1) * W2 + (x + 1);
-        if (MODE == CONV_HIDDEN || MODE == CONV_BWD) {
 #pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                float v[4];
-#pragma unroll
-                for (int r = 0; r < 4; r++) v[r] = acc[mt][r] + bias[mt][r];
-                uint16_t* dst = a.out + pix * COUT + 16 * mt + 4 * g;
-                if (MODE == CONV_HIDDEN) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) v[r] = v[r] > 0.0f ? v[r] : 0.0f;
-                } else {
-                    const uint2 m = *reinterpret_cast<const uint2*>(a.mask + pix * COUT + 16 * mt + 4 * g);
-                    const uint32_t mv[4] = {m.x & 0xffffu, m.x >> 16, m.y & 0xffffu, m.y >> 16};
-#pragma unroll
-                    for (int r = 0; r < 4; r++) v[r] = (mv[r] != 0u && mv[r] < 0x8000u) ? v[r] : 0.0f;
-                }
-                uint2 pk;
-                pk.x = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
-                pk.y = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
-                *reinterpret_cast<uint2*>(dst) = pk;
-            }
-        } else if (g == 0) {
-            // output channels 0..3 of pixel x (lanes 0..15)
+        for (int mt = 0; mt < MT; mt++) {
+            const uint2 m = *reinterpret_cast<const uint2*>(a.mask + pix * COUT + 16 * mt + 4 * g);
+            const uint32_t mv[4] = {m.x & 0xffffu, m.x >> 16, m.y & 0xffffu, m.y >> 16};
             float v[4];
 #pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = acc[0][r] + bias[0][r];
-            if (MODE == CONV_OUT) {
-                const size_t np = (size_t)a.nx * a.ny;
-#pragma unroll
-                for (int r = 0; r < 4; r++) a.outf[r * np + (size_t)y * a.nx + x] = v[r];
-            } else {
-                float* U = a.U + (size_t)y * a.pitch + x;
-                float u[4], n[4];
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    u[r] = U[r * a.plane];
-                    n[r] = u[r] + a.scale[r] * v[r];
-                }
-                const float p = (a.gamma - 1.0f) * (n[3] - 0.5f * (n[1] * n[1] + n[2] * n[2]) / n[0]);
-                const bool shock = a.shock && a.shock[(size_t)y * a.nx + x];
-                bool inrange = true;
-                if (a.max_output > 0.0f)
-#pragma unroll
-                    for (int r = 0; r < 4; r++) inrange = inrange && fabsf(v[r]) <= a.max_output;
-                const bool ok = n[0] > 0.0f && p > 0.0f && !shock && inrange && isfinite(p) && isfinite(n[1]) &&
-                                isfinite(n[2]) && isfinite(n[3]);
-                if (ok) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) U[r * a.plane] = n[r];
-                } else {
-                    nfb++;
-                }
-            }
+            for (int r = 0; r < 4; r++) v[r] = (mv[r] != 0u && mv[r] < 0x8000u) ? acc[mt][r] : 0.0f;
+            uint2 pk;
+            pk.x = pk_bf16(v[0], v[1]);
+            pk.y = pk_bf16(v[2], v[3]);
+            *reinterpret_cast<uint2*>(a.out + pix * COUT + 16 * mt + 4 * g) = pk;
         }
     };
 
@@ -188,11 +405,6 @@ __global__ __launch_bounds__(256, 3) void k_conv(const ConvArgs a)
             }
             finish(y, acc);
         }
-    }
-    if (MODE == CONV_APPLY) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) nfb += __shfl_xor(nfb, off);
-        if (lane == 0 && nfb) atomicAdd(a.fallback, nfb);
     }
 }
 
@@ -521,25 +733,30 @@ __global__ __launch_bounds__(256) void k_restrict2(const float* __restrict__ U, 
 }
 
 // ---------------------------------------------------------------- launchers --
-namespace {
-template <int CIN, int COUT, int MODE>
-hipError_t conv_t(const ConvArgs& a, hipStream_t s)
+hipError_t launch_net(NetArgs a, int mode, hipStream_t s)
 {
-    const int waves = (a.nx / 16) * ((a.ny + a.rows - 1) / a.rows);
-    hipLaunchKernelGGL((k_conv<CIN, COUT, MODE>), dim3((waves + 3) / 4), dim3(256), 0, s, a);
+    // one workgroup fills a CU: rows so that one round of the 256 CUs takes the
+    // image, at least 4 (a strip's steps are its rows and 12 more)
+    const int nstrip = (a.nx + NET_OUT - 1) / NET_OUT;
+    const int chunks = nstrip < 256 ? 256 / nstrip : 1;
+    a.rows = (a.ny + chunks - 1) / chunks;
+    if (a.rows < 4) a.rows = 4;
+    if (a.rows > 128) a.rows = 128;
+    const dim3 grid(nstrip * ((a.ny + a.rows - 1) / a.rows));
+    if (mode == NET_APPLY) hipLaunchKernelGGL((k_net<NET_APPLY, false>), grid, dim3(512), 0, s, a);
+    else if (a.act[0]) hipLaunchKernelGGL((k_net<NET_OUT_PLANES, true>), grid, dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((k_net<NET_OUT_PLANES, false>), grid, dim3(512), 0, s, a);
     return hipGetLastError();
 }
-}  // namespace
 
-hipError_t launch_conv(int cin, int cout, int mode, const ConvArgs& a, hipStream_t s)
+hipError_t launch_conv_bwd(int cin, const ConvArgs& a, hipStream_t s)
 {
-    if (cin == 8 && cout == 32 && mode == CONV_HIDDEN) return conv_t<8, 32, CONV_HIDDEN>(a, s);
-    if (cin == 32 && cout == 32 && mode == CONV_HIDDEN) return conv_t<32, 32, CONV_HIDDEN>(a, s);
-    if (cin == 32 && cout == 8 && mode == CONV_OUT) return conv_t<32, 8, CONV_OUT>(a, s);
-    if (cin == 32 && cout == 8 && mode == CONV_APPLY) return conv_t<32, 8, CONV_APPLY>(a, s);
-    if (cin == 32 && cout == 32 && mode == CONV_BWD) return conv_t<32, 32, CONV_BWD>(a, s);
-    if (cin == 8 && cout == 32 && mode == CONV_BWD) return conv_t<8, 32, CONV_BWD>(a, s);
-    return hipErrorInvalidValue;
+    const int waves = (a.nx / 16) * ((a.ny + a.rows - 1) / a.rows);
+    const dim3 grid((waves + 3) / 4);
+    if (cin == 8) hipLaunchKernelGGL((k_conv_bwd<8>), grid, dim3(256), 0, s, a);
+    else if (cin == 32) hipLaunchKernelGGL((k_conv_bwd<32>), grid, dim3(256), 0, s, a);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
 }
 
 // Rows per workgroup: the most, up to 16, that still make two workgroups for

@@ -67,6 +67,7 @@ struct hf_net {
     uint16_t* act[4] = {};
     uint16_t* g8 = nullptr;
     uint16_t* gz[2] = {};
+    bool trains = false;      // the buffers of the backward pass are there
     float* y = nullptr;
     uint8_t* shock = nullptr;
     float* part[NL] = {};     // weight-gradient partials of each layer
@@ -80,33 +81,49 @@ struct hf_net {
 
 namespace {
 
-void free_images(hf_net* n)
+// The backward pass's buffers.
+void free_training(hf_net* n)
 {
-    (void)hipFree(n->x);
     for (auto& p : n->act) (void)hipFree(p), p = nullptr;
     (void)hipFree(n->g8);
     for (auto& p : n->gz) (void)hipFree(p), p = nullptr;
     (void)hipFree(n->y);
-    (void)hipFree(n->shock);
     for (auto& p : n->part) (void)hipFree(p), p = nullptr;
     (void)hipFree(n->lossp);
-    n->x = n->g8 = nullptr;
+    n->g8 = nullptr;
     n->y = n->lossp = nullptr;
+    n->trains = false;
+}
+
+void free_images(hf_net* n)
+{
+    free_training(n);
+    (void)hipFree(n->x);
+    (void)hipFree(n->shock);
+    n->x = nullptr;
     n->shock = nullptr;
     n->nx = n->ny = 0;
 }
 
-// Buffers for nx x ny images; borders zeroed once.
-int ensure_images(hf_net* n, int nx, int ny)
+// Buffers for nx x ny images (the backward pass's on its first use); borders
+// zeroed once.
+int ensure_images(hf_net* n, int nx, int ny, bool training)
 {
     if (nx < 64 || nx % 64 != 0 || ny < 1) return fail(HF_EINVAL, "learned correction: nx must be a positive multiple of 64");
-    if (n->nx == nx && n->ny == ny) return HF_OK;
-    HF_HIP(hipDeviceSynchronize());
-    free_images(n);
     const size_t pix = (size_t)(nx + 2) * (ny + 2);
-    HF_HIP(hipMalloc(&n->x, pix * 8 * 2));
+    if (n->nx != nx || n->ny != ny) {
+        HF_HIP(hipDeviceSynchronize());
+        free_images(n);
+        HF_HIP(hipMalloc(&n->x, pix * 8 * 2));
+        HF_HIP(hipMemset(n->x, 0, pix * 8 * 2));
+        HF_HIP(hipMalloc(&n->shock, (size_t)nx * ny));
+        n->nx = nx;
+        n->ny = ny;
+    }
+    if (!training || n->trains) return HF_OK;
+    HF_HIP(hipDeviceSynchronize());
+    free_training(n);   // what an attempt that ran out of memory left
     HF_HIP(hipMalloc(&n->g8, pix * 8 * 2));
-    HF_HIP(hipMemset(n->x, 0, pix * 8 * 2));
     HF_HIP(hipMemset(n->g8, 0, pix * 8 * 2));
     for (auto& p : n->act) {
         HF_HIP(hipMalloc(&p, pix * 32 * 2));
@@ -117,14 +134,12 @@ int ensure_images(hf_net* n, int nx, int ny)
         HF_HIP(hipMemset(p, 0, pix * 32 * 2));
     }
     HF_HIP(hipMalloc(&n->y, (size_t)nx * ny * 4 * sizeof(float)));
-    HF_HIP(hipMalloc(&n->shock, (size_t)nx * ny));
     const int nwg = hfn::wgrad_workgroups(nx, ny);
     for (int l = 0; l < NL; l++)
         HF_HIP(hipMalloc(&n->part[l], (size_t)nwg * (9 * LAYERS[l].cis + 1) * LAYERS[l].cos * sizeof(float)));
     const int nloss = (int)(((int64_t)nx * ny + 255) / 256);
     HF_HIP(hipMalloc(&n->lossp, (size_t)nloss * sizeof(float)));
-    n->nx = nx;
-    n->ny = ny;
+    n->trains = true;
     return HF_OK;
 }
 
@@ -151,22 +166,8 @@ int pack_weights(hf_net* n, hipStream_t s)
     return HF_OK;
 }
 
-hfn::ConvArgs conv_args(const hf_net* n, int l, const uint16_t* in, int nx, int ny)
-{
-    hfn::ConvArgs a;
-    std::memset(&a, 0, sizeof a);
-    a.in = in;
-    a.wa = n->wf[l];
-    a.bias = n->params + LAYERS[l].off + 9 * LAYERS[l].ci * LAYERS[l].co;
-    a.co_real = LAYERS[l].co;
-    a.nx = nx;
-    a.ny = ny;
-    a.rows = conv_rows(nx, ny);
-    return a;
-}
-
-// Input packing and layers 1-4 (activations act[0..3]).
-int forward_hidden(hf_net* n, const float* U, int64_t plane, int pitch, int nx, int ny, bool sensor, hipStream_t s)
+// Input packing (and the shock sensor) into n->x.
+int pack_input(hf_net* n, const float* U, int64_t plane, int pitch, int nx, int ny, bool sensor, hipStream_t s)
 {
     hfn::PackArgs p;
     std::memset(&p, 0, sizeof p);
@@ -184,14 +185,23 @@ int forward_hidden(hf_net* n, const float* U, int64_t plane, int pitch, int nx, 
     p.gamma = n->d.gamma;
     p.theta = n->d.shock_threshold;
     HF_HIP(hfn::launch_pack(p, s));
-    const uint16_t* in = n->x;
-    for (int l = 0; l < 4; l++) {
-        hfn::ConvArgs a = conv_args(n, l, in, nx, ny);
-        a.out = n->act[l];
-        HF_HIP(hfn::launch_conv(LAYERS[l].cis, LAYERS[l].cos, hfn::CONV_HIDDEN, a, s));
-        in = n->act[l];
-    }
     return HF_OK;
+}
+
+// The forward pass over n->x, into outf unless the caller sets up more.
+hfn::NetArgs net_args(const hf_net* n, int nx, int ny, float* outf)
+{
+    hfn::NetArgs a;
+    std::memset(&a, 0, sizeof a);
+    a.x = n->x;
+    for (int l = 0; l < NL; l++) {
+        a.w[l] = n->wf[l];
+        a.bias[l] = n->params + LAYERS[l].off + 9 * LAYERS[l].ci * LAYERS[l].co;
+    }
+    a.nx = nx;
+    a.ny = ny;
+    a.outf = outf;
+    return a;
 }
 
 int wgrad(hf_net* n, int l, const uint16_t* a_in, const uint16_t* gz, int nx, int ny, hfn::ReduceArgs& red,
@@ -215,11 +225,11 @@ int wgrad(hf_net* n, int l, const uint16_t* a_in, const uint16_t* gz, int nx, in
 int gradients(hf_net* n, const float* u, const float* target, int nx, int ny, hipStream_t s)
 {
     const int64_t np = (int64_t)nx * ny;
-    int rc = forward_hidden(n, u, np, nx, nx, ny, false, s);
+    int rc = pack_input(n, u, np, nx, nx, ny, false, s);
     if (rc) return rc;
-    hfn::ConvArgs a = conv_args(n, 4, n->act[3], nx, ny);
-    a.outf = n->y;
-    HF_HIP(hfn::launch_conv(32, 8, hfn::CONV_OUT, a, s));
+    hfn::NetArgs a = net_args(n, nx, ny, n->y);
+    for (int l = 0; l < 4; l++) a.act[l] = n->act[l];
+    HF_HIP(hfn::launch_net(a, hfn::NET_OUT_PLANES, s));
 
     hfn::LossArgs la;
     std::memset(&la, 0, sizeof la);
@@ -256,7 +266,7 @@ int gradients(hf_net* n, const float* u, const float* target, int nx, int ny, hi
         b.rows = conv_rows(nx, ny);
         b.out = gout;
         b.mask = n->act[l - 1];
-        HF_HIP(hfn::launch_conv(cin, 32, hfn::CONV_BWD, b, s));
+        HF_HIP(hfn::launch_conv_bwd(cin, b, s));
         const uint16_t* a_in = (l - 1 == 0) ? n->x : n->act[l - 2];
         rc = wgrad(n, l - 1, a_in, gout, nx, ny, red, s);
         if (rc) return rc;
@@ -397,23 +407,21 @@ int hf_net_reset_optimizer(hf_net* n)
 int hf_net_forward(hf_net* n, const float* u, int nx, int ny, float* y)
 {
     if (!n || !u || !y) return fail(HF_EINVAL, "hf_net_forward: null argument");
-    int rc = ensure_images(n, nx, ny);
+    int rc = ensure_images(n, nx, ny, false);
     if (rc) return rc;
     rc = order_after(n, n->stream);
     if (rc) return rc;
     const int64_t np = (int64_t)nx * ny;
-    rc = forward_hidden(n, u, np, nx, nx, ny, false, n->stream);
+    rc = pack_input(n, u, np, nx, nx, ny, false, n->stream);
     if (rc) return rc;
-    hfn::ConvArgs a = conv_args(n, 4, n->act[3], nx, ny);
-    a.outf = y;
-    HF_HIP(hfn::launch_conv(32, 8, hfn::CONV_OUT, a, n->stream));
+    HF_HIP(hfn::launch_net(net_args(n, nx, ny, y), hfn::NET_OUT_PLANES, n->stream));
     return mark_done(n, n->stream);
 }
 
 int hf_net_gradients(hf_net* n, const float* u, const float* target, int nx, int ny, float* grads, float* loss)
 {
     if (!n || !u || !target) return fail(HF_EINVAL, "hf_net_gradients: null argument");
-    int rc = ensure_images(n, nx, ny);
+    int rc = ensure_images(n, nx, ny, true);
     if (rc) return rc;
     rc = order_after(n, n->stream);
     if (rc) return rc;
@@ -429,7 +437,7 @@ int hf_net_train_step(hf_net* n, const float* u, const float* target, int nx, in
 {
     if (!n || !u || !target) return fail(HF_EINVAL, "hf_net_train_step: null argument");
     if (!(lr > 0.0f) || !std::isfinite(lr)) return fail(HF_EINVAL, "hf_net_train_step: lr must be finite and > 0");
-    int rc = ensure_images(n, nx, ny);
+    int rc = ensure_images(n, nx, ny, true);
     if (rc) return rc;
     rc = order_after(n, n->stream);
     if (rc) return rc;
@@ -482,13 +490,13 @@ int hf_correct(hf_ctx* c, hf_net* n, int64_t* fallback)
     if (fallback) HF_HIP(hipMemsetAsync(n->fallback, 0, sizeof(uint32_t), c->stream));
     for (int b = 0; b < c->nb; b++) {
         const HfBlockDev& B = c->blocks[b];
-        rc = ensure_images(n, B.nx, B.ny);
+        rc = ensure_images(n, B.nx, B.ny, false);
         if (rc) return rc;
         float* U = interior(c, b);
         const bool sensor = n->d.shock_threshold > 0.0f;
-        rc = forward_hidden(n, U, B.plane, B.pitch, B.nx, B.ny, sensor, c->stream);
+        rc = pack_input(n, U, B.plane, B.pitch, B.nx, B.ny, sensor, c->stream);
         if (rc) return rc;
-        hfn::ConvArgs a = conv_args(n, 4, n->act[3], B.nx, B.ny);
+        hfn::NetArgs a = net_args(n, B.nx, B.ny, nullptr);
         a.U = U;
         a.plane = B.plane;
         a.pitch = B.pitch;
@@ -497,7 +505,7 @@ int hf_correct(hf_ctx* c, hf_net* n, int64_t* fallback)
         a.max_output = n->d.max_output;
         a.shock = sensor ? n->shock : nullptr;
         a.fallback = n->fallback;
-        HF_HIP(hfn::launch_conv(32, 8, hfn::CONV_APPLY, a, c->stream));
+        HF_HIP(hfn::launch_net(a, hfn::NET_APPLY, c->stream));
     }
     rc = mark_done(n, c->stream);
     if (rc) return rc;

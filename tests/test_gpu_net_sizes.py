@@ -24,3 +24,20 @@ def test_gradients_at_sizes(ny, nx):
     for l in range(5):
         a = slice(OFFS[l], OFFS[l + 1])
         assert np.linalg.norm(g[a] - gr[a]) < 1e-2 * np.linalg.norm(gr[a])
+
+
+@pytest.mark.parametrize("ny,nx", [(1, 64), (4, 64), (5, 128), (66, 192), (300, 64), (9, 704)])
+def test_forward_at_sizes(ny, nx):
+    """Strips of 80 columns and their chunks of rows: images narrower than a
+    strip, ending inside one, of one row and of several chunks; every pixel,
+    the edges above all, within the bounds of the full-size test."""
+    net = native.Net(**NORM, seed=nx)
+    u = state(ny + nx, ny, nx).astype(np.float32)
+    y = torch.full((4, ny, nx), float("nan"), device="cuda")
+    net.forward(dev(u), y)
+    net.synchronize()
+    torch.cuda.synchronize()
+    yr, _ = R.forward(net.get_params(), u, NORM["in_mean"], NORM["in_scale"], emulate=True)
+    yg = y.cpu().numpy().astype(np.float64)
+    assert np.max(np.abs(yg - yr)) < 2e-3 * np.max(np.abs(yr))
+    assert np.mean(np.abs(yg - yr)) < 2e-4 * np.mean(np.abs(yr))

@@ -72,18 +72,152 @@ __device__ __forceinline__ void block_min_to_slot(unsigned long long cand, unsig
     }
 }
 
+// The general division and root (QUICK false) or those of hf::q64, whose
+// range the rotated states are checked against: their masks gather in bad.
+template <bool QUICK>
+struct Face;
+template <>
+struct Face<false> {
+    typedef hf::State<R> State;
+    static __device__ __forceinline__ State state(const double U[4], double gamma, double g1, double, hf::q64::mask&,
+                                                  const hf::q64::Limits&)
+    {
+        return hf::make_state<MathF64>(U, gamma, g1);
+    }
+    static __device__ __forceinline__ void hllc(const State& L, const State& Rs, double F[4], hf::q64::mask&,
+                                                const hf::q64::Limits&)
+    {
+        hf::hllc<MathF64, true>(L, Rs, F);
+    }
+    static __device__ __forceinline__ double dt(const double U[4], double dr, double gamma, double g1, hf::q64::mask&,
+                                                const hf::q64::Limits&)
+    {
+        return cell_dt(U, dr, gamma, g1);
+    }
+};
+template <>
+struct Face<true> {
+    typedef hf::q64::State State;
+    static __device__ __forceinline__ State state(const double U[4], double gamma, double g1, double ig1,
+                                                  hf::q64::mask& bad, const hf::q64::Limits& lim)
+    {
+        bad |= hf::q64::out_of_range(U, lim);
+        return hf::q64::make_state(U, gamma, g1, ig1, bad, lim);
+    }
+    static __device__ __forceinline__ void hllc(const State& L, const State& Rs, double F[4], hf::q64::mask& bad,
+                                                const hf::q64::Limits& lim)
+    {
+        hf::q64::hllc<true>(L, Rs, F, bad, lim);
+    }
+    // A momentum too small for the quotient leaves a speed far below the last
+    // bit of the sound speed; at rest the root of zero is set apart.  A NaN in
+    // the new state, a pressure of zero or below make the sum NaN.
+    static __device__ __forceinline__ double dt(const double U[4], double dr, double gamma, double g1,
+                                                hf::q64::mask& bad, const hf::q64::Limits& lim)
+    {
+        const double y = hf::q64::rcp(U[0]);
+        const double u = hf::q64::div_pos(U[1], U[0], y), v = hf::q64::div_pos(U[2], U[0], y);
+        const double q2 = u * u + v * v;
+        const double p = g1 * hf::q64::fma(-0.5, U[0] * q2, U[3]);
+        const double speed = q2 == 0.0 ? 0.0 : hf::q64::sqrt(q2);
+        const double d = speed + hf::q64::sqrt(hf::q64::div_pos(gamma * p, U[0], y));
+        bad |= __ballot(!(U[0] >= lim.low)) | __ballot(!(U[3] >= lim.low)) | __ballot(!(d == d)) |
+               __ballot(!(dr >= 0x1p-200)) | __ballot(!(dr <= 0x1p200));
+        return hf::q64::div_pos(dr, d, hf::q64::rcp(d));
+    }
+};
+
 // GodunovScheme::operator() (scheme/godunov/godunov.cpp:31-77), boundary
 // states of BoundaryConditions (scheme/boundary/boundary.cpp:29-69), and
-// ForwardEulerODESolver (scheme/ode/forward_euler/forward_euler.cpp:16-30).
-// Four waves per SIMD: the compiler's free choice is 132 VGPRs (three waves);
-// at 128 it needs no spills and the latency of the neighbour gathers hides
-// better (0.0986 -> 0.0931 ms per step on 1.47 M cells).
+// ForwardEulerODESolver (scheme/ode/forward_euler/forward_euler.cpp:16-30) of
+// one cell: its new state and its term of the next dt.  Returns the lanes out
+// of range (QUICK).
+template <bool QUICK>
+__device__ __forceinline__ hf::q64::mask advance_cell(const UnsMesh& m, const UnsStep& s, int c, double dt, double N[4],
+                                                      double& term)
+{
+    typedef Face<QUICK> Fc;
+    const int n = m.n;
+    const double gamma = m.gamma, g1 = m.gamma - 1.0;
+    const double ig1 = QUICK ? 1.0 / g1 : 0.0;
+    const hf::q64::Limits lim;
+    hf::q64::mask bad = 0;
+    double U[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) U[k] = s.A[(size_t)k * n + c];
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    double shortest = 1e16;
+#pragma unroll 1   // see k_uns_step
+    for (int e = 0; e < 4; e++) {
+        const int nb = m.nbr[(size_t)e * n + c];
+        const int ct = m.cs_terms;
+        const double cr = m.cs[(size_t)(ct * e + 0) * n + c], sr = m.cs[(size_t)(ct * e + 1) * n + c];
+        double cb = cr, sb = -sr;   // the back rotation mirrors the forward one (checked on the host)
+        if (ct == 4) {
+            cb = m.cs[(size_t)(4 * e + 2) * n + c];
+            sb = m.cs[(size_t)(4 * e + 3) * n + c];
+        }
+        double V[4];
+        if (nb >= 0) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) V[k] = s.A[(size_t)k * n + nb];
+        } else if (nb == -1) {   // reflective (boundary.cpp:48-56)
+            double t[4];
+            rotate(cr, sr, U, t);
+            t[1] *= -1.0;
+            rotate(cb, sb, t, V);
+        } else if (nb == -2) {   // transmissive
+#pragma unroll
+            for (int k = 0; k < 4; k++) V[k] = U[k];
+        } else {                 // inlet
+#pragma unroll
+            for (int k = 0; k < 4; k++) V[k] = m.inlet[k];
+        }
+        double rU[4], rV[4], F[4], f[4];
+        rotate(cr, sr, U, rU);
+        rotate(cr, sr, V, rV);
+        const typename Fc::State L = Fc::state(rU, gamma, g1, ig1, bad, lim);
+        const typename Fc::State Rs = Fc::state(rV, gamma, g1, ig1, bad, lim);
+        Fc::hllc(L, Rs, F, bad, lim);
+        rotate(cb, sb, F, f);
+        const double len = m.len[(size_t)e * n + c];
+        shortest = (shortest < len) ? shortest : len;   // Polygon's incircle radius (polygon.cpp:79-91)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            f[k] *= len;
+            acc[k] += f[k];
+        }
+    }
+    const double iv = m.inv_vol[c];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        double x = acc[k];
+        x *= iv;
+        x *= -1.0;
+        x *= dt;
+        x += U[k];
+        N[k] = x;
+    }
+    term = Fc::dt(N, shortest, gamma, g1, bad, lim);
+    return bad;
+}
+
+// One step.  A wave runs hf::q64's arithmetic and, where a lane is out of its
+// range, the general one over it.
+// Bound by FP64 arithmetic: 274 VALU instructions per edge, 6 of them
+// quarter-rate (362 and 14 by the general one), with the edges in a loop so
+// that four waves per SIMD keep their registers (108; unrolled, the edges'
+// values are spilled at four waves, and at two or three waves, where they fit,
+// a step takes 27 and 29 us).  The memory side alone (184 bytes a cell) takes
+// 14.2 us, the arithmetic alone 19.8.  367 500 cells: 27.1 -> 22.3 us a step.
+// Not faster: an edge's reads requested an edge ahead (22.1-23.2), a wave per
+// edge and 64 cells per workgroup (23.7), one-wave workgroups (22.8), five
+// waves per SIMD (25.6, 8 registers spilled).
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_uns_step(const UnsMesh m,
                                                                                           const UnsStep s)
 {
     const int c = cell_chunk() * 256 + threadIdx.x;
     const int n = m.n;
-    const double gamma = m.gamma, g1 = m.gamma - 1.0;
     const int lane = threadIdx.x & 63;
     double dt;
     const long long kcall = s.kdev ? (long long)s.kdev[s.kpar] + 1 : s.kcall;
@@ -100,65 +234,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
     unsigned long long cand = ~0ull;
     if (c < n) {
-        double U[4];
+        double N[4], term;
+        hf::q64::mask bad = ~0ull;
+        if (hf::q64::constants_in_range(m.gamma, m.gamma - 1.0)) bad = advance_cell<true>(m, s, c, dt, N, term);
+        if (bad) advance_cell<false>(m, s, c, dt, N, term);
 #pragma unroll
-        for (int k = 0; k < 4; k++) U[k] = s.A[(size_t)k * n + c];
-        double acc[4] = {0.0, 0.0, 0.0, 0.0};
-        double shortest = 1e16;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int nb = m.nbr[(size_t)e * n + c];
-            const int ct = m.cs_terms;
-            const double cr = m.cs[(size_t)(ct * e + 0) * n + c], sr = m.cs[(size_t)(ct * e + 1) * n + c];
-            double cb = cr, sb = -sr;   // the back rotation mirrors the forward one (checked on the host)
-            if (ct == 4) {
-                cb = m.cs[(size_t)(4 * e + 2) * n + c];
-                sb = m.cs[(size_t)(4 * e + 3) * n + c];
-            }
-            double V[4];
-            if (nb >= 0) {
-#pragma unroll
-                for (int k = 0; k < 4; k++) V[k] = s.A[(size_t)k * n + nb];
-            } else if (nb == -1) {   // reflective (boundary.cpp:48-56)
-                double t[4];
-                rotate(cr, sr, U, t);
-                t[1] *= -1.0;
-                rotate(cb, sb, t, V);
-            } else if (nb == -2) {   // transmissive
-#pragma unroll
-                for (int k = 0; k < 4; k++) V[k] = U[k];
-            } else {                 // inlet
-#pragma unroll
-                for (int k = 0; k < 4; k++) V[k] = m.inlet[k];
-            }
-            double rU[4], rV[4], F[4], f[4];
-            rotate(cr, sr, U, rU);
-            rotate(cr, sr, V, rV);
-            const hf::State<R> L = hf::make_state<MathF64>(rU, gamma, g1);
-            const hf::State<R> Rs = hf::make_state<MathF64>(rV, gamma, g1);
-            hf::hllc<MathF64, true>(L, Rs, F);
-            rotate(cb, sb, F, f);
-            const double len = m.len[(size_t)e * n + c];
-            shortest = (shortest < len) ? shortest : len;   // Polygon's incircle radius (polygon.cpp:79-91)
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                f[k] *= len;
-                acc[k] += f[k];
-            }
-        }
-        const double iv = m.inv_vol[c];
-        double N[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            double x = acc[k];
-            x *= iv;
-            x *= -1.0;
-            x *= dt;
-            x += U[k];
-            N[k] = x;
-            s.B[(size_t)k * n + c] = x;
-        }
-        if (s.wr >= 0) cand = bits_of(cell_dt(N, shortest, gamma, g1));
+        for (int k = 0; k < 4; k++) s.B[(size_t)k * n + c] = N[k];
+        cand = bits_of(term);
     }
     if (s.wr >= 0) block_min_to_slot(cand, s.slots + s.wr * SLOT_WORDS);
 }

@@ -577,7 +577,7 @@ void to_device_layout(const hf_ctx* c, int b, const double* src, std::vector<R>&
 }
 
 template <class R>
-void from_device_layout(const hf_ctx* c, int b, const std::vector<R>& src, double* dst)
+void from_device_layout(const hf_ctx* c, int b, const R* src, double* dst)
 {
     const HfBlockDev& B = c->blocks[b];
     for (int v = 0; v < 4; v++)
@@ -589,15 +589,27 @@ void from_device_layout(const hf_ctx* c, int b, const std::vector<R>& src, doubl
 int download_block(hf_ctx* c, int b, const void* base, int64_t off, double* out)
 {
     const HfBlockDev& B = c->blocks[b];
+    const size_t n = (size_t)4 * B.tx * B.ty;
+    if (n > hfhost::SMALL) {
+        hipError_t e;
+        const bool staged = hfhost::to_host(c->stage, c->stream, n, out, e, [&](size_t first, size_t count, double* dst) {
+            return c->prec == HF_FP64
+                       ? hf::launch_dense<double>(B, (const double*)base + off, first, (uint32_t)count, dst, c->stream)
+                       : hf::launch_dense<float>(B, (const float*)base + off, first, (uint32_t)count, dst, c->stream);
+        });
+        HF_HIP(e);
+        if (staged) return HF_OK;
+    }
     HF_HIP(hipStreamSynchronize(c->stream));
+    const size_t elems = (size_t)B.plane * 4;
     if (c->prec == HF_FP64) {
-        std::vector<double> tmp((size_t)B.plane * 4);
-        HF_HIP(hipMemcpy(tmp.data(), (const double*)base + off, tmp.size() * 8, hipMemcpyDeviceToHost));
-        from_device_layout<double>(c, b, tmp, out);
+        const std::unique_ptr<double[]> tmp(new double[elems]);
+        HF_HIP(hipMemcpy(tmp.get(), (const double*)base + off, elems * 8, hipMemcpyDeviceToHost));
+        from_device_layout<double>(c, b, tmp.get(), out);
     } else {
-        std::vector<float> tmp((size_t)B.plane * 4);
-        HF_HIP(hipMemcpy(tmp.data(), (const float*)base + off, tmp.size() * 4, hipMemcpyDeviceToHost));
-        from_device_layout<float>(c, b, tmp, out);
+        const std::unique_ptr<float[]> tmp(new float[elems]);
+        HF_HIP(hipMemcpy(tmp.get(), (const float*)base + off, elems * 4, hipMemcpyDeviceToHost));
+        from_device_layout<float>(c, b, tmp.get(), out);
     }
     return HF_OK;
 }
@@ -1020,6 +1032,7 @@ void hf_destroy(hf_ctx* c)
                     (void*)c->d_fixed, (void*)c->d_fixstats, (void*)c->d_sync, (void*)c->d_rounds, (void*)c->d_pending, (void*)c->d_skip,
                     (void*)c->d_skip_next})
         if (p) (void)hipFree(p);
+    c->stage.release();
     if (c->h_calls_pinned) (void)hipHostFree(c->h_calls_pinned);
     if (c->calls_copied) (void)hipEventDestroy(c->calls_copied);
     if (c->stream) (void)hipStreamDestroy(c->stream);

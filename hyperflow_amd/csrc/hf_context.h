@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/hyperflow.h"
+#include "hf_hostcopy.h"
 #include "hf_common.h"
 
 // Records msg as the calling thread's last error and returns code.
@@ -85,6 +86,7 @@ struct hf_ctx {
     int64_t resid_elems = 0;
     std::vector<int64_t> calls;     // host mirror of the TimeStep call counters
     hipStream_t stream = nullptr;
+    hfhost::Stage stage;             // pinned pieces of large downloads
     // captured step loops by (steps, start parity, fixed-dt bits or 0 for the CFL dt, turn)
     std::map<std::tuple<int, int, uint64_t, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
 

@@ -1,0 +1,112 @@
+// hf_hostcopy.h -- device fields into pageable host memory, in pieces.
+//
+// A copy to pageable memory runs at 17.5 GB/s where the pages exist, and one
+// host thread touching fresh pages at 3-4 GB/s; pinned memory takes 57 GB/s.
+// Here the device fills pinned pieces (packing and converting on the way) and
+// several threads carry them to the caller's array, so that page faults and
+// copies of different pieces overlap.  A 2048^2 block (134 MB in binary64):
+// 40.4 -> 3.3 ms.
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstring>
+#include <system_error>
+#include <thread>
+#include <vector>
+
+namespace hfhost {
+
+constexpr int LANES = 8;                       // pieces in flight, each with its thread
+constexpr size_t PIECE = (size_t)1 << 18;      // doubles of a piece: 2 MiB
+// Up to 8 MiB the copy through one pageable array stays: at 5 MB the pieces
+// save 0.3 ms of 0.5, and pinning them costs the first copy 1.2.
+constexpr size_t SMALL = (size_t)1 << 20;
+
+// Pinned pieces of one context, allocated by its first large copy.
+struct Stage {
+    double* pinned = nullptr;
+    int lanes = 0;
+    hipEvent_t filled[LANES] = {};
+
+    hipError_t ready(int want)
+    {
+        if (want <= lanes) return hipSuccess;
+        release();
+        hipError_t e = hipHostMalloc((void**)&pinned, (size_t)want * PIECE * sizeof(double), hipHostMallocDefault);
+        if (e != hipSuccess) {
+            pinned = nullptr;
+            return e;
+        }
+        lanes = want;
+        for (int i = 0; i < want; i++)
+            if ((e = hipEventCreateWithFlags(&filled[i], hipEventDisableTiming)) != hipSuccess) {
+                filled[i] = nullptr;
+                release();
+                return e;
+            }
+        return hipSuccess;
+    }
+    // the stream must be idle
+    void release()
+    {
+        for (auto& ev : filled) {
+            if (ev) (void)hipEventDestroy(ev);
+            ev = nullptr;
+        }
+        if (pinned) (void)hipHostFree(pinned);
+        pinned = nullptr;
+        lanes = 0;
+    }
+};
+
+// out[0, n): fill(first, count, pinned) queues on `stream` the work that
+// leaves out[first, first + count) in a pinned piece.  Returns false where no
+// stage could be had (nothing was queued) and true otherwise, with the first
+// error in `err`.
+template <class F>
+bool to_host(Stage& stage, hipStream_t stream, size_t n, double* out, hipError_t& err, F&& fill)
+{
+    const size_t pieces = (n + PIECE - 1) / PIECE;
+    const int cpus = (int)std::max(1u, std::thread::hardware_concurrency());
+    const int lanes = (int)std::min<size_t>(pieces, (size_t)std::min(LANES, std::max(2, cpus)));
+    err = hipSuccess;
+    int device = 0;
+    if (stage.ready(lanes) != hipSuccess || hipGetDevice(&device) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    auto carry = [&](int lane) {
+        hipError_t e = hipSetDevice(device);
+        double* const piece = stage.pinned + (size_t)lane * PIECE;
+        while (e == hipSuccess && failed.load() == (int)hipSuccess) {
+            const size_t p = next.fetch_add(1);
+            if (p >= pieces) return;
+            const size_t first = p * PIECE, count = std::min(PIECE, n - first);
+            e = fill(first, count, piece);
+            if (e == hipSuccess) e = hipEventRecord(stage.filled[lane], stream);
+            if (e == hipSuccess) e = hipEventSynchronize(stage.filled[lane]);
+            if (e == hipSuccess) std::memcpy(out + first, piece, count * sizeof(double));
+        }
+        if (e != hipSuccess) failed.store((int)e);
+    };
+    std::thread threads[LANES];
+    int started = 1;
+    for (; started < lanes; started++) {
+        try {
+            threads[started] = std::thread(carry, started);
+        } catch (const std::system_error&) {
+            break;   // the threads there are take its pieces
+        }
+    }
+    carry(0);
+    for (int i = 1; i < started; i++) threads[i].join();
+    err = (hipError_t)failed.load();
+    if (err != hipSuccess) (void)hipStreamSynchronize(stream);
+    return true;
+}
+
+}  // namespace hfhost

@@ -1464,6 +1464,19 @@ __global__ __launch_bounds__(256) void k_scan(const HfItem* __restrict__ items, 
     }
 }
 
+// n values of a block's dense [4][ty][tx] form from value x0 of row row0 on,
+// in binary64: src is the block's padded planes, dst pinned host memory (the
+// link bounds it).
+template <class R>
+__global__ __launch_bounds__(256) void k_dense(const R* __restrict__ src, int64_t plane, int pitch, uint32_t tx,
+                                               uint32_t ty, uint32_t row0, uint32_t x0, uint32_t n, double* dst)
+{
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        const uint32_t t = x0 + i, row = row0 + t / tx, x = t % tx;
+        dst[i] = (double)src[(row / ty) * plane + (int64_t)(row % ty) * pitch + x];
+    }
+}
+
 // --------------------------------------------------- conservation sums --
 // Neumaier-compensated FP64 partial sums of the four conserved variables
 // over a block's interior; one (sum, compensation) pair per workgroup and

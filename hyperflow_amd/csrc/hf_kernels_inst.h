@@ -84,6 +84,15 @@ hipError_t launch_scan<Real>(const HfItem* items, int n, const HfBlockDev* block
 }
 
 template <>
+hipError_t launch_dense<Real>(const HfBlockDev& bd, const Real* A, size_t first, uint32_t n, double* dst, hipStream_t s)
+{
+    const uint32_t grid = n > 1024 * 256 ? 1024 : (n + 255) / 256;
+    hipLaunchKernelGGL((k_dense<Real>), dim3(grid), dim3(256), 0, s, A, bd.plane, bd.pitch, (uint32_t)bd.tx,
+                       (uint32_t)bd.ty, (uint32_t)(first / bd.tx), (uint32_t)(first % bd.tx), n, dst);
+    return hipGetLastError();
+}
+
+template <>
 hipError_t launch_conserve<Real>(const HfBlockDev& bd, const Real* A, double* part, int nwg, hipStream_t s)
 {
     hipLaunchKernelGGL((k_conserve<Real>), dim3(nwg), dim3(256), 0, s, bd, A, part);

@@ -36,6 +36,10 @@ struct ClearArgs {
     int n[HF_CLEARS];
 };
 hipError_t launch_clear(const ClearArgs& a, hipStream_t s);
+// Values [first, first + n) of a block's dense [4][ty][tx] form, in binary64
+// (n <= 2^31); A: the block's planes.
+template <class R>
+hipError_t launch_dense(const HfBlockDev& bd, const R* A, size_t first, uint32_t n, double* dst, hipStream_t s);
 template <class R>
 hipError_t launch_conserve(const HfBlockDev& bd, const R* A, double* part, int nwg, hipStream_t s);
 

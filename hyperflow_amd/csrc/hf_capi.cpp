@@ -950,58 +950,65 @@ int hf_create(const hf_case_desc* desc, hf_ctx** out)
         HF_HIPC(hipMalloc(&C->buf[i], (size_t)C->total * C->esize));
         HF_HIPC(hipMemset(C->buf[i], 0, (size_t)C->total * C->esize));
     }
-    HF_HIPC(hipMalloc(&C->d_blocks, sizeof(HfBlockDev) * C->nb));
-    HF_HIPC(hipMemcpy(C->d_blocks, C->blocks.data(), sizeof(HfBlockDev) * C->nb, hipMemcpyHostToDevice));
-    HF_HIPC(hipMalloc(&C->d_probs, sizeof(HfProbDev) * C->np));
-    HF_HIPC(hipMemcpy(C->d_probs, C->probs.data(), sizeof(HfProbDev) * C->np, hipMemcpyHostToDevice));
-    HF_HIPC(hipMalloc(&C->d_items, sizeof(HfItem) * C->items.size()));
-    HF_HIPC(hipMemcpy(C->d_items, C->items.data(), sizeof(HfItem) * C->items.size(), hipMemcpyHostToDevice));
-    HF_HIPC(hipMalloc(&C->d_scan_items, sizeof(HfItem) * C->scan_items.size()));
-    HF_HIPC(hipMemcpy(C->d_scan_items, C->scan_items.data(), sizeof(HfItem) * C->scan_items.size(), hipMemcpyHostToDevice));
-    HF_HIPC(hipMalloc(&C->d_fill, sizeof(HfGhost) * fill.size()));
-    HF_HIPC(hipMemcpy(C->d_fill, fill.data(), sizeof(HfGhost) * fill.size(), hipMemcpyHostToDevice));
-    HF_HIPC(hipMalloc(&C->d_copy, sizeof(HfGhost) * copy.size()));
-    HF_HIPC(hipMemcpy(C->d_copy, copy.data(), sizeof(HfGhost) * copy.size(), hipMemcpyHostToDevice));
-    {
-        std::vector<double> cd(16 * (size_t)C->nb);
-        for (int b = 0; b < C->nb; b++)
-            for (int s = 0; s < 4; s++)
-                for (int v = 0; v < 4; v++) cd[(b * 4 + s) * 4 + v] = C->bdesc[b].state[s][v];
-        if (C->prec == HF_FP64) {
-            HF_HIPC(hipMalloc(&C->d_consts, cd.size() * 8));
-            HF_HIPC(hipMemcpy(C->d_consts, cd.data(), cd.size() * 8, hipMemcpyHostToDevice));
-        } else {
-            std::vector<float> cf(cd.begin(), cd.end());
-            HF_HIPC(hipMalloc(&C->d_consts, cf.size() * 4));
-            HF_HIPC(hipMemcpy(C->d_consts, cf.data(), cf.size() * 4, hipMemcpyHostToDevice));
+    // The tables and the zeroed working arrays in one allocation, the small
+    // ones in one copy: each of its own costs 15-20 us, which a short run of a
+    // small case notices.
+    struct Part {
+        void** p;
+        const void* data;   // null: zeros
+        size_t bytes, at;
+    };
+    std::vector<Part> parts;
+    auto put = [&](auto** p, const void* data, size_t count) {
+        parts.push_back({(void**)p, data, sizeof(**p) * count, 0});
+    };
+    put(&C->d_blocks, C->blocks.data(), C->nb);
+    put(&C->d_probs, C->probs.data(), C->np);
+    put(&C->d_items, C->items.data(), C->items.size());
+    put(&C->d_scan_items, C->scan_items.data(), C->scan_items.size());
+    put(&C->d_fill, fill.data(), fill.size());
+    put(&C->d_copy, copy.data(), copy.size());
+    std::vector<double> cd(16 * (size_t)C->nb);
+    for (int b = 0; b < C->nb; b++)
+        for (int s = 0; s < 4; s++)
+            for (int v = 0; v < 4; v++) cd[(b * 4 + s) * 4 + v] = C->bdesc[b].state[s][v];
+    const std::vector<float> cf(cd.begin(), cd.end());
+    if (C->prec == HF_FP64) put((double**)&C->d_consts, cd.data(), cd.size());
+    else put((float**)&C->d_consts, cf.data(), cf.size());
+    const std::vector<int32_t> rt = plan_table(*C);
+    put(&C->d_rounds, rt.data(), rt.size());
+    put(&C->d_imax, nullptr, 3 * C->max_words());
+    put(&C->d_gmax, nullptr, 4 * (size_t)C->nb);
+    put(&C->d_scan, nullptr, 4 * (size_t)C->nb);
+    put(&C->d_imax_fix, nullptr, 2 * C->max_words());
+    put(&C->d_fixed, nullptr, 2 * (size_t)C->nb);
+    put(&C->d_fixstats, nullptr, 4);
+    put(&C->d_skip, nullptr, C->nb);
+    put(&C->d_skip_next, nullptr, C->nb);
+    put(&C->d_sync, nullptr, HF_SLOTS * HF_SYNC_WORDS);
+    put(&C->d_pending, nullptr, C->npending);
+    put(&C->d_calls, nullptr, 2 * (size_t)C->np);
+    const size_t small = 64 << 10;
+    std::stable_partition(parts.begin(), parts.end(), [&](const Part& t) { return t.bytes <= small; });
+    size_t size = 0, nimage = 0;
+    for (Part& t : parts) {
+        t.at = size;
+        size += (t.bytes + 255) / 256 * 256;
+        if (t.bytes <= small) nimage = size;
+    }
+    std::vector<char> image(nimage, 0);
+    HF_HIPC(hipMalloc(&C->d_tables, size));
+    for (const Part& t : parts) {
+        char* const d = (char*)C->d_tables + t.at;
+        *t.p = d;
+        if (t.bytes > small) {
+            if (t.data) HF_HIPC(hipMemcpy(d, t.data, t.bytes, hipMemcpyHostToDevice));
+            else HF_HIPC(hipMemset(d, 0, t.bytes));
+        } else if (t.data && t.bytes) {
+            std::memcpy(image.data() + t.at, t.data, t.bytes);
         }
     }
-    HF_HIPC(hipMalloc(&C->d_imax, sizeof(unsigned long long) * 3 * C->max_words()));
-    HF_HIPC(hipMalloc(&C->d_gmax, sizeof(unsigned long long) * 4 * C->nb));
-    HF_HIPC(hipMalloc(&C->d_scan, sizeof(unsigned long long) * 4 * C->nb));
-    HF_HIPC(hipMemset(C->d_imax, 0, sizeof(unsigned long long) * 3 * C->max_words()));
-    HF_HIPC(hipMemset(C->d_gmax, 0, sizeof(unsigned long long) * 4 * C->nb));
-    HF_HIPC(hipMalloc(&C->d_imax_fix, sizeof(unsigned long long) * 2 * C->max_words()));
-    HF_HIPC(hipMemset(C->d_imax_fix, 0, sizeof(unsigned long long) * 2 * C->max_words()));
-    HF_HIPC(hipMalloc(&C->d_fixed, sizeof(uint32_t) * 2 * C->nb));
-    HF_HIPC(hipMalloc(&C->d_fixstats, sizeof(unsigned long long) * 4));
-    HF_HIPC(hipMemset(C->d_fixstats, 0, sizeof(unsigned long long) * 4));
-    HF_HIPC(hipMemset(C->d_fixed, 0, sizeof(uint32_t) * 2 * C->nb));
-    for (uint32_t** p : {&C->d_skip, &C->d_skip_next}) {
-        HF_HIPC(hipMalloc(p, sizeof(uint32_t) * C->nb));
-        HF_HIPC(hipMemset(*p, 0, sizeof(uint32_t) * C->nb));
-    }
-    HF_HIPC(hipMalloc(&C->d_sync, sizeof(uint32_t) * HF_SLOTS * HF_SYNC_WORDS));
-    HF_HIPC(hipMemset(C->d_sync, 0, sizeof(uint32_t) * HF_SLOTS * HF_SYNC_WORDS));
-    {
-        const std::vector<int32_t> rt = plan_table(*C);
-        HF_HIPC(hipMalloc(&C->d_rounds, sizeof(int32_t) * rt.size()));
-        HF_HIPC(hipMemcpy(C->d_rounds, rt.data(), sizeof(int32_t) * rt.size(), hipMemcpyHostToDevice));
-    }
-    HF_HIPC(hipMalloc(&C->d_pending, sizeof(uint32_t) * C->npending));
-    HF_HIPC(hipMemset(C->d_pending, 0, sizeof(uint32_t) * C->npending));
-    HF_HIPC(hipMalloc(&C->d_calls, sizeof(uint32_t) * 2 * C->np));
-    HF_HIPC(hipMemset(C->d_calls, 0, sizeof(uint32_t) * 2 * C->np));
+    HF_HIPC(hipMemcpy(C->d_tables, image.data(), nimage, hipMemcpyHostToDevice));
     HF_HIPC(hipHostMalloc((void**)&C->h_calls_pinned, sizeof(uint32_t) * C->np, hipHostMallocDefault));
     HF_HIPC(hipEventCreateWithFlags(&C->calls_copied, hipEventDisableTiming));
     HF_HIPC(hipEventRecord(C->calls_copied, C->stream));
@@ -1026,11 +1033,7 @@ void hf_destroy(hf_ctx* c)
     destroy_graphs(c);
     for (auto& e : c->ev_pending) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
     for (auto& e : c->ev_free) { (void)hipEventDestroy(e.first); (void)hipEventDestroy(e.second); }
-    for (void* p : {c->buf[0], c->buf[1], (void*)c->d_blocks, (void*)c->d_probs, (void*)c->d_items, (void*)c->d_scan_items, (void*)c->d_fill,
-                    (void*)c->d_copy, c->d_consts, (void*)c->d_imax, (void*)c->d_gmax, (void*)c->d_scan,
-                    (void*)c->d_calls, (void*)c->d_hist, (void*)c->d_part, c->d_resid, (void*)c->d_imax_fix,
-                    (void*)c->d_fixed, (void*)c->d_fixstats, (void*)c->d_sync, (void*)c->d_rounds, (void*)c->d_pending, (void*)c->d_skip,
-                    (void*)c->d_skip_next})
+    for (void* p : {c->buf[0], c->buf[1], c->d_tables, (void*)c->d_hist, (void*)c->d_part, c->d_resid})
         if (p) (void)hipFree(p);
     c->stage.release();
     if (c->h_calls_pinned) (void)hipHostFree(c->h_calls_pinned);

@@ -54,6 +54,7 @@ struct hf_ctx {
     bool ghosts_pending = false;   // buf[cur^1]'s ghosts equal buf[cur]'s (apply_bcs done)
     bool partials_valid = false;   // imax[cur] describes buf[cur], gmax[cur] is zero
 
+    void* d_tables = nullptr;      // the allocation that holds the tables and working arrays up to d_calls
     HfBlockDev* d_blocks = nullptr;
     HfProbDev* d_probs = nullptr;
     HfItem* d_items = nullptr;

@@ -82,7 +82,8 @@ __device__ __forceinline__ typename M::R sound(typename M::R gamma, typename M::
 //    the primitives (rho (q^2/2 + p/(rho (gamma-1))) equals E up to rounding);
 //  * rho u and rho v are the conserved momenta themselves in the fluxes;
 //  * the limiters with one reciprocal (the ratio and xi(r) folded into one
-//    quotient), HLLC's star state with two, the flux of the upwind side only;
+//    quotient), each difference of neighbours clamped once for the two cells
+//    that use it, HLLC's star state with two, the flux of the upwind side only;
 //  * multiply-adds written as explicit fmaf.  The build disables contraction,
 //    so no other operation is fused and every copy of this code (warm-up and
 //    loop body of a sweep) rounds the same way: results do not depend on how
@@ -92,12 +93,24 @@ namespace f32 {
 __device__ __forceinline__ float fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
-// the limiter ratio's tolerance clamp (muscl_hancock.cpp:8-11,78-94):
-// |d| <= 1e-6 becomes +-1e-6 (zero becomes +1e-6)
+// the limiter ratio's tolerance clamp (muscl_hancock.cpp:8-11,78-94): |d| is
+// raised to 1e-6 under the sign of d, +1e-6 for either zero.  Only momenta
+// (ZERO) can differ by -0.  A NaN becomes a number here: see slope().
+template <bool ZERO>
 __device__ __forceinline__ float clamp_tol(float d)
 {
-    const float tol = 1e-6f;
-    return (__builtin_fabsf(d) <= tol) ? ((d >= 0.0f) ? tol : -tol) : d;
+    return __builtin_copysignf(__builtin_fmaxf(__builtin_fabsf(d), 1e-6f), ZERO ? d + 0.0f : d);
+}
+
+// Differences b - a of two neighbouring cells, raw and clamped: they serve
+// the slopes of both cells.
+__device__ __forceinline__ void differences(const float a[4], const float b[4], float d[4], float c[4])
+{
+    for (int k = 0; k < 4; k++) d[k] = b[k] - a[k];
+    c[0] = clamp_tol<false>(d[0]);
+    c[1] = clamp_tol<true>(d[1]);
+    c[2] = clamp_tol<true>(d[2]);
+    c[3] = clamp_tol<false>(d[3]);
 }
 
 // u, v, p of a conserved state; ri = 1/rho
@@ -148,8 +161,11 @@ template <bool X>
 __device__ __forceinline__ void hllc(const State<float>& L, const State<float>& Rs, float F[4])
 {
     const float qL = X ? L.u : L.v, qR = X ? Rs.u : Rs.v;
-    const float S_L = smin(qL - L.a, qR - Rs.a);
-    const float S_R = smax(qL + L.a, qR + Rs.a);
+    // The reference's std::min / std::max drop a NaN of the right state and
+    // keep one of the left: so do these, with the left speeds in `chk`.
+    const float aL = qL - L.a, bL = qL + L.a;
+    const float S_L = __builtin_fminf(aL, qR - Rs.a);
+    const float S_R = __builtin_fmaxf(bL, qR + Rs.a);
     const float mL = L.U0 * (S_L - qL), mR = Rs.U0 * (S_R - qR);
     const float Ss = fma(mL, qL, fma(-mR, qR, Rs.p - L.p)) * rcp(mL - mR);
 
@@ -160,8 +176,8 @@ __device__ __forceinline__ void hllc(const State<float>& L, const State<float>& 
     // S_K (zero for a full flux) is min(S_L, 0) on the left, max(S_R, 0) on
     // the right.  A NaN speed gives the zero flux, as in the reference.
     const bool useR = (S_L < 0.0f) & (Ss < 0.0f);
-    const float wL = (S_L < 0.0f) ? S_L : 0.0f, wR = (S_R > 0.0f) ? S_R : 0.0f;
-    const float chk = S_L + S_R + Ss;
+    const float wL = __builtin_fminf(S_L, 0.0f), wR = __builtin_fmaxf(S_R, 0.0f);
+    const float chk = aL + bL + Ss;
     const bool none = !(chk == chk);
     const float dK = useR ? Rs.U0 : L.U0;
     const float U1K = useR ? Rs.U1 : L.U1;
@@ -202,35 +218,33 @@ __device__ __forceinline__ void hllc(const State<float>& L, const State<float>& 
 //          r >  1: xi = 2/(1+r)        -> (dl+dr) * drc / (drc + dlc)
 //  VanLeer xi = 2 min(r, 1)/(1+r)      -> (dl+dr) * m / (dlc + drc), m = dlc or drc, whichever is
 //          smaller in magnitude (both have the sign of drc)
+// r > 0 where the clamped deltas have one sign; their median with zero is then
+// the smaller of them, and zero otherwise.  The product with dl + dr is
+// positive in the first case (or dl + dr is zero) and zero or a NaN in the
+// others: s is zero there, as it is for a NaN difference in the reference.
 template <int LIM>
-__device__ __forceinline__ float slope(float um, float uc, float up)
+__device__ __forceinline__ float slope(float dl, float dr, float dlc, float drc)
 {
-    const float dl = uc - um, dr = up - uc;
-    const float dlc = clamp_tol(dl), drc = clamp_tol(dr);
-    // r > 0: the clamped deltas have one sign (they are never zero, and their
-    // product stays far above the FP32 underflow)
-    const bool same = dlc * drc > 0.0f;
-    const bool le1 = __builtin_fabsf(dlc) <= __builtin_fabsf(drc);   // |r| <= 1
-    float num, den;
+    const float m = __builtin_amdgcn_fmed3f(dlc, drc, 0.0f);
+    float num = m, den = dlc + drc;
     if (LIM == 0) {
-        num = le1 ? 0.5f * dlc : drc;
-        den = le1 ? drc : drc + dlc;
-    } else {
-        num = le1 ? dlc : drc;
-        den = dlc + drc;
+        const bool le1 = __builtin_fabsf(dlc) <= __builtin_fabsf(drc);   // |r| <= 1
+        num = le1 ? 0.5f * m : m;
+        den = le1 ? drc : den;
     }
-    const float s = (dl + dr) * num * rcp(den);
-    return same ? s : 0.0f;
+    const float t = (dl + dr) * num;
+    return t > 0.0f ? t * rcp(den) : 0.0f;
 }
 
-// One direction of MUSCL-Hancock reconstruction of a cell: face states
-// U -+ s/2 and the split half-step predictor face += h (F(lo) - F(hi)).
+// One direction of MUSCL-Hancock reconstruction of a cell from its
+// differences: face states U -+ s/2 and the split half-step predictor
+// face += h (F(lo) - F(hi)).
 template <int LIM, bool X>
-__device__ __forceinline__ void reconstruct(const float um[4], const float uc[4], const float up[4], float h, float g1,
-                                            float lo[4], float hi[4])
+__device__ __forceinline__ void reconstruct(const float uc[4], const float dl[4], const float dr[4], const float cl[4],
+                                            const float cr[4], float h, float g1, float lo[4], float hi[4])
 {
     for (int k = 0; k < 4; k++) {
-        const float s = slope<LIM>(um[k], uc[k], up[k]);
+        const float s = slope<LIM>(dl[k], dr[k], cl[k], cr[k]);
         lo[k] = fma(-0.5f, s, uc[k]);
         hi[k] = fma(0.5f, s, uc[k]);
     }
@@ -245,6 +259,15 @@ __device__ __forceinline__ void reconstruct(const float um[4], const float uc[4]
         lo[k] = fma(h, d, lo[k]);
         hi[k] = fma(h, d, hi[k]);
     }
+}
+template <int LIM, bool X>
+__device__ __forceinline__ void reconstruct(const float um[4], const float uc[4], const float up[4], float h, float g1,
+                                            float lo[4], float hi[4])
+{
+    float dl[4], dr[4], cl[4], cr[4];
+    differences(um, uc, dl, cl);
+    differences(uc, up, dr, cr);
+    reconstruct<LIM, X>(uc, dl, dr, cl, cr, h, g1, lo, hi);
 }
 
 // |u| + c and |v| + c of a state (TimeStep's per-cell terms)

@@ -95,27 +95,41 @@ __device__ __forceinline__ void output(const NetArgs& a, int x, int y, const f32
 //  * Waves 0-5: layers 2-4, two waves each, three segments per wave.  Layer k's
 //    18 weight operands stay in registers, and so does the 3-row window of its
 //    input (a ring of rows named at compile time: three LDS reads per segment
-//    and row).  Waves 6-7: layer 1 (input read from memory a row ahead) and
-//    layer 5 (window read from LDS).
+//    and row).  Waves 6-7: layer 1 (input rows requested three steps ahead and
+//    kept in LDS) and layer 5 (window read from LDS), in one piece of code.
 //  * An MFMA is 16x16x32: A = weights (rows = output channels), B = 32 input
 //    values of 16 pixels.  Lane (g = lane/16, j = lane%16) feeds pixel j and K
 //    chunk g and receives channels 16 mt + 4g + r.  For 32 input channels an
 //    MFMA is one tap; for 8, K chunk 4s + g is tap 4s + g.  Pixels outside the
 //    image are stored as zeros ("same" padding of every layer).
 // Bound by the step's chain (LDS reads, 54 MFMAs per wave with two waves per
-// SIMD, the epilogue, the barrier: about 3 900 cycles of which the MFMAs fill
+// SIMD, the epilogue, the barrier: about 3 000 cycles of which the MFMAs fill
 // 1 728), H + 12 steps.  As five launches, each layer wrote and read 64 bytes a
-// pixel (27 us of memory time per layer, 40 taken): planes at 1024^2 169 us in
-// all, now 120; corrected state 188, now 172; stored activations at 256^2 27,
-// now 26.  A barrier that waits for LDS only lets the loads and stores of a
-// step cross it (planes 128 us with __syncthreads()); a prefetch of the state a
-// step ahead spilled (250 us).
-constexpr int NET_OUT = 80, NET_SEGS = 6, NET_PX = NET_SEGS * 16 + 2;
+// pixel (27 us of memory time per layer, 40 taken).  us for planes at 1024^2,
+// corrected state at 1024^2, stored activations at 256^2:
+//   five launches                                          169   188   27
+//   one, rows as 64 bytes a pixel, __syncthreads()         128   181
+//   barrier that waits for LDS only                        120   172   26
+//   a plane per K chunk (NetRow)                           111   171   24.2
+//   layer 1's input through LDS, state requested ahead     107   142   23.4
+//   waves 6-7 first (without layer 5 a step would be a quarter shorter)
+//                                                           97   132   22.6
+// Layer 5's window in registers: 100, but 161 (spills); without the conditions
+// that leave out a strip's unused steps the third column is 30.
+constexpr int NET_OUT = 80, NET_SEGS = 6;
+// A hidden row in LDS: a plane per K chunk (8 channels, 16 bytes a pixel), its
+// 98 pixels padded to a multiple of the 256 bytes of a pass over the banks.
+// Reads (16 lanes with consecutive pixels of one plane) and writes (8 bytes)
+// then touch every bank once; with a pixel's 64 bytes together 74 % of the LDS
+// cycles were conflicts (21 % now).
+constexpr int NET_PX = 112;
+typedef uint16_t NetRow[4][NET_PX][8];
 
 template <int MODE, bool STORE>
 __global__ __launch_bounds__(512, 2) void k_net(const NetArgs a)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t buf[10][NET_PX][32];
+    __shared__ __attribute__((aligned(256))) NetRow buf[10];
+    __shared__ __attribute__((aligned(256))) uint16_t input[2][4][50][8];
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, j = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nstrip = (a.nx + NET_OUT - 1) / NET_OUT;
@@ -126,9 +140,9 @@ __global__ __launch_bounds__(512, 2) void k_net(const NetArgs a)
 
     // A 16-pixel segment of a hidden row: bias, ReLU, BF16, zeros outside the
     // image, into an LDS row and (STORE) the stored activation.
-    auto finish = [&](int k, int row, int f0, const f32x4 (&acc)[2], const float (&bias)[2][4], uint16_t (*dst)[32]) {
+    auto finish = [&](int k, int row, int f0, const f32x4 (&acc)[2], const float (&bias)[2][4], NetRow& dst) {
         const int f = f0 + j, x = X0 + f;
-        const bool in = x >= 0 && x < a.nx;
+        const bool in = x >= 0 && x < a.nx && row >= 0 && row < a.ny;
 #pragma unroll
         for (int mt = 0; mt < 2; mt++) {
             float v[4];
@@ -137,17 +151,10 @@ __global__ __launch_bounds__(512, 2) void k_net(const NetArgs a)
             uint2 pk;
             pk.x = in ? pk_bf16(v[0], v[1]) : 0u;
             pk.y = in ? pk_bf16(v[2], v[3]) : 0u;
-            *reinterpret_cast<uint2*>(&dst[f + 1][16 * mt + 4 * g]) = pk;
+            *reinterpret_cast<uint2*>(&dst[2 * mt + (g >> 1)][f + 1][4 * (g & 1)]) = pk;
             if (STORE && in && f >= 8 && f < 8 + NET_OUT && row >= yc && row < ye)
                 *reinterpret_cast<uint2*>(a.act[k - 1] + ((size_t)(row + 1) * W2 + x + 1) * 32 + 16 * mt + 4 * g) = pk;
         }
-    };
-    auto zero_row = [&](int f0, uint16_t (*dst)[32]) {
-#pragma unroll
-        for (int q = 0; q < 3; q++)
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++)
-                *reinterpret_cast<uint2*>(&dst[f0 + 16 * q + j + 1][16 * mt + 4 * g]) = make_uint2(0u, 0u);
     };
     auto load_bias = [&](int k, float (&bias)[2][4]) {
 #pragma unroll
@@ -171,34 +178,31 @@ __global__ __launch_bounds__(512, 2) void k_net(const NetArgs a)
 #pragma unroll
             for (int ph = 0; ph < 3; ph++) {
                 const int s = s0 + ph;
-                const uint16_t (*src)[32] = buf[2 * (k - 2) + ((s + 1) & 1)];   // written last step
+                const NetRow& src = buf[2 * (k - 2) + ((s + 1) & 1)];   // written last step
 #pragma unroll
                 for (int q = 0; q < 3; q++)
 #pragma unroll
-                    for (int d = 0; d < 3; d++) ring[ph][q][d] = load8(&src[f0 + 16 * q + j + d][8 * g]);
+                    for (int d = 0; d < 3; d++) ring[ph][q][d] = load8(src[g][f0 + 16 * q + j + d]);
                 const int row = yc - 4 + s - 2 * (k - 1);
                 if (row >= yc - (5 - k) && row < ye + (5 - k)) {
-                    uint16_t (*dst)[32] = buf[k < 4 ? 2 * (k - 1) + (s & 1) : 6 + (s & 3)];
-                    if (row >= 0 && row < a.ny) {
+                    NetRow& dst = buf[k < 4 ? 2 * (k - 1) + (s & 1) : 6 + (s & 3)];
 #pragma unroll
-                        for (int q = 0; q < 3; q++) {   // a segment's epilogue runs beside the next one's MFMAs
-                            f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+                    for (int q = 0; q < 3; q++) {   // a segment's epilogue runs beside the next one's MFMAs
+                        f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
-                            for (int t = 0; t < 9; t++)
+                        for (int t = 0; t < 9; t++)
 #pragma unroll
-                                for (int mt = 0; mt < 2; mt++)
-                                    acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                                        wA[mt][t], ring[(ph + 1 + t / 3) % 3][q][t % 3], acc[mt], 0, 0, 0);
-                            finish(k, row, f0 + 16 * q, acc, bias, dst);
-                        }
-                    } else {
-                        zero_row(f0, dst);
+                            for (int mt = 0; mt < 2; mt++)
+                                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    wA[mt][t], ring[(ph + 1 + t / 3) % 3][q][t % 3], acc[mt], 0, 0, 0);
+                        finish(k, row, f0 + 16 * q, acc, bias, dst);
                     }
                 }
                 lds_barrier();
             }
         }
     } else {          // layers 1 and 5
+        __builtin_amdgcn_s_setprio(2);   // the longest chain of a step: first choice beside waves 2 and 3
         const int h = wave - 6, f0 = h * 48;
         bf16x8 w1[2][3], w5[9];
 #pragma unroll
@@ -211,89 +215,93 @@ __global__ __launch_bounds__(512, 2) void k_net(const NetArgs a)
         load_bias(1, bias);
 #pragma unroll
         for (int r = 0; r < 4; r++) b5[r] = g == 0 ? a.bias[4][r] : 0.0f;
-        // layer 1's operands of a row; pixels outside the padded image (which
-        // only junk columns and rows reach) read its nearest ones
-        uint32_t xoff[3][3];   // byte offsets in a row; 32 bits reach the largest image
-        int dy[3];
-#pragma unroll
-        for (int t = 0; t < 3; t++) {
-            const int tap = min(4 * t + g, 8);
-            dy[t] = tap / 3;
-#pragma unroll
-            for (int q = 0; q < 3; q++)
-                xoff[q][t] = (uint32_t)min(max(X0 + f0 + 16 * q + j + tap % 3, 0), a.nx + 1) * 16u;
-        }
-        auto fetch = [&](int row, bf16x8 (&dst)[3][3]) {
-#pragma unroll
-            for (int t = 0; t < 3; t++) {
-                const uint32_t yoff = (uint32_t)min(max(row + dy[t], 0), a.ny + 1) * (uint32_t)W2 * 16u;
-#pragma unroll
-                for (int q = 0; q < 3; q++)
-                    dst[q][t] = load8(reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(a.x) +
-                                                                        (yoff + xoff[q][t])));
-            }
+        // Layer 1's input: each wave keeps the 50 pixels of its segments, four
+        // rows of them, in its own part of LDS; a row is requested two steps
+        // before it is put there and read.  Pixels outside the padded image
+        // (which only junk columns and rows reach) read its nearest ones.
+        uint16_t (*const img)[50][8] = input[h];
+        const uint32_t xoff = (uint32_t)min(max(X0 + f0 + min(lane, 49), 0), a.nx + 1) * 8u;
+        auto fetch = [&](int row) {
+            return load8(a.x + (size_t)min(max(row, 0), a.ny + 1) * ((size_t)W2 * 8) + xoff);
         };
+        auto keep = [&](int row, const bf16x8& v) {
+            if (lane < 50) *reinterpret_cast<bf16x8*>(img[row & 3][lane]) = v;
+        };
+        int tap[3];
+#pragma unroll
+        for (int t = 0; t < 3; t++) tap[t] = min(4 * t + g, 8);
         // the state under layer 5's output pixels (lanes g = 0)
         auto fetch_state = [&](int row, float (&u)[3][4], uint32_t (&shock)[3]) {
-            if (MODE != NET_APPLY || row < yc || row >= ye) return;
+            if (MODE != NET_APPLY) return;
+            const int y = min(max(row, yc), ye - 1);
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                const uint32_t x = (uint32_t)min(X0 + 8 + 16 * (3 * h + q) + j, a.nx - 1);
+#pragma unroll
+                for (int r = 0; r < 4; r++) u[q][r] = (a.U + r * a.plane + (int64_t)y * a.pitch)[x];
+                shock[q] = a.shock ? (a.shock + (int64_t)y * a.nx)[x] : 0u;
+            }
+        };
+        auto layer1 = [&](int row, NetRow& dst) {
+#pragma unroll
+            for (int q = 0; q < 3; q++) {
+                f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+                for (int t = 0; t < 3; t++) {
+                    const bf16x8 v = load8(img[(row + tap[t] / 3) & 3][16 * q + j + tap[t] % 3]);
+                    const bf16x8 B = (4 * t + g < 9) ? v : zero8();
+#pragma unroll
+                    for (int mt = 0; mt < 2; mt++)
+                        acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[mt][t], B, acc[mt], 0, 0, 0);
+                }
+                finish(1, row, f0 + 16 * q, acc, bias, dst);
+            }
+        };
+        auto layer5 = [&](int s, f32x4 (&acc)[3]) {
+#pragma unroll
+            for (int q = 0; q < 3; q++) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int t = 0; t < 9; t++)
+#pragma unroll
+                for (int q = 0; q < 3; q++) {   // five segments: wave 7's last repeats its second
+                    const int f = 8 + 16 * min(3 * h + q, NET_OUT / 16 - 1) + j;
+                    const bf16x8 B = load8(buf[6 + ((s + 1 + t / 3) & 3)][g][f + t % 3]);
+                    acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w5[t], B, acc[q], 0, 0, 0);
+                }
+        };
+        auto put = [&](int row, const f32x4 (&acc)[3], const float (&u)[3][4], const uint32_t (&shock)[3]) {
 #pragma unroll
             for (int q = 0; q < 3; q++) {
                 const int x = X0 + 8 + 16 * (3 * h + q) + j;
-                if (3 * h + q < NET_OUT / 16 && g == 0 && x < a.nx) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                        u[q][r] = (a.U + r * a.plane + (int64_t)row * a.pitch)[(uint32_t)x];
-                    shock[q] = a.shock ? (a.shock + (int64_t)row * a.nx)[(uint32_t)x] : 0u;
-                }
+                if (3 * h + q < NET_OUT / 16 && g == 0 && x < a.nx) output<MODE>(a, x, row, acc[q], b5, u[q], shock[q], nfb);
             }
         };
-        bf16x8 in1[3][3][3];   // rings of rows, requested a step ahead
-        fetch(yc - 4, in1[0]);
+        float us[3][3][4];
+        uint32_t sh[3][3];
+        bf16x8 ahead[3];   // rows r1 + 2 to r1 + 4 of the padded image
+#pragma unroll
+        for (int r = 0; r < 2; r++) keep(yc - 4 + r, fetch(yc - 4 + r));
+#pragma unroll
+        for (int r = 0; r < 3; r++) ahead[r] = fetch(yc - 2 + r);
+        fetch_state(yc - 12, us[0], sh[0]);
         for (int s0 = 0; s0 < steps; s0 += 3) {
 #pragma unroll
             for (int ph = 0; ph < 3; ph++) {
                 const int s = s0 + ph, r1 = yc - 4 + s, r5 = r1 - 8;
-                if (r1 + 1 < ye + 4) fetch(r1 + 1, in1[(ph + 1) % 3]);
-                float us[3][4];
-                uint32_t sh[3];
-                fetch_state(r5, us, sh);   // used at the step's end
-                if (r1 < ye + 4) {
-                    uint16_t (*dst)[32] = buf[s & 1];
-                    if (r1 >= 0 && r1 < a.ny) {
-#pragma unroll
-                        for (int q = 0; q < 3; q++) {
-                            f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
-#pragma unroll
-                            for (int t = 0; t < 3; t++) {
-                                const bf16x8 B = (4 * t + g < 9) ? in1[ph][q][t] : zero8();
-#pragma unroll
-                                for (int mt = 0; mt < 2; mt++)
-                                    acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[mt][t], B, acc[mt], 0, 0, 0);
-                            }
-                            finish(1, r1, f0 + 16 * q, acc, bias, dst);
-                        }
-                    } else {
-                        zero_row(f0, dst);
-                    }
-                }
-                if (r5 >= yc && r5 < ye) {
-                    f32x4 acc[3];
-#pragma unroll
-                    for (int q = 0; q < 3; q++) acc[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int t = 0; t < 9; t++)
-#pragma unroll
-                        for (int q = 0; q < 3; q++) {   // five segments: wave 7's last repeats its second
-                            const int f = 8 + 16 * min(3 * h + q, NET_OUT / 16 - 1) + j;
-                            const bf16x8 B = load8(&buf[6 + ((s + 1 + t / 3) & 3)][f + t % 3][8 * g]);
-                            acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w5[t], B, acc[q], 0, 0, 0);
-                        }
-#pragma unroll
-                    for (int q = 0; q < 3; q++) {
-                        const int x = X0 + 8 + 16 * (3 * h + q) + j;
-                        if (3 * h + q < NET_OUT / 16 && g == 0 && x < a.nx)
-                            output<MODE>(a, x, r5, acc[q], b5, us[q], sh[q], nfb);
-                    }
+                keep(r1 + 2, ahead[ph]);
+                ahead[ph] = fetch(r1 + 5);
+                fetch_state(r5 + 1, us[(ph + 1) % 3], sh[(ph + 1) % 3]);
+                const bool one = r1 < ye + 4, five = r5 >= yc && r5 < ye;
+                f32x4 acc[3];
+                if (one && five) {   // in one piece of code: the layers fill each other's waits
+                    layer5(s, acc);   // first: its reads cannot pass layer 1's writes
+                    layer1(r1, buf[s & 1]);
+                    put(r5, acc, us[ph], sh[ph]);
+                } else if (one) {
+                    layer1(r1, buf[s & 1]);
+                } else if (five) {
+                    layer5(s, acc);
+                    put(r5, acc, us[ph], sh[ph]);
                 }
                 lds_barrier();
             }

@@ -51,11 +51,13 @@ BYTES_PER_CELL = {"fp64": 64, "fp32": 32}   # read U^n + write U^{n+1}, 4 conser
 # the average launch duration is sampled over the whole timed region at a tenth of the timing cost
 PROFILE_EVERY = 10
 # The FP64 MUSCL-Hancock row loop of k_muscl (one row of 60 output cells per
-# wave), counted in the gfx950 assembly: MinBee 1 397 VALU instructions, Van
-# Leer 1 429, 60 of them quarter-rate (v_rcp_f64 / v_rsq_f64).  A wave64 VALU
-# instruction holds its SIMD for 4 cycles (16 for quarter rate); 1 024 SIMDs
-# at 2.4 GHz.
+# wave), counted in the gfx950 assembly.  General rows: MinBee 1 397 VALU
+# instructions, Van Leer 1 429, 60 of them quarter-rate (v_rcp_f64 /
+# v_rsq_f64); rows in range of the shortened divisions, nearly all: 970 and
+# 975, 36 quarter-rate.  A wave64 VALU instruction holds its SIMD for 4 cycles
+# (16 for quarter rate); 1 024 SIMDs at 2.4 GHz.
 VALU_ROW = {("MUSCLHancock", "MinBee", "fp64"): (1397, 60), ("MUSCLHancock", "VanLeer", "fp64"): (1429, 60)}
+VALU_ROW_IN_RANGE = {("MUSCLHancock", "MinBee", "fp64"): (970, 36), ("MUSCLHancock", "VanLeer", "fp64"): (975, 36)}
 VALU_SIMDS, VALU_GHZ, VALU_CELLS_PER_ROW = 1024, 2.4, 60
 
 
@@ -65,13 +67,17 @@ def valu_bound(scheme, limiter, precision, cells_per_s):
     key = (scheme, limiter, precision)
     if key not in VALU_ROW:
         return None
+    def limit(n, quarter):
+        cycles = (n - quarter) * 4 + quarter * 16
+        return VALU_SIMDS * VALU_GHZ * 1e9 / cycles * VALU_CELLS_PER_ROW / 1e6
+
     n, quarter = VALU_ROW[key]
-    cycles = (n - quarter) * 4 + quarter * 16
-    bound = VALU_SIMDS * VALU_GHZ * 1e9 / cycles * VALU_CELLS_PER_ROW / 1e6
+    bound, in_range = limit(n, quarter), limit(*VALU_ROW_IN_RANGE[key])
     achieved = cells_per_s / 1e6
     return {"unit": "Mcell-updates/s", "achieved": round(achieved, 1), "bound": round(bound, 1),
             "frac": round(achieved / bound, 4), "valu_per_row": n, "quarter_rate_per_row": quarter,
-            "cells_per_row": VALU_CELLS_PER_ROW}
+            "cells_per_row": VALU_CELLS_PER_ROW, "valu_per_row_in_range": VALU_ROW_IN_RANGE[key][0],
+            "bound_in_range": round(in_range, 1), "frac_in_range": round(achieved / in_range, 4)}
 
 
 def cpu_baseline(sample_n: int = 256, sample_steps: int = 5):

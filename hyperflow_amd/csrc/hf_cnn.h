@@ -49,13 +49,6 @@ struct ConvArgs {
     const uint16_t* mask;     // activation whose positive entries pass the gradient
 };
 
-struct WgradArgs {
-    const uint16_t* a;      // layer input activation, NHWC padded, CI channels
-    const uint16_t* gz;     // gradient at the layer's pre-activation, NHWC padded, CO channels
-    float* part;            // [workgroups][9*CI*CO + CO] partial sums
-    int32_t nx, ny, rows;
-};
-
 // One layer's weight-gradient partials and where their sum goes.
 struct ReduceLayer {
     const float* part;
@@ -63,9 +56,27 @@ struct ReduceLayer {
     int32_t nparts, ci, co, ci_r, co_r, first;   // first: set by launch_reduce_grad
 };
 constexpr int MAX_LAYERS = 5;
+
+// The weight gradients of all layers.
+struct WgradLayer {
+    const uint16_t* a;      // layer input activation, NHWC padded, ci channels
+    const uint16_t* gz;     // gradient at the layer's pre-activation, NHWC padded, co channels
+    float* part;            // [workgroups][9*ci*co + co] partial sums
+    int32_t ci, co;         // storage channels: (8, 32), (32, 32) or (32, 8)
+};
+struct WgradArgs {
+    WgradLayer layer[MAX_LAYERS];
+    int32_t nlayers, nx, ny;
+    int32_t rows, nwg;      // rows and workgroups per layer, set by launch_wgrad
+};
+
 struct ReduceArgs {
     ReduceLayer layer[MAX_LAYERS];
     int32_t nlayers;
+    int32_t nloss;
+    const float* lossp;     // [nloss] partial sums of the loss
+    float loss_scale;
+    float* loss;            // their sum times loss_scale
 };
 
 // Input normalisation + optional shock sensor.  U: planes of the conserved
@@ -95,13 +106,11 @@ struct LossArgs {
 // Launchers (hf_cnn.hip).  cin/cout are storage channel counts (8 or 32).
 hipError_t launch_net(NetArgs a, int mode, hipStream_t s);
 hipError_t launch_conv_bwd(int cin, const ConvArgs& a, hipStream_t s);
-hipError_t launch_wgrad(int ci, int co, const WgradArgs& a, int* nwg, hipStream_t s);
-int wgrad_rows(int nx, int ny);   // rows per workgroup, WgradArgs::rows
-int wgrad_workgroups(int nx, int ny);
+hipError_t launch_wgrad(WgradArgs a, hipStream_t s);
+int wgrad_workgroups(int nx, int ny);   // per layer
 hipError_t launch_pack(const PackArgs& a, hipStream_t s);
 hipError_t launch_loss(const LossArgs& a, int* nblocks, hipStream_t s);
 hipError_t launch_reduce_grad(ReduceArgs a, hipStream_t s);
-hipError_t launch_reduce_sum(const float* part, int n, float scale, float* out, hipStream_t s);
 hipError_t launch_adam(float* w, const float* g, float* m, float* v, int n, float lr, float b1, float b2, float eps,
                        float c1, float c2, hipStream_t s);
 // Packs the FP32 layer weights W[9][ci_r][co_r] into the A-operand order of

@@ -429,31 +429,38 @@ __global__ __launch_bounds__(256, 3) void k_conv_bwd(const ConvArgs a)
 // wave owns a fixed set of (tap, ci tile) pairs, reads each pair's B operand
 // once for all co tiles, and wave 3 also multiplies A by ones, which gives db;
 // partial sums go to part[workgroup].
-// Bound by the LDS round of a row (staging, barrier, operand reads), so a
-// small image is cut into as few rows per workgroup as fill the chip
-// (wgrad_rows).  256^2, 32 -> 32: 16 rows, a B and an A read per product and
-// db summed by 32 threads took 44.6 us, now 13.3.
+// Bound by the LDS round of a row (staging, barrier, operand reads).
 constexpr int LPX = 72;   // LDS row pitch in elements (64 pixels + 8 padding)
 
+// All layers in one launch, which needs every layer's gradient image kept: a
+// launch per layer of a small image fills the chip only with two rows per
+// workgroup, which stages as many again and leaves four times the partials.
+// 256^2, the five layers and their reduction: 64 + 13 us as five launches (44.6
+// for one 32 -> 32 layer with 16 rows, two operand reads per product and db
+// summed by threads), now 29 + 5; a training step at 1024^2 0.82 -> 0.73 ms.
+constexpr int WGRAD_FILL = 384;
+constexpr int WGRAD_LDS = (9 * 32 + 32) * LPX;
+
 template <int CI, int CO>
-__global__ __launch_bounds__(256) void k_wgrad(const WgradArgs a)
+__device__ __forceinline__ void wgrad(const WgradLayer& a, int wg, int nx, int ny, int rows, uint16_t* lds)
 {
     constexpr int CIL = CI < 16 ? 16 : CI;
     constexpr int COL = CO < 16 ? 16 : CO;
     constexpr int MT = COL / 16, NT = CIL / 16;
     constexpr int PAIRS = 9 * NT;
     constexpr int NPW = (PAIRS + 3) / 4;
-    __shared__ __attribute__((aligned(16))) uint16_t aT[3][3][CIL][LPX];
-    __shared__ __attribute__((aligned(16))) uint16_t gT[COL][LPX];
+    uint16_t (*const aT)[3][CIL][LPX] = reinterpret_cast<uint16_t (*)[3][CIL][LPX]>(lds);
+    uint16_t (*const gT)[LPX] = reinterpret_cast<uint16_t (*)[LPX]>(lds + 9 * CIL * LPX);
+    static_assert((9 * CIL + COL) * LPX <= WGRAD_LDS, "LDS of a workgroup");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, g = lane >> 4, j = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nstrip = a.nx >> 6;
-    const int x0 = (blockIdx.x % nstrip) * 64;
-    const int y0 = (blockIdx.x / nstrip) * a.rows;
-    const int y1 = min(a.ny, y0 + a.rows);
-    const int W2 = a.nx + 2;
+    const int nstrip = nx >> 6;
+    const int x0 = (wg % nstrip) * 64;
+    const int y0 = (wg / nstrip) * rows;
+    const int y1 = min(ny, y0 + rows);
+    const int W2 = nx + 2;
 
     // zero the padding channels once (never written below)
     if (CIL > CI)
@@ -530,7 +537,7 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradArgs a)
         }
     }
 
-    float* P = a.part + (size_t)blockIdx.x * (9 * CI * CO + CO);
+    float* P = a.part + (size_t)wg * (9 * CI * CO + CO);
 #pragma unroll
     for (int u = 0; u < NPW; u++) {
         const int q = wave + 4 * u;
@@ -553,6 +560,16 @@ __global__ __launch_bounds__(256) void k_wgrad(const WgradArgs a)
                 const int co = 16 * mt + 4 * g + r;
                 if (co < CO) P[9 * CI * CO + co] = db[mt][r];
             }
+}
+
+__global__ __launch_bounds__(256) void k_wgrad(const WgradArgs a)
+{
+    __shared__ __attribute__((aligned(16))) uint16_t lds[WGRAD_LDS];
+    const WgradLayer& l = a.layer[blockIdx.x / a.nwg];
+    const int wg = (int)(blockIdx.x % a.nwg);
+    if (l.ci == 8) wgrad<8, 32>(l, wg, a.nx, a.ny, a.rows, lds);
+    else if (l.co == 8) wgrad<32, 8>(l, wg, a.nx, a.ny, a.rows, lds);
+    else wgrad<32, 32>(l, wg, a.nx, a.ny, a.rows, lds);
 }
 
 // ------------------------------------------------------------------ helpers --
@@ -625,11 +642,26 @@ __global__ __launch_bounds__(256) void k_loss(const LossArgs a)
 // Sums of the weight gradients' workgroup partials, every layer in one launch:
 // a workgroup adds 64 consecutive entries of one layer, its 16 waves interleaved
 // subsets of the partials, combined in a fixed order, and writes the layer's
-// real layout W[9][ci_r][co_r] followed by b[co_r] (padding channels dropped).
-// Ten launches (two per layer) took 50 us of a 256^2 gradient, this one 13.
+// real layout W[9][ci_r][co_r] followed by b[co_r] (padding channels dropped);
+// the last workgroup sums the loss.  Bound by the partials' bytes.  Ten
+// launches (two per layer) took 50 us of a 256^2 gradient, one 13, with
+// wgrad_rows()'s longer workgroups 5 (and the loss 3.7 in a launch of its own).
 __global__ __launch_bounds__(1024) void k_reduce_grad(const ReduceArgs a)
 {
     __shared__ float red[16][64];
+    if (blockIdx.x == gridDim.x - 1) {
+        float* const sum = red[0];
+        float s = 0.0f;
+        if (threadIdx.x < 256)
+            for (int i = threadIdx.x; i < a.nloss; i += 256) s += a.lossp[i];
+        sum[threadIdx.x] = s;
+        for (int k = 128; k > 0; k >>= 1) {
+            __syncthreads();
+            if ((int)threadIdx.x < k) sum[threadIdx.x] += sum[threadIdx.x + k];
+        }
+        if (threadIdx.x == 0) a.loss[0] = sum[0] * a.loss_scale;
+        return;
+    }
     int l = 0;
     while (l + 1 < a.nlayers && (int)blockIdx.x >= a.layer[l + 1].first) l++;
     const ReduceLayer L = a.layer[l];
@@ -655,21 +687,6 @@ __global__ __launch_bounds__(1024) void k_reduce_grad(const ReduceArgs a)
         if (co < L.co_r) dst = 9 * L.ci_r * L.co_r + co;
     }
     if (dst >= 0) L.grads[dst] = v;
-}
-
-__global__ __launch_bounds__(256) void k_reduce_sum(const float* __restrict__ part, int n, float scale,
-                                                    float* __restrict__ out)
-{
-    __shared__ float red[256];
-    float s = 0.0f;
-    for (int i = threadIdx.x; i < n; i += 256) s += part[i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[0] = red[0] * scale;
 }
 
 __global__ __launch_bounds__(256) void k_adam(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
@@ -767,12 +784,14 @@ hipError_t launch_conv_bwd(int cin, const ConvArgs& a, hipStream_t s)
     return hipGetLastError();
 }
 
-// Rows per workgroup: the most, up to 16, that still make two workgroups for
-// each of the 256 CUs (at least 2 rows: every workgroup stages two more).
-int wgrad_rows(int nx, int ny)
+// Rows per workgroup: the most, up to 16, with which the layers together still
+// make WGRAD_FILL workgroups (at least 2 rows: every workgroup stages two
+// more).  256^2, sums and reduction: 384 workgroups 29 + 5 us, 768 31 + 8, 1536
+// 38 + 13; 128^2, 512^2 and 1024^2 the same with each.
+static int wgrad_rows(int nx, int ny)
 {
     int rows = 16;
-    while (rows > 2 && (nx / 64) * ((ny + rows - 1) / rows) < 512) rows /= 2;
+    while (rows > 2 && MAX_LAYERS * (int64_t)(nx / 64) * ((ny + rows - 1) / rows) < WGRAD_FILL) rows /= 2;
     return rows;
 }
 int wgrad_workgroups(int nx, int ny)
@@ -781,14 +800,15 @@ int wgrad_workgroups(int nx, int ny)
     return (nx / 64) * ((ny + rows - 1) / rows);
 }
 
-hipError_t launch_wgrad(int ci, int co, const WgradArgs& a, int* nwg, hipStream_t s)
+hipError_t launch_wgrad(WgradArgs a, hipStream_t s)
 {
-    const int n = wgrad_workgroups(a.nx, a.ny);
-    *nwg = n;
-    if (ci == 8 && co == 32) hipLaunchKernelGGL((k_wgrad<8, 32>), dim3(n), dim3(256), 0, s, a);
-    else if (ci == 32 && co == 32) hipLaunchKernelGGL((k_wgrad<32, 32>), dim3(n), dim3(256), 0, s, a);
-    else if (ci == 32 && co == 8) hipLaunchKernelGGL((k_wgrad<32, 8>), dim3(n), dim3(256), 0, s, a);
-    else return hipErrorInvalidValue;
+    for (int l = 0; l < a.nlayers; l++) {
+        const int ci = a.layer[l].ci, co = a.layer[l].co;
+        if (!((ci == 8 && co == 32) || (ci == 32 && co == 32) || (ci == 32 && co == 8))) return hipErrorInvalidValue;
+    }
+    a.rows = wgrad_rows(a.nx, a.ny);
+    a.nwg = wgrad_workgroups(a.nx, a.ny);
+    hipLaunchKernelGGL(k_wgrad, dim3((unsigned)a.nlayers * a.nwg), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -814,13 +834,7 @@ hipError_t launch_reduce_grad(ReduceArgs a, hipStream_t s)
         a.layer[l].first = blocks;
         blocks += (9 * a.layer[l].ci * a.layer[l].co + a.layer[l].co + 63) / 64;
     }
-    hipLaunchKernelGGL(k_reduce_grad, dim3(blocks), dim3(1024), 0, s, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_reduce_sum(const float* part, int n, float scale, float* out, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_reduce_sum, dim3(1), dim3(256), 0, s, part, n, scale, out);
+    hipLaunchKernelGGL(k_reduce_grad, dim3(blocks + 1), dim3(1024), 0, s, a);
     return hipGetLastError();
 }
 

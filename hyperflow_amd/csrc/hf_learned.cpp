@@ -66,7 +66,7 @@ struct hf_net {
     uint16_t* x = nullptr;
     uint16_t* act[4] = {};
     uint16_t* g8 = nullptr;
-    uint16_t* gz[2] = {};
+    uint16_t* gz[4] = {};
     bool trains = false;      // the buffers of the backward pass are there
     float* y = nullptr;
     uint8_t* shock = nullptr;
@@ -204,23 +204,6 @@ hfn::NetArgs net_args(const hf_net* n, int nx, int ny, float* outf)
     return a;
 }
 
-int wgrad(hf_net* n, int l, const uint16_t* a_in, const uint16_t* gz, int nx, int ny, hfn::ReduceArgs& red,
-          hipStream_t s)
-{
-    const Layer& L = LAYERS[l];
-    hfn::WgradArgs w;
-    w.a = a_in;
-    w.gz = gz;
-    w.part = n->part[l];
-    w.nx = nx;
-    w.ny = ny;
-    w.rows = hfn::wgrad_rows(nx, ny);
-    int nwg = 0;
-    HF_HIP(hfn::launch_wgrad(L.cis, L.cos, w, &nwg, s));
-    red.layer[red.nlayers++] = hfn::ReduceLayer{n->part[l], n->grads + L.off, nwg, L.cis, L.cos, L.ci, L.co, 0};
-    return HF_OK;
-}
-
 // Forward, loss and backward: grads and the loss (device) of one image.
 int gradients(hf_net* n, const float* u, const float* target, int nx, int ny, hipStream_t s)
 {
@@ -245,18 +228,12 @@ int gradients(hf_net* n, const float* u, const float* target, int nx, int ny, hi
     la.part = n->lossp;
     int nb = 0;
     HF_HIP(hfn::launch_loss(la, &nb, s));
-    HF_HIP(hfn::launch_reduce_sum(n->lossp, nb, inv, n->loss, s));
 
-    // layer 5: gradient at its output is g8
-    hfn::ReduceArgs red;
-    red.nlayers = 0;
-    rc = wgrad(n, 4, n->act[3], n->g8, nx, ny, red, s);
-    if (rc) return rc;
+    // gradients at the pre-activations, layer by layer (g8 is the last one's) ...
     const uint16_t* gin = n->g8;
     int cin = 8;
     for (int l = 4; l >= 1; l--) {
         // data gradient of layer l+1 (index l) into the pre-activation of layer l (index l-1)
-        uint16_t* gout = n->gz[l & 1];
         hfn::ConvArgs b;
         std::memset(&b, 0, sizeof b);
         b.in = gin;
@@ -264,15 +241,30 @@ int gradients(hf_net* n, const float* u, const float* target, int nx, int ny, hi
         b.nx = nx;
         b.ny = ny;
         b.rows = conv_rows(nx, ny);
-        b.out = gout;
+        b.out = n->gz[l - 1];
         b.mask = n->act[l - 1];
         HF_HIP(hfn::launch_conv_bwd(cin, b, s));
-        const uint16_t* a_in = (l - 1 == 0) ? n->x : n->act[l - 2];
-        rc = wgrad(n, l - 1, a_in, gout, nx, ny, red, s);
-        if (rc) return rc;
-        gin = gout;
+        gin = n->gz[l - 1];
         cin = 32;
     }
+    // ... then the weights', the layers with most work first
+    hfn::WgradArgs w;
+    hfn::ReduceArgs red;
+    w.nlayers = red.nlayers = NL;
+    w.nx = nx;
+    w.ny = ny;
+    const int nwg = hfn::wgrad_workgroups(nx, ny), order[NL] = {1, 2, 3, 4, 0};
+    for (int i = 0; i < NL; i++) {
+        const int l = order[i];
+        const Layer& L = LAYERS[l];
+        w.layer[i] = hfn::WgradLayer{l ? n->act[l - 1] : n->x, l == NL - 1 ? n->g8 : n->gz[l], n->part[l], L.cis, L.cos};
+        red.layer[i] = hfn::ReduceLayer{n->part[l], n->grads + L.off, nwg, L.cis, L.cos, L.ci, L.co, 0};
+    }
+    HF_HIP(hfn::launch_wgrad(w, s));
+    red.lossp = n->lossp;
+    red.nloss = nb;
+    red.loss_scale = inv;
+    red.loss = n->loss;
     HF_HIP(hfn::launch_reduce_grad(red, s));
     return HF_OK;
 }

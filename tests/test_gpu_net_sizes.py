@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-@pytest.mark.parametrize("ny,nx", [(1, 64), (3, 128), (17, 192), (67, 64), (128, 1024)])
+@pytest.mark.parametrize("ny,nx", [(1, 64), (3, 128), (17, 192), (67, 64), (251, 256), (128, 1024)])
 def test_gradients_at_sizes(ny, nx):
     net = native.Net(**NORM, seed=ny)
     p = net.get_params()

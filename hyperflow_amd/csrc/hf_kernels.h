@@ -1404,8 +1404,8 @@ __global__ __launch_bounds__(256) void k_ghost(const HfGhost* __restrict__ tab, 
     // block, so a workgroup issues one atomic per block it covers (device-
     // scope atomics on one address serialise: one per wave made this launch
     // take 20 us on 66 k ghost cells, one per workgroup 13 us; reading the
-    // slot first, as raise_max does, made it slower still).  A wave spanning
-    // two blocks uses per-lane atomics.
+    // slot first made it slower still).  A wave spanning two blocks uses
+    // per-lane atomics.
     __shared__ int wblk[GHOST_WAVES];
     __shared__ double wmx[GHOST_WAVES], wmy[GHOST_WAVES];
     const int w = threadIdx.x >> 6;

@@ -19,6 +19,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <new>
 #include <string>
 #include <utility>
 #include <vector>
@@ -603,11 +604,13 @@ int download_block(hf_ctx* c, int b, const void* base, int64_t off, double* out)
     HF_HIP(hipStreamSynchronize(c->stream));
     const size_t elems = (size_t)B.plane * 4;
     if (c->prec == HF_FP64) {
-        const std::unique_ptr<double[]> tmp(new double[elems]);
+        const std::unique_ptr<double[]> tmp(new (std::nothrow) double[elems]);
+        if (!tmp) return fail(HF_ENOMEM, "download: out of host memory");
         HF_HIP(hipMemcpy(tmp.get(), (const double*)base + off, elems * 8, hipMemcpyDeviceToHost));
         from_device_layout<double>(c, b, tmp.get(), out);
     } else {
-        const std::unique_ptr<float[]> tmp(new float[elems]);
+        const std::unique_ptr<float[]> tmp(new (std::nothrow) float[elems]);
+        if (!tmp) return fail(HF_ENOMEM, "download: out of host memory");
         HF_HIP(hipMemcpy(tmp.get(), (const float*)base + off, elems * 4, hipMemcpyDeviceToHost));
         from_device_layout<float>(c, b, tmp.get(), out);
     }

@@ -12,7 +12,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -98,7 +98,7 @@ bool to_host(Stage& stage, hipStream_t stream, size_t n, double* out, hipError_t
     for (; started < lanes; started++) {
         try {
             threads[started] = std::thread(carry, started);
-        } catch (const std::system_error&) {
+        } catch (const std::exception&) {
             break;   // the threads there are take its pieces
         }
     }

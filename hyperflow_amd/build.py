@@ -50,6 +50,9 @@ CLI = os.path.join(HERE, "bin", "hyperflow")
 CLIS = ((CLI, "host/hf_cli.cpp"), (os.path.join(HERE, "bin", "hyperflow_uns"), "host/hf_uns_cli.cpp"))
 # test driver of the reference-typed C++ surface (tests/cpp), linked like the CLIs
 TEST_DRIVERS = ((os.path.join(ROOT, "tests", "bin", "ref_loop"), os.path.join(ROOT, "tests", "cpp", "ref_loop.cpp")),)
+# the tests' view of a context's plan, a library of its own
+TEST_PROBE = (os.path.join(ROOT, "tests", "bin", "libcontext_probe.so"),
+              os.path.join(ROOT, "tests", "cpp", "context_probe.cpp"))
 
 
 def _compile(unit, flags, hidden, outdir):
@@ -92,6 +95,13 @@ def build(verbose: bool = False) -> str:
         if r.returncode != 0:
             raise RuntimeError(f"{src}: link failed:\n" + r.stdout)
         os.replace(exe + ".tmp", exe)
+    exe, src = TEST_PROBE
+    obj = _compile(src, ["-x", "c++", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-O2"], False, outdir)
+    r = subprocess.run([HIPCC, "-shared", "-o", exe + ".tmp", obj], stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                       text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{src}: link failed:\n" + r.stdout)
+    os.replace(exe + ".tmp", exe)
     if verbose:
         print(f"built {LIB} and {', '.join(e for e, _ in CLIS)}")
     return LIB

@@ -879,7 +879,7 @@ int build_plan(hf_ctx* c, const hf_case_desc* desc, bool dense)
             for (int ph = 0; ph < 3; ph++) n += c->segs[2 * (ph * c->nb + b) + 1];
             per = std::max(per, n);
         }
-        const int cap = c->maxnb == 1 ? 64 : 8;
+        const int cap = c->maxnb == 1 ? 64 : HF_MAX_BLOCK_SLOTS;
         c->ways = 1;
         while (c->ways < cap && c->ways * 16 < per && c->ways * 2 * c->nb <= 256) c->ways *= 2;
         c->way_stride = c->ways > 1 ? 16 : 2;

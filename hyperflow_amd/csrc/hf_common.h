@@ -101,6 +101,8 @@ struct HfStepArgs {
     uint32_t* skip_next;                 // [nblocks] the exact verdict for the next step
 };
 
+// Most slots of a block where a problem has several blocks (a power of two).
+#define HF_MAX_BLOCK_SLOTS 8
 // First word (x; y follows) of slot w of block b in a maxima array.
 #define HF_MAX_SLOT(b, w, ways, stride) (((int64_t)(b) * (ways) + (w)) * (stride))
 

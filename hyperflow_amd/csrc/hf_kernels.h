@@ -708,18 +708,26 @@ __device__ __forceinline__ void muscl_item_t(const HfStepArgs<typename M::R>& a,
 
 // The guess launch's plan of problem p (plan_scan with the main list's
 // maxima): its first block to fix, the guess minimum m and the speculative
-// minimum O.
+// minimum O; t: the terms of the first 64 blocks, for a plan_scan that follows.
+template <class R>
+__device__ __forceinline__ int guess_plan(const HfStepArgs<R>& a, int p, const HfProbDev& pr, double& O, double& m,
+                                          long long& kstep, PlanTerms& t)
+{
+    kstep = (long long)a.calls[p] - pr.cps + 1;
+    t = plan_terms<R>(a, pr, a.nblocks);
+    double o = smin(1e16, t.o);
+    const int end = pr.first + pr.nb;
+    for (int c = pr.first + 64 + (int)(threadIdx.x & 63); c < end; c += 64) o = smin(o, term_old(a, c));
+    O = wave_min(o);
+    m = 0.0;
+    return plan_scan<R, PRE_MAIN>(a, pr, a.nblocks, kstep, O, t, m, false);
+}
 template <class R>
 __device__ __forceinline__ int guess_plan(const HfStepArgs<R>& a, int p, const HfProbDev& pr, double& O, double& m,
                                           long long& kstep)
 {
-    kstep = (long long)a.calls[p] - pr.cps + 1;
-    double o = 1e16;
-    const int end = pr.first + pr.nb;
-    for (int c = pr.first + (int)(threadIdx.x & 63); c < end; c += 64) o = smin(o, term_old(a, c));
-    O = wave_min(o);
-    m = 0.0;
-    return plan_scan<R, PRE_MAIN>(a, pr, a.nblocks, kstep, O, m, false);
+    PlanTerms t;
+    return guess_plan<R>(a, p, pr, O, m, kstep, t);
 }
 
 // Check-launch rounds from round l on, while none of their blocks needs
@@ -1063,8 +1071,9 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
         if (pr.nb < 2) continue;
         double O, m;
         long long kstep;
-        guess_plan<R>(a, p, pr, O, m, kstep);
-        const int w = plan_scan<R, PRE_GUESS>(a, pr, a.nblocks, kstep, O, m, rec);
+        PlanTerms t;
+        guess_plan<R>(a, p, pr, O, m, kstep, t);
+        const int w = plan_scan<R, PRE_GUESS>(a, pr, a.nblocks, kstep, O, t, m, rec);
         first = w < first ? w : first;
     }
     if (first > a.nrounds) return;   // every block has its exact dt

@@ -759,7 +759,7 @@ __device__ __forceinline__ double dpp_f64(double x)   // the partner's x, or x w
     return __longlong_as_double(((long long)h2 << 32) | (unsigned int)l2);
 }
 template <class F>
-__device__ __forceinline__ double wave_reduce(double x, F pick)
+__device__ __forceinline__ double wave_prefix(double x, F pick)   // over lanes 0..lane
 {
     x = pick(x, dpp_f64<0x111, 0xf>(x));   // row_shr:1, 2, 4, 8
     x = pick(x, dpp_f64<0x112, 0xf>(x));
@@ -767,10 +767,19 @@ __device__ __forceinline__ double wave_reduce(double x, F pick)
     x = pick(x, dpp_f64<0x118, 0xf>(x));
     x = pick(x, dpp_f64<0x142, 0xa>(x));   // row_bcast:15 into rows 1 and 3
     x = pick(x, dpp_f64<0x143, 0xc>(x));   // row_bcast:31 into rows 2 and 3
+    return x;
+}
+__device__ __forceinline__ double lane_value(double x, int lane)   // the same for every lane
+{
     const long long b = __double_as_longlong(x);
-    const unsigned lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), 63);
-    const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+    const unsigned lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <class F>
+__device__ __forceinline__ double wave_reduce(double x, F pick)
+{
+    return lane_value(wave_prefix(x, pick), 63);
 }
 
 // Maximum / minimum over the wave (NaN-free inputs; every lane calls).
@@ -851,18 +860,28 @@ __device__ __forceinline__ double term_new(const HfStepArgs<R>& a, int c, unsign
     return smin(cdx / smax(bitsd(mx), gx), cdy / smax(bitsd(my), gy));
 }
 
-// The same from the block's slots in a maxima array
+// The same from the block's slots in a maxima array.  All slots are requested
+// at once (of fewer than HF_MAX_BLOCK_SLOTS, some twice): one round trip to the
+// caches, where a loop over the slots took one for each, and the guess and check
+// launches' plans wait for little else.  Shortest guess / check launch, us, by
+// such a loop with every plan reading its own terms and scanning through LDS,
+// and now: 8 x 97^2 channel 7.0 / 9.4, 4.4 / 5.2; 8 x 1024^2 10.1 / 10.4, 5.6 /
+// 6.4; 16 channels of 8 x 97^2 in one context 38 / 62, 27 / 40.
 template <class R>
 __device__ __forceinline__ double term_slots(const HfStepArgs<R>& a, int c, const unsigned long long* m)
 {
-    const unsigned long long* p = m + HF_MAX_SLOT(c, 0, a.ways, a.way_stride);
-    unsigned long long mx = p[0], my = p[1];
-    for (int w = 1; w < a.ways; w++) {
-        const unsigned long long x = p[(int64_t)w * a.way_stride], y = p[(int64_t)w * a.way_stride + 1];
-        mx = x > mx ? x : mx;
-        my = y > my ? y : my;
+    typedef unsigned long long pair __attribute__((ext_vector_type(2)));
+    const pair* p = (const pair*)(m + HF_MAX_SLOT(c, 0, a.ways, a.way_stride));
+    pair v = p[0];
+    if (a.ways > 1) {
+        pair s[HF_MAX_BLOCK_SLOTS];
+        for (int w = 1; w < HF_MAX_BLOCK_SLOTS; w++) s[w] = p[(w & (a.ways - 1)) * (a.way_stride / 2)];
+        for (int w = 1; w < HF_MAX_BLOCK_SLOTS; w++) {
+            v.x = s[w].x > v.x ? s[w].x : v.x;
+            v.y = s[w].y > v.y ? s[w].y : v.y;
+        }
     }
-    return term_new(a, c, mx, my);
+    return term_new(a, c, v.x, v.y);
 }
 
 template <class R>
@@ -911,21 +930,19 @@ __device__ __forceinline__ double term_pre(const HfStepArgs<R>& a, int nb_all, i
 // Inclusive minimum over lanes 0..lane (scan_lo) or lane..63 (scan_hi).
 __device__ __forceinline__ double scan_min_lo(double x)
 {
-    const int lane = threadIdx.x & 63;
-    for (int d = 1; d < 64; d <<= 1) {
-        const double o = __shfl_up(x, d, 64);
-        if (lane >= d) x = (o < x) ? o : x;
-    }
-    return x;
+    return wave_prefix(x, [](double a, double b) { return (b < a) ? b : a; });
 }
 __device__ __forceinline__ double scan_min_hi(double x)
 {
-    const int lane = threadIdx.x & 63;
-    for (int d = 1; d < 64; d <<= 1) {
-        const double o = __shfl_down(x, d, 64);
-        if (lane + d < 64) x = (o < x) ? o : x;
-    }
-    return x;
+    // within rows of 16 lanes, then the minima of the rows above (their first lanes')
+    x = smin(x, dpp_f64<0x101, 0xf>(x));   // row_shl:1, 2, 4, 8
+    x = smin(x, dpp_f64<0x102, 0xf>(x));
+    x = smin(x, dpp_f64<0x104, 0xf>(x));
+    x = smin(x, dpp_f64<0x108, 0xf>(x));
+    const double r3 = lane_value(x, 48), r2 = smin(lane_value(x, 32), r3), r1 = smin(lane_value(x, 16), r2);
+    const int row = (int)(threadIdx.x & 63) >> 4;
+    const double above = row == 0 ? r1 : row == 1 ? r2 : r3;
+    return row == 3 ? x : smin(x, above);
 }
 
 // The fix-up plan of one problem from maxima written by earlier launches
@@ -944,9 +961,26 @@ __device__ __forceinline__ double scan_min_hi(double x)
 //    the next step's skip verdicts (exact != speculative) of the blocks up to
 //    it when `record`.
 // O: the problem's speculative minimum min(1e16, min over c of old_c).
+// first64: plan_terms(), which the caller's O needs too.
+struct PlanTerms {
+    double o, n;   // old_c and pre_c by the main launch's maxima; infinite past the last block
+};
+// The terms of this lane's block of the problem's first 64.
+template <class R>
+__device__ __forceinline__ PlanTerms plan_terms(const HfStepArgs<R>& a, const HfProbDev& pr, int nb_all)
+{
+    const int lane = threadIdx.x & 63;
+    const double inf = __builtin_huge_val();
+    PlanTerms t = {inf, inf};
+    if (lane < pr.nb) {
+        t.o = term_old(a, pr.first + lane);
+        t.n = term_pre<R, PRE_MAIN>(a, nb_all, pr.first + lane);
+    }
+    return t;
+}
 template <class R, int SRC>
 __device__ int plan_scan(const HfStepArgs<R>& a, const HfProbDev& pr, int nb_all, long long kstep, double O,
-                         double& m, bool record)
+                         const PlanTerms& first64, double& m, bool record)
 {
     const int lane = threadIdx.x & 63;
     const int nb = pr.nb;
@@ -956,15 +990,22 @@ __device__ int plan_scan(const HfStepArgs<R>& a, const HfProbDev& pr, int nb_all
         const int c = c0 + lane;
         const bool in = c < nb;
         const int b = pr.first + (in ? c : 0);
-        double o = inf, n = inf;
-        if (in) {
-            o = term_old(a, b);
-            n = term_pre<R, SRC>(a, nb_all, b);
+        double o = first64.o, n = first64.n;
+        if (c0 > 0) {
+            o = n = inf;
+            if (in) {
+                o = term_old(a, b);
+                n = term_pre<R, SRC>(a, nb_all, b);
+            }
+        } else if (SRC == PRE_GUESS && in && a.fixed[b]) {
+            n = term_slots(a, b, a.imax_fix);
         }
         double tail = inf;   // minimum of old_c after this chunk
-        for (int t = c0 + 64 + lane; t < nb; t += 64) tail = smin(tail, term_old(a, pr.first + t));
-        tail = wave_min(tail);
-        double pre = __shfl_up(scan_min_lo(n), 1, 64);
+        if (c0 + 64 < nb) {
+            for (int t = c0 + 64 + lane; t < nb; t += 64) tail = smin(tail, term_old(a, pr.first + t));
+            tail = wave_min(tail);
+        }
+        double pre = dpp_f64<0x138, 0xf>(scan_min_lo(n));   // wave_shr:1
         pre = (lane == 0 || pre > carry) ? carry : pre;
         double suf = scan_min_hi(o);
         suf = (tail < suf) ? tail : suf;
@@ -987,7 +1028,7 @@ __device__ int plan_scan(const HfStepArgs<R>& a, const HfProbDev& pr, int nb_all
             if (SRC != PRE_GUESS) m = __shfl(e, first, 64);
             return c0 + first;
         }
-        carry = smin(carry, wave_min(n));
+        if (c0 + 64 < nb) carry = smin(carry, wave_min(n));
     }
     return nb;
 }

@@ -454,7 +454,6 @@ int ensure_partials(hf_ctx* c)
     hf::ClearArgs z;
     std::memset(&z, 0, sizeof z);
     auto clear = [&, k = 0](void* p, size_t words) mutable { z.p[k] = (uint32_t*)p; z.n[k++] = (int)words; };
-    c->turn = 0;
     if (c->mirrored) clear(c->imax(0), 6 * c->max_words());   // and no ghost maxima: they repeat interior cells'
     else clear(c->imax(c->cur), 2 * c->max_words());
     clear(c->gmax(c->cur), 4 * (size_t)c->nb);
@@ -473,10 +472,13 @@ int ensure_partials(hf_ctx* c)
 // bound by their launches, and a fill of narrow columns moves a cache line
 // per cell.  Per step with a fill each / without: 100 x 5 Godunov 11.0 / 6.6
 // us, 400^2 16.3 / 11.9, 50^2 MUSCL 15.2 / 11.3, FP32 1024^2 28.9 / 25.4, 512
-// blocks FP32 801 / 712.
+// blocks FP32 801 / 712.  The maxima buffers of the steps take turns; the fill
+// leaves the last state's in buffer 0, so that every run starts there and a
+// captured one serves all runs of its length.
 int enqueue_mirrored(hf_ctx* c, int nsteps, bool timed, bool fixed, double dt)
 {
-    const int c0 = c->cur, t0 = c->turn;
+    const int c0 = c->cur;
+    c->turn = 0;
     const bool timing = timed;
     for (int s = 0; s < nsteps; s++) {
         timed = timing && (c->prof_step++ % c->profile == 0);
@@ -495,10 +497,15 @@ int enqueue_mirrored(hf_ctx* c, int nsteps, bool timed, bool fixed, double dt)
         c->cur ^= 1;
         if (!fixed) c->turn = (c->turn + 1) % 3;
     }
-    const int rc = launch_ghost(c, c->d_fill, c->nfill, c->buf[c->cur ^ 1], c->buf[c->cur], c->d_scan + 2 * c->nb,
-                                no_book());
+    GhostBook bk = no_book();
+    if (c->turn != 0) {
+        bk.turns = c->imax(0);
+        bk.nturn = (int)c->max_words();
+        bk.turn = c->turn;
+    }
+    const int rc = launch_ghost(c, c->d_fill, c->nfill, c->buf[c->cur ^ 1], c->buf[c->cur], c->d_scan + 2 * c->nb, bk);
     c->cur = c0;
-    c->turn = t0;
+    c->turn = 0;
     return rc;
 }
 
@@ -515,7 +522,7 @@ int enqueue_steps(hf_ctx* c, int nsteps, bool timed, bool fixed = false, double 
         const int k = c->cur;
         void* A = c->buf[k];
         void* B = c->buf[k ^ 1];
-        GhostBook bk;
+        GhostBook bk = no_book();
         bk.calls = c->d_calls;
         bk.probs = c->d_probs;
         bk.nprob = c->np;
@@ -1171,7 +1178,7 @@ static int run_loop(hf_ctx* c, int nsteps, int flags, bool fixed, double dt)
     if (flags & HF_RUN_GRAPH) {
         uint64_t dtbits = 0;
         if (fixed) std::memcpy(&dtbits, &dt, sizeof dtbits);
-        const auto key = std::make_tuple(nsteps, c->cur, dtbits, c->turn);
+        const auto key = std::make_tuple(nsteps, c->cur, dtbits);
         auto it = c->graphs.find(key);
         if (it == c->graphs.end()) {
             hipGraph_t g = nullptr;
@@ -1193,7 +1200,6 @@ static int run_loop(hf_ctx* c, int nsteps, int flags, bool fixed, double dt)
         if (rc) return rc;
     }
     c->cur ^= (nsteps & 1);
-    if (c->mirrored && !fixed) c->turn = (c->turn + nsteps) % 3;
     if (!fixed)
         for (int p = 0; p < c->np; p++) c->calls[p] += (int64_t)nsteps * c->probs[p].cps;
     else

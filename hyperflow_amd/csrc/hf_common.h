@@ -132,6 +132,10 @@ struct GhostBook {
     uint32_t* pending;            // pending bitmap of this step's check launch
     int32_t npending;             // words
     int32_t nblocks;
+    // after a mirrored run: the maxima of buffer `turn` of the three (of nturn
+    // words each) move to buffer 0, the others are cleared
+    unsigned long long* turns;
+    int32_t nturn, turn;
     // fold the previous step's fix-ups into its maxima (the check launch's
     // over the guess launch's), then clear them
     unsigned long long* imax_prev;   // maxima of the state this step starts from

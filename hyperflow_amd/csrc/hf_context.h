@@ -88,8 +88,8 @@ struct hf_ctx {
     std::vector<int64_t> calls;     // host mirror of the TimeStep call counters
     hipStream_t stream = nullptr;
     hfhost::Stage stage;             // pinned pieces of large downloads
-    // captured step loops by (steps, start parity, fixed-dt bits or 0 for the CFL dt, turn)
-    std::map<std::tuple<int, int, uint64_t, int>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
+    // captured step loops by (steps, start parity, fixed-dt bits or 0 for the CFL dt)
+    std::map<std::tuple<int, int, uint64_t>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
 
     int profile = 0;                 // 0 off, else time the launches of every profile-th step
     int64_t prof_step = 0;
@@ -100,7 +100,8 @@ struct hf_ctx {
     size_t max_words() const { return (size_t)nb * ways * way_stride; }   // a maxima array
     // Mirrored steps (HfStepArgs::mirrored): three maxima buffers take turns as
     // the read, the written and the cleared one, the maxima of buf[cur] in
-    // imax(turn); ghost layers are filled once, after the last step of a run.
+    // imax(turn), which is imax(0) between runs; ghost layers are filled once,
+    // after the last step of a run.
     bool mirrored = false;
     int turn = 0;
     int now() const { return mirrored ? turn : cur; }   // which imax describes buf[cur]

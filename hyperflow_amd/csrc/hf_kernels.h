@@ -1354,6 +1354,12 @@ __global__ __launch_bounds__(256) void k_ghost(const HfGhost* __restrict__ tab, 
             book.calls[p] += (uint32_t)book.probs[p].cps;
         for (int i = threadIdx.x; i < book.nclear0; i += blockDim.x) book.clear0[i] = 0ull;
         for (int i = threadIdx.x; i < book.nclear1; i += blockDim.x) book.clear1[i] = 0ull;
+        for (int i = threadIdx.x; i < book.nturn; i += blockDim.x) {
+            unsigned long long* const t = book.turns + i;
+            t[0] = t[(int64_t)book.turn * book.nturn];
+            t[book.nturn] = 0ull;
+            t[2 * (int64_t)book.nturn] = 0ull;
+        }
         for (int i = threadIdx.x; i < book.nqueue; i += blockDim.x) book.queue[i] = 0u;
         for (int i = threadIdx.x; i < book.npending; i += blockDim.x) book.pending[i] = 0u;
         const int nb = book.nblocks, bw = book.block_words;

@@ -288,6 +288,7 @@ __device__ __forceinline__ int muscl_rows_q64(const HfStepArgs<double>& a, const
         bad = q64::out_of_range(um, lim) | q64::out_of_range(uc, lim);
         bc = q64::out_of_range(up, lim);
         bp = q64::out_of_range(un, lim);
+        if ((bad | bc | bp) & m0) return 0;   // before arithmetic that would be done twice
         q64::differences(um, uc, dl, cl, lim);
         q64::differences(uc, up, dr, cr, lim);
         q64::reconstruct<LIM, false>(uc, dl, dr, cl, cr, hy, g1, ig1, lo, hi, bad, lim);     // cell y0-1
@@ -540,6 +541,7 @@ __device__ __forceinline__ int muscl_cols_q64(const HfStepArgs<double>& a, const
         bad = q64::out_of_range(um, lim) | q64::out_of_range(uc, lim);
         bc = q64::out_of_range(up, lim);
         bp = q64::out_of_range(un, lim);
+        if ((bad | bc | bp) & m0) return 0;   // before arithmetic that would be done twice
         q64::differences(um, uc, dl, cl, lim);
         q64::differences(uc, up, dr, cr, lim);
         q64::reconstruct<LIM, true>(uc, dl, dr, cl, cr, hx, g1, ig1, lo, hi, bad, lim);      // column x0-1
@@ -1180,8 +1182,11 @@ __device__ __forceinline__ int godunov_rows_q64(const HfStepArgs<double>& a, con
     const double ig1 = 1.0 / g1, rdx = 1.0 / bd.dx, rdy = 1.0 / bd.dy;
     const q64::Limits lim;
     q64::mask bad = q64::out_of_range(ub, lim), bc = q64::out_of_range(uc, lim);
-    q64::State sc = q64::make_state(uc, gam, g1, ig1, bc, lim);
-    {
+    q64::State sc;
+    if ((bad | bc) & m0) {   // before arithmetic that would be done twice
+        bad = m0;
+    } else {
+        sc = q64::make_state(uc, gam, g1, ig1, bc, lim);
         const q64::State sb = q64::make_state(ub, gam, g1, ig1, bad, lim);
         q64::hllc<false>(sb, sc, Gs, bad, lim);         // face y0-1/2
     }

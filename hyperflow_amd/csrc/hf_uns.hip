@@ -133,8 +133,8 @@ struct Face<true> {
 // one cell: its new state and its term of the next dt.  Returns the lanes out
 // of range (QUICK).
 template <bool QUICK>
-__device__ __forceinline__ hf::q64::mask advance_cell(const UnsMesh& m, const UnsStep& s, int c, double dt, double N[4],
-                                                      double& term)
+__device__ __forceinline__ hf::q64::mask advance_cell(const UnsMesh& m, const UnsStep& s, int c, const double U[4],
+                                                      double dt, double N[4], double& term)
 {
     typedef Face<QUICK> Fc;
     const int n = m.n;
@@ -142,9 +142,6 @@ __device__ __forceinline__ hf::q64::mask advance_cell(const UnsMesh& m, const Un
     const double ig1 = QUICK ? 1.0 / g1 : 0.0;
     const hf::q64::Limits lim;
     hf::q64::mask bad = 0;
-    double U[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) U[k] = s.A[(size_t)k * n + c];
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
     double shortest = 1e16;
 #pragma unroll 1   // see k_uns_step
@@ -234,10 +231,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     }
     unsigned long long cand = ~0ull;
     if (c < n) {
-        double N[4], term;
-        hf::q64::mask bad = ~0ull;
-        if (hf::q64::constants_in_range(m.gamma, m.gamma - 1.0)) bad = advance_cell<true>(m, s, c, dt, N, term);
-        if (bad) advance_cell<false>(m, s, c, dt, N, term);
+        double U[4], N[4], term;
+#pragma unroll
+        for (int k = 0; k < 4; k++) U[k] = s.A[(size_t)k * n + c];
+        // density and energy, which the rotations leave alone, before arithmetic
+        // that would be done twice
+        const hf::q64::Limits lim;
+        hf::q64::mask bad = __ballot(!(U[0] >= lim.low)) | __ballot(!(U[0] <= lim.high)) |
+                            __ballot(!(U[3] >= lim.low)) | __ballot(!(U[3] <= lim.high));
+        if (!bad && hf::q64::constants_in_range(m.gamma, m.gamma - 1.0))
+            bad = advance_cell<true>(m, s, c, U, dt, N, term);
+        else
+            bad = 1;
+        if (bad) advance_cell<false>(m, s, c, U, dt, N, term);
 #pragma unroll
         for (int k = 0; k < 4; k++) s.B[(size_t)k * n + c] = N[k];
         cand = bits_of(term);

@@ -216,7 +216,7 @@ __global__ __launch_bounds__(512, 2) void k_net(const NetArgs a)
 #pragma unroll
         for (int r = 0; r < 4; r++) b5[r] = g == 0 ? a.bias[4][r] : 0.0f;
         // Layer 1's input: each wave keeps the 50 pixels of its segments, four
-        // rows of them, in its own part of LDS; a row is requested two steps
+        // rows of them, in its own part of LDS; a row is requested three steps
         // before it is put there and read.  Pixels outside the padded image
         // (which only junk columns and rows reach) read its nearest ones.
         uint16_t (*const img)[50][8] = input[h];

@@ -492,8 +492,8 @@ __device__ __forceinline__ void reconstruct(const typename M::R um[4], const typ
 // 26.0.
 //
 // In assembly, one row of k_muscl (60 cells) went from 1 397 (MinBee) and
-// 1 429 (Van Leer) to 1 013 and 1 022 VALU instructions, 60 of them
-// quarter-rate to 36.  8192^2 Van Leer: 3.13 -> 2.41 ms per step, the 8 x
+// 1 429 (Van Leer) to 970 and 975 VALU instructions, 60 of them quarter-rate
+// to 36 (general rows now 1 371 and 1 401).  8192^2 Van Leer: 3.13 -> 2.41 ms per step, the 8 x
 // 1024^2 channel 0.440 -> 0.379, Godunov 400^2 0.0258 -> 0.0248.
 namespace q64 {
 

@@ -39,7 +39,7 @@ import numpy as np
 from . import native
 
 CACHE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "tuning.json")
-ROWS = (8, 16, 24, 32, 40, 42, 44, 48, 56, 64)
+ROWS = (48, 8, 16, 24, 32, 40, 42, 44, 56, 64)   # the library's default first
 TAILS = (4, 6, 8, 12, 16)
 FIXES = (0, 4, 6, 9, 12, 16)   # 0: sized by the library to one round of the resident waves
 PARAMS = ("tile_rows", "tail_rows", "fix_rows")
@@ -145,11 +145,11 @@ def tune(cases, fields: Sequence[np.ndarray], precision: str = "fp64", dt_mode: 
     for compat MUSCL problems of several blocks), each candidate timed
     `repeats` times on `steps` steps (HIP-graph captured, or eager launches as
     the workload's benchmark runs them) from the given fields.  The search
-    starts from the class's cached plan (else the library default), and a
-    candidate takes its place only if it is faster by more than the runs of
-    either differ: other sizes of the class get the plan too, and where a
-    launch is one round whatever the plan (1024^2 in FP32), the fastest of ten
-    equal candidates was 8 rows, which costs 1536^2 0.090 ms for 0.052.  Returns the
+    starts from the class's cached plan (else the first rows), and a candidate
+    takes its place only if it is faster by more than the runs of either differ:
+    other sizes of the class get the plan too, and where a launch is one round
+    whatever the plan (1024^2 in FP32), the fastest of ten equal candidates was
+    8 rows, which costs 1536^2 0.090 ms for 0.052.  Returns the
     chosen plan with its median time and spread, every candidate's times and
     the candidates rejected for differing results."""
     cases = _cases(cases)
@@ -182,7 +182,7 @@ def tune(cases, fields: Sequence[np.ndarray], precision: str = "fp64", dt_mode: 
 
     cls = problem_class(cases, precision, dt_mode)
     entry = load_cache().get(class_key(cls))
-    best = {p: int(entry[p]) for p in PARAMS} if entry else dict(default)
+    best = {p: int(entry[p]) for p in PARAMS} if entry else dict(default, tile_rows=rows[0])
     best_t = measure(best)
     for p, cands in (("tile_rows", rows), ("tail_rows", tails), ("fix_rows", fixes)):
         if p == "fix_rows" and not (dt_mode == "compat" and cases[0].scheme == "MUSCLHancock"

@@ -77,7 +77,8 @@ def valu_bound(scheme, limiter, precision, cells_per_s):
     return {"unit": "Mcell-updates/s", "achieved": round(achieved, 1), "bound": round(bound, 1),
             "frac": round(achieved / bound, 4), "valu_per_row": n, "quarter_rate_per_row": quarter,
             "cells_per_row": VALU_CELLS_PER_ROW, "valu_per_row_in_range": VALU_ROW_IN_RANGE[key][0],
-            "bound_in_range": round(in_range, 1), "frac_in_range": round(achieved / in_range, 4)}
+            "quarter_rate_per_row_in_range": VALU_ROW_IN_RANGE[key][1], "bound_in_range": round(in_range, 1),
+            "frac_in_range": round(achieved / in_range, 4)}
 
 
 def valu_line(v):
@@ -85,7 +86,8 @@ def valu_line(v):
     nearly every item runs, the general rows' bound apart (the kernel passes it
     where all rows are in range)."""
     return {"unit": v["unit"], "achieved": v["achieved"], "bound": v["bound_in_range"], "frac": v["frac_in_range"],
-            "valu_per_row": v["valu_per_row_in_range"], "cells_per_row": v["cells_per_row"],
+            "valu_per_row": v["valu_per_row_in_range"],
+            "quarter_rate_per_row": v["quarter_rate_per_row_in_range"], "cells_per_row": v["cells_per_row"],
             "general_rows": {k: v[k] for k in ("bound", "valu_per_row", "quarter_rate_per_row")}}
 
 

@@ -732,24 +732,45 @@ __device__ __forceinline__ int guess_plan(const HfStepArgs<R>& a, int p, const H
     return guess_plan<R>(a, p, pr, O, m, kstep, t);
 }
 
+// What a wave of the check launch knows of a block (verdict_on), and of its
+// problem: the guess minimum, which the launch does not change.  A wave that
+// goes through the rounds takes them from here instead of planning again for
+// every round and item: the check launch of a step that recomputes blocks of the
+// 8 x 97^2 channel took 185 us with that, 160 without.
+struct Verdict {
+    int block = -1, problem = -1;
+    bool need = false;
+    double mg = 0.0, step = 0.0, pred = 0.0;
+    long long kstep = 0, kpred = 0;
+};
+template <class R>
+__device__ __forceinline__ void verdict_on(const HfStepArgs<R>& a, int p, const HfProbDev& pr, int lb, Verdict& v)
+{
+    if (p != v.problem) {
+        double O;
+        guess_plan<R>(a, p, pr, O, v.mg, v.kstep);
+        v.problem = p;
+    }
+    v.block = pr.first + lb;
+    v.need = check_verdict<R>(a, p, pr, a.nblocks, lb, v.mg, v.step, v.pred, v.kstep, v.kpred);
+}
+
 // Check-launch rounds from round l on, while none of their blocks needs
 // computing: round l holds the l-th block of every problem with more than l
 // blocks, and its verdicts need the blocks before it final, which holds while
 // every earlier round has been completed.  The queue counter jumps past each
 // round passed over (its unissued items are counted complete).  Returns the
-// first round to compute, or nrounds + 1.
+// first round to compute, or nrounds + 1; v keeps the last verdict.
 template <class R>
-__device__ int first_busy_round(const HfStepArgs<R>& a, int l, int lane, unsigned base)
+__device__ int first_busy_round(const HfStepArgs<R>& a, int l, int lane, unsigned base, Verdict& v)
 {
     for (; l <= a.nrounds; l++) {
         bool need = false;
         for (int p = 0; p < a.nprob; p++) {
             const HfProbDev pr = a.probs[p];
             if (pr.nb <= l) continue;
-            double O, mg, st, pd;
-            long long ks, kp;
-            guess_plan<R>(a, p, pr, O, mg, ks);
-            need = check_verdict<R>(a, p, pr, a.nblocks, l, mg, st, pd, ks, kp) || need;
+            verdict_on<R>(a, p, pr, l, v);
+            need = v.need || need;
         }
         if (need) return l;
         const unsigned end = (unsigned)a.rounds[l + 1] - base;
@@ -1068,25 +1089,30 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
     // the first round with a wrong block; wave 0 records the skip verdicts
     int first = a.nrounds + 1;
     const bool rec = wave_id() == 0;
+    Verdict v;
     for (int p = 0; p < a.nprob; p++) {
         const HfProbDev pr = a.probs[p];
         if (pr.nb < 2) continue;
-        double O, m;
-        long long kstep;
+        double O;
         PlanTerms t;
-        guess_plan<R>(a, p, pr, O, m, kstep, t);
-        const int w = plan_scan<R, PRE_GUESS>(a, pr, a.nblocks, kstep, O, t, m, rec);
+        v.problem = p;
+        guess_plan<R>(a, p, pr, O, v.mg, v.kstep, t);
+        const int w = plan_scan<R, PRE_GUESS>(a, pr, a.nblocks, v.kstep, O, t, v.mg, rec);
         first = w < first ? w : first;
     }
     if (first > a.nrounds) return;   // every block has its exact dt
 
+    // one round computes at a time: more waves than the largest has items would
+    // only draw tickets and poll (8 x 97^2 channel, 194 items a round: 160 us a
+    // launch with all 2 048, now 80)
+    unsigned waves = 0u;
+    for (int l = first; l <= a.nrounds; l++) waves = max(waves, (unsigned)(a.rounds[l + 1] - a.rounds[l]));
+    waves = min(waves, total_waves());
+    if (wave_id() >= waves) return;
+
     const MaxOut imax_chk = {a.imax_fix + HF_MAX_SLOT(a.nblocks, 0, a.ways, a.way_stride), 0};
     uint32_t* fixed_chk = a.fixed + a.nblocks;
     const unsigned base = (unsigned)a.rounds[first];   // item of queue counter value 0
-    int cached = -1, cp = -1;   // the block whose verdict this wave holds, the problem of its guess minimum
-    bool c_need = false;
-    double cm = 0.0, c_step = 0.0, c_pred = 0.0;
-    long long c_kstep = 0, c_kpred = 0;
     int r_from = -1, r_busy = 0;   // first_busy_round(r_from) as this wave last computed it
     for (unsigned idx = next_ticket(a.sync, lane, base);; idx = next_ticket(a.sync, lane, base)) {
         if (idx >= (unsigned)a.nitems) break;
@@ -1099,29 +1125,22 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
                 continue;   // left to the last wave, not counted complete
             }
             r_from = l;
-            r_busy = first_busy_round<R>(a, l, lane, base);
+            r_busy = first_busy_round<R>(a, l, lane, base, v);
         }
         if (r_busy == l) {
             const HfBlockDev bd = a.blocks[it.block];
-            if (it.block != cached) {
-                cached = it.block;
+            if (it.block != v.block) {
                 const HfProbDev pr = a.probs[bd.problem];
-                if (bd.problem != cp) {
-                    cp = bd.problem;
-                    double O;
-                    long long ks;
-                    guess_plan<R>(a, cp, pr, O, cm, ks);
-                }
-                c_need = check_verdict<R>(a, bd.problem, pr, a.nblocks, bd.lb, cm, c_step, c_pred, c_kstep, c_kpred);
+                verdict_on<R>(a, bd.problem, pr, bd.lb, v);
             }
-            if (c_need) {
+            if (v.need) {
                 // Or, not an exchange: the compiler leaves one lane's of an or
                 // with one value for the wave, and 64 of an exchange, which
                 // took 1.3 ms of the 1.5 ms a recomputed 1024^2 block cost
                 // (the channel's first 200 steps: 2.9 -> 0.83 ms per step).
                 atomicOr(&fixed_chk[it.block], 1u);
-                record_dts<R>(a, it, bd, false, c_step, c_pred, c_kstep, c_kpred);
-                auto dts = [&](double& step, double& pred) { step = c_step; pred = c_pred; };
+                record_dts<R>(a, it, bd, false, v.step, v.pred, v.kstep, v.kpred);
+                auto dts = [&](double& step, double& pred) { step = v.step; pred = v.pred; };
                 muscl_go<M, LIM, false>(a, it, lane, dts, imax_chk);
             }
         }
@@ -1132,7 +1151,7 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
     // those items was written by another wave.
     __builtin_amdgcn_s_waitcnt(0xF70);   // this wave's atomics are performed before it counts as gone
     const unsigned left = __builtin_amdgcn_readfirstlane(atomicAdd(&a.sync[HF_SYNC_EXITED], lane == 0 ? 1u : 0u));
-    if (left != total_waves() - 1) return;
+    if (left != waves - 1) return;
     if (!(__builtin_amdgcn_readfirstlane(coherent_read(&a.sync[HF_SYNC_DONE])) & HF_SYNC_ABORT_BIT)) return;
     const unsigned nfix = (unsigned)(a.nitems - a.nmain);
     for (unsigned w = 0; w * 32 < nfix; w++) {
@@ -1143,13 +1162,11 @@ __global__ __launch_bounds__(256, 2) void k_muscl_check(const HfStepArgs<typenam
             const HfItem it = a.items[a.item0 + idx];
             const HfBlockDev bd = a.blocks[it.block];
             const HfProbDev pr = a.probs[bd.problem];
-            double O, mg, dt_step, dt_pred;
-            long long kstep, kpred;
-            guess_plan<R>(a, bd.problem, pr, O, mg, kstep);
-            if (check_verdict<R>(a, bd.problem, pr, a.nblocks, bd.lb, mg, dt_step, dt_pred, kstep, kpred)) {
+            verdict_on<R>(a, bd.problem, pr, bd.lb, v);
+            if (v.need) {
                 atomicOr(&fixed_chk[it.block], 1u);
-                record_dts<R>(a, it, bd, false, dt_step, dt_pred, kstep, kpred);
-                auto dts = [&](double& step, double& pred) { step = dt_step; pred = dt_pred; };
+                record_dts<R>(a, it, bd, false, v.step, v.pred, v.kstep, v.kpred);
+                auto dts = [&](double& step, double& pred) { step = v.step; pred = v.pred; };
                 muscl_go<M, LIM, false, false>(a, it, lane, dts, imax_chk);   // rare: the general rows only
                 __builtin_amdgcn_s_waitcnt(0xF70);   // its maxima are performed before the next verdict reads them
             }

@@ -1,7 +1,7 @@
 """Plans of the guess and check launches over blocks whose wave-speed maxima
 lie in one to eight slots, in problems of more than 64 blocks and in several
 problems of one context: bit for bit the CPU oracle's fields and TimeStep
-results."""
+results, also where the check launch computes."""
 import numpy as np
 import pytest
 
@@ -22,14 +22,16 @@ def row_of_blocks(count, nx, ny, limiter):
     return base
 
 
-def check(cases, ways, steps):
+def check(cases, ways, steps, computed=None):
+    """computed: tallies of fixup_stats() that must have counted blocks."""
     data = [(c, C.perturbed_fields(C.Case(**{**c.__dict__, "initial_condition": C.quad_case(8, 8, 2).initial_condition}), 2))
             for c in cases]
     ref = [G.oracle_run(c, f, steps) for c, f in data]
     s, out, hist = G.gpu_run(cases, [U for _, f in data for U in f], steps)
-    got = context_probe.ways(s)
+    got, fixups = context_probe.ways(s), s.fixup_stats()
     s.close()
-    assert got == ways
+    assert ways is None or got == ways
+    assert all(fixups[k] > 0 for k in computed or ()), fixups
     assert np.array_equal(hist, ref[0][1])
     for a, b in zip(out, [U for r in ref for U in r[0]]):
         assert np.array_equal(a, b)
@@ -47,3 +49,13 @@ def test_more_than_64_blocks():
 
 def test_several_problems():
     check([C.step_channel(97, "MinBee", 0.5), row_of_blocks(3, 33, 20, "MinBee"), C.step_channel(17, "MinBee", 0.5)], 8, 13)
+
+
+@pytest.mark.parametrize("sizes", [(20, 170, 70), (33, 20, 9), (61, 97, 5), (128, 64, 12)])
+@pytest.mark.parametrize("count", [1, 3])
+def test_check_launch_that_computes(sizes, count):
+    """Rows of blocks in which the check launch recomputes blocks, round after
+    round, with fewer waves than are resident (one per item of a round)."""
+    nx, ny, blocks = sizes
+    cases = [row_of_blocks(blocks, nx, ny, "VanLeer")] + [row_of_blocks(3 + k, 33, 20, "VanLeer") for k in range(count - 1)]
+    check(cases, None, 40, ("check",))

@@ -488,8 +488,8 @@ __device__ __forceinline__ void reconstruct(const typename M::R um[4], const typ
 // states (units far from 1) then cost a second request of those rows, us per
 // step by the general code alone / found after the first face / found at once:
 // Van Leer 50^2 11.8 / 14.2 / 12.9, 300^2 17.1 / 19.5 / 18.2, 2048^2 215 / 218 /
-// 215, Godunov 400^2 12.1 / 13.4 / 13.0, unstructured 367 500 cells 25.9 / 38.7 /
-// 26.0.
+// 215, Godunov 400^2 12.1 / 13.4 / 13.0, unstructured 367 500 cells 25.9 / 38.6 /
+// 25.0.
 //
 // In assembly, one row of k_muscl (60 cells) went from 1 397 (MinBee) and
 // 1 429 (Van Leer) to 970 and 975 VALU instructions, 60 of them quarter-rate

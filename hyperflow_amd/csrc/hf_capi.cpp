@@ -5,7 +5,9 @@
 // buf[cur^1] from buf[cur] (table-driven gather, the reference's side order
 // replayed on the host), then the update kernels read the interior from
 // buf[cur] and the ghosts from buf[cur^1] and write the new interior into
-// buf[cur^1]; cur flips.  The dt of every step stays on the device: the
+// buf[cur^1]; cur flips.  (Runs of single blocks between transmissive and
+// reflective sides read ghosts where they mirror to and fill them once, after
+// the last step: enqueue_mirrored.)  The dt of every step stays on the device: the
 // update kernels derive it from per-block wave-speed maxima that the previous
 // update and the ghost fill reduced, and from a device-resident TimeStep call
 // counter that the ghost fill advances.

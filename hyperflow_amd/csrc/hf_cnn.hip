@@ -437,7 +437,9 @@ constexpr int LPX = 72;   // LDS row pitch in elements (64 pixels + 8 padding)
 // workgroup, which stages as many again and leaves four times the partials.
 // 256^2, the five layers and their reduction: 64 + 13 us as five launches (44.6
 // for one 32 -> 32 layer with 16 rows, two operand reads per product and db
-// summed by threads), now 29 + 5; a training step at 1024^2 0.82 -> 0.73 ms.
+// summed by threads), now 29 + 5; a training step at 1024^2 0.805 -> 0.726 ms
+// against the same kernels layer by layer, although the data gradients, back to
+// back, then miss the cache (1024^2: 49 -> 58 us, 31 -> 47 the last).
 constexpr int WGRAD_FILL = 384;
 constexpr int WGRAD_LDS = (9 * 32 + 32) * LPX;
 

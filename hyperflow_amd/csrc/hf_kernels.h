@@ -253,7 +253,7 @@ __device__ __forceinline__ void half_steps(const HfBlockDev& bd, Dts&& dts, doub
 // of this row and, kept, of the next; the x slopes take theirs from the right
 // neighbour, and the left one's by a lane shift.
 // FP64 VALU issue bounds it, with two waves per SIMD: 8192^2 Van Leer runs at
-// 27.8 Gcell-updates/s, 21.5 with the general rows.
+// 27.5 Gcell-updates/s, 21.5 with the general rows.
 template <class M, int LIM, class Dts>
 __device__ __forceinline__ int muscl_rows_q64(const HfStepArgs<double>& a, const HfItem it, const HfBlockDev& bd,
                                               const int lane, Dts&& dts, double& dt_step, double& hx, double& hy,

@@ -102,7 +102,9 @@ HF_API int hf_ghost_cells(const hf_ctx* ctx);
 
 /* MeshBlock::set_fields (mesh_block.cpp:155-158): n = 4*(nx+2g)*(ny+2g). */
 HF_API int hf_upload(hf_ctx* ctx, int block, const double* fields, size_t n);
-/* MeshBlock::get_fields (mesh_block.cpp:161-164); synchronises the stream. */
+/* MeshBlock::get_fields (mesh_block.cpp:161-164); synchronises the stream.
+ * Blocks of more than 8 MiB go through pinned memory (up to 16 MiB, kept by the
+ * context until hf_destroy) and up to seven short-lived host threads. */
 HF_API int hf_download(hf_ctx* ctx, int block, double* fields, size_t n);
 
 /* Mesh::apply_bcs (mesh.cpp:31-39): ghost fill of every block, sides in the

@@ -60,7 +60,9 @@ HF_API int hf_net_forward(hf_net* net, const float* u_dev, int nx, int ny, float
 /* Gradient of the mean squared error between the network output and
  * (target_dev - u_dev) / out_scale over all cells and the 4 variables, with
  * respect to every parameter (same order as the parameters).  grads may be
- * null; *loss receives the loss (may be null).  Synchronises the stream. */
+ * null; *loss receives the loss (may be null).  Synchronises the stream.
+ * The first gradient of an image size allocates the backward pass's images
+ * (about 0.71 GB at 1024^2), kept until another size or hf_net_destroy. */
 HF_API int hf_net_gradients(hf_net* net, const float* u_dev, const float* target_dev, int nx, int ny, float* grads,
                             float* loss);
 /* One Adam step (beta1 0.9, beta2 0.999, eps 1e-8) on that loss.  loss_dev,

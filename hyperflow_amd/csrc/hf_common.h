@@ -117,7 +117,7 @@ enum { HF_SYNC_QUEUE = 0, HF_SYNC_DONE = 1, HF_SYNC_EXITED = 2, HF_SYNC_NSKIP = 
 enum { HF_SLOT_MAIN = 0, HF_SLOT_HOST = 1, HF_SLOT_GUESS = 2, HF_SLOT_CHECK = 3, HF_SLOTS = 4 };
 #define HF_SYNC_ABORT_BIT 0x80000000u
 
-// Step bookkeeping done by the first workgroup of a ghost-fill launch.
+// Step bookkeeping done by the last workgroup of a ghost-fill launch.
 struct GhostBook {
     uint32_t* calls;
     const HfProbDev* probs;
